@@ -7,9 +7,9 @@
 // products are exact in fp32, accumulation in fp32); the squared norms are
 // fp32 sums in element order. Ties are ordered by (distance, id).
 //
-// One-pass path, used for bases under four samples (262,144 rows at k = 10),
-// for rows longer than 512 values, for the threshold sample of the two-pass
-// path and for queries that overflow it:
+// One-pass path, used for small bases (under 16,384 rows; under four samples,
+// 262,144 rows at k = 10, where rows hold up to 128 values), for the threshold
+// sample of the two-pass path and for queries that overflow the other paths:
 // bf_scan_kernel: one wave owns 32 queries and one chunk of the base. It
 // holds the A fragments of its queries in registers and walks the chunk 32
 // vectors at a time (one 32x32 output tile, K over the padded dim), loading
@@ -21,14 +21,18 @@
 // wave per query merges the chunk lists. Rows longer than 32 K steps (512
 // values, config 4's 960) take the same kernel with the query and base
 // fragments read per slice of 8 K steps.
-// The two-pass path for large bases is described before bf_filter_kernel.
+// The two-pass path for large bases of rows of up to 128 values is described
+// before bf_filter_kernel, the rounds path for longer rows before
+// bf_tile_kernel.
 #include "bruteforce.hpp"
 #include "common.hpp"
 #include "graph.hpp"
+#include "mfma_gemm.hpp"
 
 #include <algorithm>
 #include <cfloat>
 #include <cstdlib>
+#include <numeric>
 #include <stdexcept>
 
 namespace jasper_amd {
@@ -60,7 +64,9 @@ __device__ __forceinline__ half8 u4_as_h8(uint4 v) {
 // two rows of a wave share a bank when they read the same column.
 constexpr uint32_t kSqnRows = 256, kSqnChunk = 64, kSqnStride = kSqnChunk * 2 + 8;  // bytes
 __global__ __launch_bounds__(kSqnRows) void row_sqnorm_kernel(const uint16_t* __restrict__ x, int64_t n,
-                                                              uint32_t dp, uint32_t dim, float* __restrict__ out) {
+                                                              uint32_t dp, uint32_t dim, float* __restrict__ out,
+                                                              const uint32_t* __restrict__ wanted) {
+  if (wanted && !*wanted) return;  // the norms are for queries left over, and there are none
   __shared__ __align__(16) uint8_t tile[kSqnRows * kSqnStride];  // 34,816 bytes
   const uint32_t t = threadIdx.x;
   const int64_t r0 = (int64_t)blockIdx.x * kSqnRows;
@@ -397,12 +403,11 @@ __device__ __forceinline__ void bf_sstore(uint4* tile, float* tvs, uint32_t buf,
 
 // TILES: 32-query tiles per wave; SUB: 32-row base tiles per step (one
 // barrier per SUB tiles, SUB independent matrix-core chains per query tile).
-// Two waves per SIMD up to 128 values per row (the pipelined loop's two
-// accumulator sets then fit 256 registers: config 2, 1M x 128, 5.38 ms ->
-// 4.98 ms against one wave); wider rows keep one (two spill: 1M x 256,
-// 12.9 ms at one wave, 18.2 ms at two).
+// Two waves per SIMD: the pipelined loop's two accumulator sets fit 256
+// registers at up to 128 values per row (config 2, 1M x 128, 5.38 ms ->
+// 4.98 ms against one wave). Longer rows take the rounds path.
 template <int KS, int TILES, int SUB, int METRIC>
-__global__ __launch_bounds__(256, (KS <= 8 ? 2 : 1)) void bf_filter_kernel(const uint16_t* __restrict__ base, int64_t n, uint32_t dp,
+__global__ __launch_bounds__(256, 2) void bf_filter_kernel(const uint16_t* __restrict__ base, int64_t n, uint32_t dp,
                                                         const uint16_t* __restrict__ queries, int64_t nq,
                                                         const float* __restrict__ vsq, const float* __restrict__ qsq,
                                                         const float* __restrict__ qthr, uint32_t thr_stride,
@@ -628,6 +633,379 @@ __global__ __launch_bounds__(256, (KS <= 8 ? 2 : 1)) void bf_filter_kernel(const
   }
 }
 
+// ------------------------------------------------------------ rounds path
+// The base is scored in rounds over its tiles, in an order that spreads every
+// round over the whole base (tile i of the order is tile i * mul mod n_tiles,
+// mul coprime to n_tiles: rows stored cluster by cluster meet every round
+// alike). Round 0 (kBfFirst rows) writes every distance; after each round a
+// trim kernel keeps a query's best k keys and its k-th distance T_q, and the
+// next round, 4 or 16 times as many rows, appends only keys with d <= T_q:
+// about k * (ratio - 1) of them. Every row is scored once.
+constexpr uint32_t kBfFirst = 4096;  // rows of round 0
+
+__device__ __forceinline__ uint32_t bf_tile_at(uint32_t i, uint32_t mul, uint32_t n_tiles) {
+  return (uint32_t)(((uint64_t)i * mul) % n_tiles);
+}
+
+// Work-group barrier for LDS alone: loads in flight (the next tile's) go on.
+__device__ __forceinline__ void lds_block_sync() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// One round over the order's tiles [t0, t1) with the product loop of
+// mfma_gemm.hpp: G::TM queries per work-group, tiles of G::TN base rows, n_ch
+// work-groups per query block taking contiguous parts of the round. The work
+// order is XCD-aware as in bf_filter_kernel: the query blocks of one part run
+// on one XCD and share its L2's copy of the tiles. The base rows' squared
+// norms are summed from the fragments the products read (v_dot2, in the
+// shadow of the MFMAs; each of the WAM waves that read the same fragments
+// takes one K step of a slice), so the base is read once, without a pass of
+// its own for the norms. dense: round 0, every distance to its own slot of
+// dist [nq][kBfFirst] (NaN for rows past the base).
+template <class G>
+struct BfTileLds {
+  static constexpr uint32_t kLocal = 11;  // keys staged per query
+  // after the loop's buffers, per query: staged keys, norm, threshold, the
+  // cheap test's bound, a count; then the norms' parts. 256 x 256: 161,792
+  // of 163,840 bytes
+  static constexpr size_t bytes = G::kLds + (size_t)G::TM * (8 * kLocal + 4 * 4) + (size_t)G::WAM * G::TN * 4;
+};
+
+template <class G, int METRIC>
+__global__ __launch_bounds__(G::kThreads, 2) void bf_tile_kernel(
+    const uint16_t* __restrict__ base, int64_t n, uint32_t dp, const uint16_t* __restrict__ queries, int64_t nq,
+    const float* __restrict__ qsq, const float* __restrict__ qthr, uint32_t t0, uint32_t t1, uint32_t n_tiles,
+    uint32_t mul, uint32_t n_ch, uint32_t qblocks, float* __restrict__ dense, uint32_t* __restrict__ qcount,
+    uint64_t* __restrict__ qcand) {
+  static_assert(G::KC / 2 == G::WAM, "one K step of a slice per wave that shares a column");
+  extern __shared__ uint4 bf_tile_lds[];
+  constexpr uint32_t kLocal = BfTileLds<G>::kLocal;
+  char* lds = reinterpret_cast<char*>(bf_tile_lds);
+  uint64_t* lbuf = reinterpret_cast<uint64_t*>(lds + G::kLds);         // [TM][kLocal]
+  float* sqs = reinterpret_cast<float*>(lbuf + (size_t)G::TM * kLocal);  // [TM] query norms
+  float* sth = sqs + G::TM;                                              // [TM] thresholds
+  float* scr = sth + G::TM;                                              // [TM] the cheap test's c_q
+  uint32_t* lcnt = reinterpret_cast<uint32_t*>(scr + G::TM);             // [TM]
+  float* part = reinterpret_cast<float*>(lcnt + G::TM);                  // [WAM][TN] parts of the rows' norms
+  const uint32_t W = gridDim.x, p = blockIdx.x, xcd = p & 7u, per = W >> 3, extra = W & 7u;
+  const uint32_t L = xcd * per + min(xcd, extra) + (p >> 3);
+  const uint32_t qblock = L % qblocks, ch = L / qblocks;
+  // part ch of the round: its tiles differ by at most one between parts
+  const uint32_t total = t1 - t0, each = total / n_ch, more = total % n_ch;
+  const uint32_t first = t0 + ch * each + min(ch, more), count = each + (ch < more ? 1u : 0u);
+  const int64_t qbase = (int64_t)qblock * G::TM;
+  for (uint32_t r = threadIdx.x; r < (uint32_t)G::TM; r += G::kThreads) {
+    const int64_t q = qbase + r;
+    // a NaN threshold passes nothing (rows past the last query)
+    const float qn = (METRIC == kL2 && q < nq) ? qsq[q] : 0.0f;
+    const float th = q >= nq ? __builtin_nanf("") : dense ? __builtin_inff() : qthr[q];
+    sqs[r] = qn;
+    sth[r] = th;
+    // L2: the bound of bf_filter_kernel. IP: fp16(q.v) >= -T_q needs q.v >=
+    // -T_q less half an fp16 step; a whole step (or the subnormal step) here.
+    const double t = (double)th;
+    const double c = METRIC == kL2 ? ((double)qn - t) - ((double)qn + fabs(t)) * 0x1p-19
+                                   : -t - fabs(t) * 0x1p-10 - 0x1p-24;
+    scr[r] = (float)(c - fabs(c) * 0x1p-22);
+    lcnt[r] = 0u;
+  }
+  __syncthreads();
+  const uint32_t lane = threadIdx.x & 63u, wave = uniform(threadIdx.x >> 6), am = lane & 31u, ah = lane >> 5;
+  const uint32_t wm = wave % G::WAM, wn = wave / G::WAM;
+  float vs[G::WTN];  // this lane's part of its columns' squared norms
+#pragma unroll
+  for (int b = 0; b < G::WTN; ++b) vs[b] = 0.0f;
+  // the tiles being loaded and being tested
+  uint32_t next = bf_tile_at(first, mul, n_tiles), here = next;
+  gemm_walk<G>(
+      lds, queries, qbase, nq - 1, base, n - 1, dp / 8, &kBfZeroChunk, count,
+      [&](uint32_t) {
+        const int64_t row = (int64_t)next * G::TN;
+        next += mul;
+        next -= next >= n_tiles ? n_tiles : 0u;
+        return row;
+      },
+      [&](int step, const gemm_half8 (&y)[G::WTN]) {
+        if (METRIC == kL2 && (uint32_t)step == wm) {
+          typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+#pragma unroll
+          for (int b = 0; b < G::WTN; ++b)
+#pragma unroll
+            for (int e = 0; e < 8; e += 2) {
+              const half2v h = {y[b][e], y[b][e + 1]};
+              vs[b] = __builtin_amdgcn_fdot2(h, h, vs[b], false);
+            }
+        }
+      },
+      [&](uint32_t t, const gemm_acc (&acc)[G::WTM][G::WTN]) {
+        const int64_t v0 = (int64_t)here * G::TN + wn * G::WTN * 32 + am;
+        here += mul;
+        here -= here >= n_tiles ? n_tiles : 0u;
+        float vn[G::WTN];
+#pragma unroll
+        for (int b = 0; b < G::WTN; ++b) vn[b] = 0.0f;
+        if constexpr (METRIC == kL2) {
+          // the last tile's readers are past the barriers of this tile's slices
+#pragma unroll
+          for (int b = 0; b < G::WTN; ++b) {
+            vs[b] += __shfl_xor(vs[b], 32, 64);
+            if (ah == 0) part[wm * G::TN + wn * G::WTN * 32 + 32 * b + am] = vs[b];
+            vs[b] = 0.0f;
+          }
+          lds_block_sync();
+#pragma unroll
+          for (int b = 0; b < G::WTN; ++b)
+#pragma unroll
+            for (int w = 0; w < G::WAM; ++w) vn[b] += part[w * G::TN + wn * G::WTN * 32 + 32 * b + am];
+        }
+#pragma unroll
+        for (int a = 0; a < G::WTM; ++a) {
+          // rows r0 + 8g + j of this lane; opaque, or the compiler reads every
+          // row's values once for the whole walk and spills
+          uint32_t r0 = wm * G::WTM * 32 + 32 * a + 4 * ah;
+          asm volatile("" : "+v"(r0));
+          float cq[16];
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            const float4 c4 = *reinterpret_cast<const float4*>(scr + r0 + 8 * g);
+            cq[4 * g] = c4.x, cq[4 * g + 1] = c4.y, cq[4 * g + 2] = c4.z, cq[4 * g + 3] = c4.w;
+          }
+#pragma unroll
+          for (int b = 0; b < G::WTN; ++b) {
+            const float vsm = vn[b] * kBfVsShrink;
+            uint64_t any = 0;  // lanes with a passing score
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+              const float y = METRIC == kL2 ? __builtin_fmaf(2.0f, acc[a][b][i], -vsm) : acc[a][b][i];
+              any |= ballot(y >= cq[i]);
+            }
+            if (any == 0 && !dense) continue;
+            const int64_t v = v0 + 32 * b;
+            uint32_t re = r0;
+            asm volatile("" : "+v"(re));
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+              const float y = METRIC == kL2 ? __builtin_fmaf(2.0f, acc[a][b][i], -vsm) : acc[a][b][i];
+              if (!dense && ballot(y >= cq[i]) == 0) continue;
+              const uint32_t r = re + 8 * (i >> 2) + (i & 3);
+              float d;
+              if constexpr (METRIC == kL2) d = __builtin_fmaf(-2.0f, acc[a][b][i], sqs[r] + vn[b]);
+              else d = -__half2float(__float2half_rn(acc[a][b][i]));
+              const bool pass = v < n && d <= sth[r];
+              if constexpr (METRIC == kL2) d = d < 0.0f ? 0.0f : d;
+              if (dense) {
+                const int64_t q = qbase + r;
+                if (q < nq)
+                  dense[(size_t)q * kBfFirst + (first + t) * G::TN + wn * G::WTN * 32 + 32 * b + am] =
+                      pass ? d : __builtin_nanf("");
+              } else if (pass) {
+                const uint64_t key = bf_key(d, (uint32_t)v);
+                const uint32_t s = atomicAdd(&lcnt[r], 1u);
+                if (s < kLocal) lbuf[(size_t)r * kLocal + s] = key;
+                else {
+                  // (inline: a call would save every accumulator around it)
+                  const size_t q = (size_t)qbase + r;
+                  const uint32_t at = atomicAdd(&qcount[q], 1u);
+                  if (at < kBfCandCap) qcand[q * kBfCandCap + at] = key;
+                }
+              }
+            }
+          }
+        }
+      });
+  if (dense) return;
+  // flush the staged keys: one reservation in the query's list
+  __syncthreads();
+  for (uint32_t r = threadIdx.x; r < (uint32_t)G::TM; r += G::kThreads) {
+    const uint32_t c = min(lcnt[r], kLocal);
+    if (qbase + r >= nq || c == 0) continue;
+    const uint32_t at = atomicAdd(&qcount[qbase + r], c);
+    for (uint32_t i = 0; i < c && at + i < kBfCandCap; ++i)
+      qcand[(size_t)(qbase + r) * kBfCandCap + at + i] = lbuf[(size_t)r * kLocal + i];
+  }
+}
+
+// ||x||^2 per row, a wave per row (the rounds path's query norms: few rows,
+// so the lanes share a row's sum instead of a row each).
+__global__ __launch_bounds__(256) void bf_query_sqnorm_kernel(const uint16_t* __restrict__ x, int64_t n, uint32_t dp,
+                                                              float* __restrict__ out) {
+  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const uint32_t lane = threadIdx.x & 63u;
+  if (row >= n) return;
+  float s = 0.0f;
+  for (uint32_t c = lane; c < dp / 8; c += 64) {
+    const half8 h = u4_as_h8(reinterpret_cast<const uint4*>(x + (size_t)row * dp)[c]);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s = __builtin_fmaf((float)h[e], (float)h[e], s);
+  }
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) s += __shfl_xor(s, m, 64);
+  if (lane == 0) out[row] = s;
+}
+
+// After a round, a work-group per query: finds the query's k-th key and keeps
+// the k smallest in the list (in any order), their k-th distance as the
+// threshold. The k-th is found by bits, from the top: a key's word takes a 0
+// where at least k keys are then no larger (keys in registers, 16 per lane);
+// the id word only where the k-th distance ties. That needs no sort of the
+// list (1,024 keys sorted through LDS by a wave took 216 us for 10k queries);
+// only the last round sorts, and only k keys. Four waves for round 0's 4,096
+// keys: with 64 per lane the unrolled code ran once per wave from a cold
+// instruction cache (272 us for 10k queries).
+// A list that overflowed, or with fewer than k keys of finite distance
+// (infinite or NaN rows), flags its query for the one-pass kernels, and a NaN
+// threshold keeps later rounds from appending to it.
+// TN > 0: the keys are round 0's distances and the ids those of the order's
+// first tiles of TN rows.
+constexpr int kBfTrimRows = kBfCandCap / 64;  // keys per lane
+
+template <int TN>
+__global__ __launch_bounds__(TN > 0 ? 256 : 64) void bf_trim_kernel(
+    const float* __restrict__ dense, uint32_t mul, uint32_t n_tiles, uint32_t* __restrict__ qcount,
+    uint64_t* __restrict__ qcand, uint32_t k, bool last, uint32_t* __restrict__ any_flag, float* __restrict__ qthr,
+    int32_t* __restrict__ out_ids, float* __restrict__ out_d, uint8_t* __restrict__ q_flags,
+    uint8_t* __restrict__ tile_flags) {
+  constexpr bool DENSE = TN > 0;
+  constexpr int kWaves = DENSE ? 4 : 1;
+  static_assert(!DENSE || kBfFirst == 64 * kBfTrimRows * kWaves, "round 0 fills the registers");
+  __shared__ uint64_t best[128];
+  __shared__ uint32_t red[2][4];
+  __shared__ uint32_t taken;
+  const int64_t q = blockIdx.x;
+  const uint32_t lane = threadIdx.x & 63u, wave = uniform(threadIdx.x >> 6);
+  if (!DENSE && q_flags[q]) return;
+  const uint32_t cnt = DENSE ? kBfFirst : uniform(qcount[q]);
+  uint64_t* list = qcand + (size_t)q * kBfCandCap;
+  uint32_t hi[kBfTrimRows], lo[kBfTrimRows];  // empty slots and NaN: all ones
+  const uint32_t rows = DENSE ? (uint32_t)kBfTrimRows : min((cnt + 63u) / 64u, (uint32_t)kBfTrimRows);
+#pragma unroll
+  for (int j = 0; j < kBfTrimRows; ++j) {
+    hi[j] = lo[j] = ~0u;
+    if constexpr (DENSE) {
+      const uint32_t slot = (wave * kBfTrimRows + (uint32_t)j) * 64u;  // of lane 0
+      const float d = dense[(size_t)q * kBfFirst + slot + lane];
+      lo[j] = bf_tile_at(slot / (uint32_t)TN, mul, n_tiles) * (uint32_t)TN + slot % (uint32_t)TN + lane;
+      if (d == d) hi[j] = dist_to_ord(d);
+    } else if ((uint32_t)j < rows && (uint32_t)j * 64u + lane < cnt) {
+      const uint64_t key = list[(uint32_t)j * 64u + lane];
+      hi[j] = (uint32_t)(key >> 32);
+      lo[j] = (uint32_t)key;
+    }
+  }
+  uint32_t turn = 0;
+  // f(a, b) over the work-group's values
+  auto reduce = [&](uint32_t x, auto f) {
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) x = f(x, (uint32_t)__shfl_xor((int)x, m, 64));
+    if constexpr (kWaves > 1) {
+      if (lane == 0) red[turn][wave] = x;
+      __syncthreads();
+      x = f(f(red[turn][0], red[turn][1]), f(red[turn][2], red[turn][3]));
+      turn ^= 1u;
+    }
+    return uniform(x);
+  };
+  auto add = [](uint32_t a, uint32_t b) { return a + b; };
+  auto larger = [](uint32_t a, uint32_t b) { return max(a, b); };
+  auto smaller = [](uint32_t a, uint32_t b) { return min(a, b); };
+  auto count_to = [&](uint32_t top) {  // keys whose distance word is at most top
+    uint32_t c = 0;
+#pragma unroll
+    for (int j = 0; j < kBfTrimRows; ++j)
+      if ((uint32_t)j < rows) c += hi[j] <= top ? 1u : 0u;
+    return reduce(c, add);
+  };
+  // the k-th smallest distance word: below the bits that all words share
+  // (most of a float's top bits), and only until a word has exactly k below it
+  uint32_t mn = ~0u, mx = 0u;
+#pragma unroll
+  for (int j = 0; j < kBfTrimRows; ++j) {
+    mn = min(mn, hi[j]);
+    if (hi[j] != ~0u) mx = max(mx, hi[j]);
+  }
+  mn = reduce(mn, smaller);
+  mx = reduce(mx, larger);
+  uint32_t v = ~0u, below = 0;  // below: keys smaller than v
+  bool exact = false;           // no key beyond the k-th ties with it
+  if (mn != ~0u && count_to(mx) >= k) {
+    int bit = mn == mx ? -1 : 31 - __builtin_clz(mn ^ mx);
+    v = bit < 0 ? mn : mn & ~((2u << bit) - 1u);
+    for (; bit >= 0; --bit) {
+      const uint32_t top = v | ((1u << bit) - 1u);  // the largest word with a 0 here
+      const uint32_t c = count_to(top);
+      if (c == k) {
+        uint32_t x = 0;
+#pragma unroll
+        for (int j = 0; j < kBfTrimRows; ++j)
+          if (hi[j] <= top) x = max(x, hi[j]);
+        v = reduce(x, larger);
+        exact = true;
+        break;
+      }
+      if (c < k) {
+        v |= 1u << bit;
+        below = c;
+      }
+    }
+  }
+  const float t = ord_to_dist(v);
+  if (cnt > 64u * kBfTrimRows * kWaves || v == ~0u || !(fabsf(t) < __builtin_inff())) {
+    if (threadIdx.x == 0) {
+      q_flags[q] = 1;
+      tile_flags[q >> 5] = 1;
+      *any_flag = 1;
+      qthr[q] = __builtin_nanf("");
+    }
+    return;
+  }
+  // ties at it: the smallest k - below ids
+  uint32_t w = ~0u;
+  if (!exact && count_to(v) > k) {
+    w = 0;
+    for (int bit = 31; bit >= 0; --bit) {
+      const uint32_t top = w | ((1u << bit) - 1u);
+      uint32_t c = 0;
+#pragma unroll
+      for (int j = 0; j < kBfTrimRows; ++j) c += hi[j] == v && lo[j] <= top ? 1u : 0u;
+      if (below + reduce(c, add) < k) w |= 1u << bit;
+    }
+  }
+  if (threadIdx.x == 0) taken = 0;
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < kBfTrimRows; ++j) {
+    if (hi[j] < v || (hi[j] == v && lo[j] <= w)) {
+      const uint64_t key = ((uint64_t)hi[j] << 32) | lo[j];
+      const uint32_t at = atomicAdd(&taken, 1u);  // exactly k in all
+      if (last) best[at] = key;
+      else list[at] = key;
+    }
+  }
+  if (DENSE || !last) {  // (round 0 is never the last)
+    if (threadIdx.x == 0) {
+      qcount[q] = k;
+      qthr[q] = t;
+    }
+    return;
+  }
+  const uint32_t N = max(pow2_ceil(k), 2u);
+  for (uint32_t i = k + lane; i < N; i += 64u) best[i] = ~0ull;
+  wave_sync();
+  lds_bitonic_sort(best, N);
+  for (uint32_t i = lane; i < k; i += 64) {
+    out_ids[(size_t)q * k + i] = (int32_t)(uint32_t)best[i];
+    out_d[(size_t)q * k + i] = ord_to_dist((uint32_t)(best[i] >> 32));
+  }
+}
+
+__global__ void bf_clear_kernel(uint8_t* __restrict__ flags, int64_t n, uint32_t* __restrict__ word) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) flags[i] = 0;
+  if (i == 0) *word = 0;
+}
+
 // Per query: sort the candidate list by (distance, id) and write the best k;
 // a list that overflowed flags the query (and its 32-query tile) for the
 // one-pass kernels.
@@ -753,7 +1131,7 @@ static void launch_filter(const void* base, int64_t n, uint32_t dp, const void* 
     const char* e = std::getenv("JASPER_BF_SUB");
     return e ? std::atoi(e) : 2;
   }();
-  if (sub == 1 || KS > 16)
+  if (sub == 1)
     launch_filter_sub<KS, 1, METRIC>(base, n, dp, queries, nq, vsq, qsq, qthr, thr_stride, qcount, qcand, s);
   else
     launch_filter_sub<KS, 2, METRIC>(base, n, dp, queries, nq, vsq, qsq, qthr, thr_stride, qcount, qcand, s);
@@ -766,12 +1144,112 @@ static void dispatch_filter(uint32_t ks, const void* base, int64_t n, uint32_t d
   switch (ks) {
 #define JA_F(K) \
   case K: launch_filter<K, METRIC>(base, n, dp, queries, nq, vsq, qsq, qthr, thr_stride, qcount, qcand, s); break;
-    JA_F(1) JA_F(2) JA_F(3) JA_F(4) JA_F(5) JA_F(6) JA_F(7) JA_F(8) JA_F(9) JA_F(10) JA_F(11) JA_F(12) JA_F(13)
-    JA_F(14) JA_F(15) JA_F(16) JA_F(17) JA_F(18) JA_F(19) JA_F(20) JA_F(21) JA_F(22) JA_F(23) JA_F(24) JA_F(25)
-    JA_F(26) JA_F(27) JA_F(28) JA_F(29) JA_F(30) JA_F(31) JA_F(32)
+    JA_F(1) JA_F(2) JA_F(3) JA_F(4) JA_F(5) JA_F(6) JA_F(7) JA_F(8)
 #undef JA_F
     default: throw std::invalid_argument("bruteforce_knn: unsupported dim");
   }
+}
+
+// Scores the whole base in rounds and writes the results; flags (cleared by
+// the caller) name the queries that are left to the one-pass kernels.
+template <class G>
+static void bf_rounds(const void* base, int64_t n, uint32_t dp, const void* queries, int64_t nq, uint32_t k,
+                      int metric, const float* qsq, float* qthr, float* dense, uint32_t* qcount, uint64_t* qcand,
+                      uint8_t* q_flags, uint8_t* tile_flags, int32_t* out_ids, float* out_d, hipStream_t s) {
+  const uint32_t n_tiles = (uint32_t)((n + G::TN - 1) / G::TN);
+  const uint32_t qblocks = (uint32_t)((nq + G::TM - 1) / G::TM);
+  uint32_t mul = std::max<uint32_t>(1u, (uint32_t)(0.6180339887 * n_tiles));
+  while (std::gcd(mul, n_tiles) != 1u) ++mul;
+  constexpr size_t lds = BfTileLds<G>::bytes;
+  // work-groups the chip holds at once: eight waves per CU (two per SIMD)
+  constexpr uint32_t kResident = 256u * (8 / G::kWaves);
+  auto go = [&](auto kern, uint32_t t0, uint32_t t1, float* dist) {
+    hip_check(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), "LDS");
+    // parts per query block: the count whose last turn of resident
+    // work-groups is fullest (a part's tiles set its time)
+    uint32_t best = 1;
+    uint64_t cost = ~0ull;
+    for (uint32_t c = 1; c <= std::min<uint32_t>(t1 - t0, 4096u); ++c) {
+      const uint64_t turns = ((uint64_t)qblocks * c + kResident - 1) / kResident;
+      if (turns > 4 && c > 1) break;
+      const uint64_t x = turns * ((t1 - t0 + c - 1) / c);
+      if (x < cost) {
+        cost = x;
+        best = c;
+      }
+    }
+    hipLaunchKernelGGL(kern, dim3(qblocks * best), dim3(G::kThreads), lds, s, (const uint16_t*)base, n, dp,
+                       (const uint16_t*)queries, nq, qsq, (const float*)qthr, t0, t1, n_tiles, mul, best, qblocks,
+                       dist, qcount, qcand);
+    hip_check(hipGetLastError(), "launch bf_tile_kernel");
+  };
+  constexpr uint32_t kFirstTiles = kBfFirst / G::TN;
+  static_assert(kFirstTiles * G::TN == kBfFirst, "round 0 is whole tiles");
+  uint32_t t0 = 0, t1 = kFirstTiles;  // n >= 4 kBfFirst
+  while (true) {
+    float* dist = t0 == 0 ? dense : nullptr;
+    if (metric == kL2) go(bf_tile_kernel<G, kL2>, t0, t1, dist);
+    else go(bf_tile_kernel<G, kIP>, t0, t1, dist);
+    const bool last = t1 == n_tiles;
+    auto trim = [&](auto kern, uint32_t threads) {
+      hipLaunchKernelGGL(kern, dim3((uint32_t)nq), dim3(threads), 0, s, (const float*)dense, mul, n_tiles, qcount,
+                         qcand, k, last, qcount + nq, qthr, out_ids, out_d, q_flags, tile_flags);
+      hip_check(hipGetLastError(), "launch bf_trim_kernel");
+    };
+    if (t0 == 0) trim(bf_trim_kernel<G::TN>, 256);
+    else trim(bf_trim_kernel<0>, 64);
+    if (last) break;
+    // the last two rounds grow fourfold (few candidates where most rows
+    // are), earlier ones 16-fold where a list holds 16 k keys with room
+    t0 = t1;
+    const uint64_t grow = k <= 32 && (uint64_t)t1 * 64 <= n_tiles ? 16 : 4;
+    t1 = (uint32_t)std::min<uint64_t>(n_tiles, (uint64_t)t1 * grow);
+  }
+}
+
+// The rounds path: scratch, the rounds, and the one-pass kernels for the
+// queries the rounds flagged (none, in the ordinary case: they then end at
+// once).
+static void bf_in_rounds(const void* base, int64_t n, uint32_t dim, uint32_t dp, const void* queries, int64_t nq,
+                         uint32_t k, int metric, int32_t* out_ids, float* out_d, hipStream_t s) {
+  float* qsq = nullptr;
+  float* vsq = nullptr;
+  float* qthr = nullptr;
+  float* dense = nullptr;     // [nq][kBfFirst] round 0's distances
+  uint32_t* qcount = nullptr;  // [nq] counts, then one word: is any query flagged
+  uint64_t* qcand = nullptr;
+  uint8_t* flags = nullptr;  // [nq] query flags, then [ceil(nq / 32)] tile flags
+  const int64_t ntiles = (nq + 31) / 32;
+  hip_check(hipMallocAsync((void**)&qthr, (size_t)nq * 4, s), "alloc thresholds");
+  hip_check(hipMallocAsync((void**)&dense, (size_t)nq * kBfFirst * 4, s), "alloc first distances");
+  hip_check(hipMallocAsync((void**)&qcount, (size_t)(nq + 1) * 4, s), "alloc candidate counts");
+  hip_check(hipMallocAsync((void**)&qcand, (size_t)nq * kBfCandCap * 8, s), "alloc candidate lists");
+  hip_check(hipMallocAsync((void**)&flags, (size_t)(nq + ntiles), s), "alloc overflow flags");
+  hipLaunchKernelGGL(bf_clear_kernel, dim3((uint32_t)((nq + ntiles + 255) / 256)), dim3(256), 0, s, flags,
+                     nq + ntiles, qcount + nq);
+  if (metric == kL2) {
+    hip_check(hipMallocAsync((void**)&qsq, (size_t)nq * 4, s), "alloc query norms");
+    hip_check(hipMallocAsync((void**)&vsq, (size_t)n * 4, s), "alloc base norms");
+    hipLaunchKernelGGL(bf_query_sqnorm_kernel, dim3((uint32_t)((nq + 3) / 4)), dim3(256), 0, s,
+                       (const uint16_t*)queries, nq, dp, qsq);
+  }
+  // 256 queries per work-group at 991 TFLOP/s or 128 at 850 (mfma_gemm.hpp),
+  // whichever finishes the padded queries first
+  const uint64_t by256 = (uint64_t)((nq + 255) / 256) * 256 * 850, by128 = (uint64_t)((nq + 127) / 128) * 128 * 991;
+  auto rounds = by256 <= by128 ? bf_rounds<GemmTile<2, 4, 4, 2, 8>> : bf_rounds<GemmTile<2, 4, 2, 2, 4>>;
+  rounds(base, n, dp, queries, nq, k, metric, qsq, qthr, dense, qcount, qcand, flags, flags + nq, out_ids, out_d, s);
+  if (metric == kL2) {
+    hipLaunchKernelGGL(row_sqnorm_kernel, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, s, (const uint16_t*)base, n,
+                       dp, dim, vsq, (const uint32_t*)(qcount + nq));
+  }
+  bf_one_pass(base, n, dp, queries, nq, k, metric, vsq, qsq, out_ids, out_d, flags + nq, flags, s);
+  (void)hipFreeAsync(qthr, s);
+  (void)hipFreeAsync(dense, s);
+  (void)hipFreeAsync(qcount, s);
+  (void)hipFreeAsync(qcand, s);
+  (void)hipFreeAsync(flags, s);
+  if (vsq) (void)hipFreeAsync(vsq, s);
+  if (qsq) (void)hipFreeAsync(qsq, s);
 }
 
 void bruteforce_knn(const void* base, int64_t n, uint32_t dim, uint32_t dp, const void* queries, int64_t nq,
@@ -782,21 +1260,29 @@ void bruteforce_knn(const void* base, int64_t n, uint32_t dim, uint32_t dp, cons
   if (n <= 0) throw std::invalid_argument("empty base");
   if (n > 0x7FFFFFFFll) throw std::invalid_argument("too many base vectors");
   if (nq > 0x7FFFFFFFll) throw std::invalid_argument("too many queries");
+  // rows of more than 128 values: rounds (1M x 256, 3,750 queries, k = 10:
+  // 5.1 ms with the two passes below, 3.4 ms; 1M x 480, 2,000 queries, k =
+  // 100: 26.6 and 3.8 ms). Below 4 kBfFirst rows the one-pass kernels: round 0
+  // alone would be a quarter of the base.
+  if (dp > 128 && n >= 4 * (int64_t)kBfFirst) {
+    bf_in_rounds(base, n, dim, dp, queries, nq, k, metric, out_ids, out_d, s);
+    return;
+  }
   float* vsq = nullptr;
   float* qsq = nullptr;
   if (metric == kL2) {
     hip_check(hipMallocAsync((void**)&vsq, (size_t)n * 4, s), "alloc base norms");
     hip_check(hipMallocAsync((void**)&qsq, (size_t)nq * 4, s), "alloc query norms");
     hipLaunchKernelGGL(row_sqnorm_kernel, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, s, (const uint16_t*)base,
-                       n, dp, dim, vsq);
+                       n, dp, dim, vsq, nullptr);
     hipLaunchKernelGGL(row_sqnorm_kernel, dim3((uint32_t)((nq + 255) / 256)), dim3(256), 0, s,
-                       (const uint16_t*)queries, nq, dp, dim, qsq);
+                       (const uint16_t*)queries, nq, dp, dim, qsq, nullptr);
   }
-  // the two-pass path: rows of up to 32 K steps (512 values), and a sample
+  // the two-pass path: a sample
   // large enough that a query's filtered list (about k * n / sample keys)
   // stays near half of kBfCandCap
   const int64_t sample = std::max<int64_t>(kBfSample, ((int64_t)2 * k * n / kBfCandCap + 63) / 64 * 64);
-  if (n < 4 * sample || dp > 512) {
+  if (n < 4 * sample || dp > 128) {
     bf_one_pass(base, n, dp, queries, nq, k, metric, vsq, qsq, out_ids, out_d, nullptr, nullptr, s);
   } else {
     // 1. thresholds from the sample rows [0, sample)

@@ -156,3 +156,39 @@ def test_two_pass_overflow_falls_back(jasper, oracle_lib):
     rid, rd = _ref(base, q, 10, "l2")
     assert np.array_equal(d, rd)
     assert np.array_equal(ids, rid)
+
+
+# rounds path (rows of more than 128 values, 16,384 rows and more): one query
+# block and its edges (128 / 256 queries), a partial last tile of base rows, a
+# partial last slice of a row (dims that are no multiple of 64), k = 1 and the
+# largest; values small enough that every sum is an exact integer.
+@pytest.mark.parametrize("dim,n,nq,k", [(136, 16384, 1, 10), (200, 20001, 129, 128), (256, 66001, 256, 1),
+                                        (520, 17001, 257, 33), (960, 30003, 100, 100)])
+@pytest.mark.parametrize("distance", ["l2", "ip"])
+def test_rounds_integer_exact(jasper, oracle_lib, dim, n, nq, k, distance):
+    rng = np.random.default_rng(dim + n)
+    base = rng.integers(0, 12, size=(n, dim)).astype(np.float32)
+    q = rng.integers(0, 12, size=(nq, dim)).astype(np.float32)
+    ids, d = _run(jasper, base, q, k, distance)
+    rid, rd = _ref(base, q, k, distance)
+    assert np.array_equal(d, rd)
+    assert np.array_equal(ids, rid)
+
+
+def test_rounds_overflow_and_not_finite_rows(jasper, oracle_lib):
+    """Queries whose lists overflow (thousands of rows at distance 0, stored
+    together) are redone in one pass; rows with a NaN or an infinity (here
+    inf - inf) have no distance and are never returned."""
+    rng = np.random.default_rng(47)
+    base = rng.integers(0, 12, size=(40_000, 160)).astype(np.float32)
+    base[20_000:26_000] = base[7]
+    bad = rng.choice(np.arange(30_000, 40_000), size=900, replace=False)
+    q = rng.integers(1, 12, size=(70, 160)).astype(np.float32)
+    q[:20] = base[7]
+    keep = np.setdiff1d(np.arange(len(base)), bad)
+    rid, rd = _ref(base[keep], q, 10, "l2")
+    base[bad[:450], 3] = np.nan
+    base[bad[450:], 90] = np.inf
+    ids, d = _run(jasper, base, q, 10, "l2")
+    assert np.array_equal(d, rd)
+    assert np.array_equal(ids, keep[rid])
