@@ -720,7 +720,7 @@ __global__ __launch_bounds__(G::kThreads, 2) void bf_tile_kernel(
   // the tiles being loaded and being tested
   uint32_t next = bf_tile_at(first, mul, n_tiles), here = next;
   gemm_walk<G>(
-      lds, queries, qbase, nq - 1, base, n - 1, dp / 8, &kBfZeroChunk, count,
+      lds, queries, dp / 8, qbase, nq - 1, base, dp / 8, n - 1, dp / 8, &kBfZeroChunk, count,
       [&](uint32_t) {
         const int64_t row = (int64_t)next * G::TN;
         next += mul;
@@ -1165,21 +1165,9 @@ static void bf_rounds(const void* base, int64_t n, uint32_t dp, const void* quer
   constexpr uint32_t kResident = 256u * (8 / G::kWaves);
   auto go = [&](auto kern, uint32_t t0, uint32_t t1, float* dist) {
     hip_check(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), "LDS");
-    // parts per query block: the count whose last turn of resident
-    // work-groups is fullest (a part's tiles set its time)
-    uint32_t best = 1;
-    uint64_t cost = ~0ull;
-    for (uint32_t c = 1; c <= std::min<uint32_t>(t1 - t0, 4096u); ++c) {
-      const uint64_t turns = ((uint64_t)qblocks * c + kResident - 1) / kResident;
-      if (turns > 4 && c > 1) break;
-      const uint64_t x = turns * ((t1 - t0 + c - 1) / c);
-      if (x < cost) {
-        cost = x;
-        best = c;
-      }
-    }
-    hipLaunchKernelGGL(kern, dim3(qblocks * best), dim3(G::kThreads), lds, s, (const uint16_t*)base, n, dp,
-                       (const uint16_t*)queries, nq, qsq, (const float*)qthr, t0, t1, n_tiles, mul, best, qblocks,
+    const uint32_t parts = gemm_parts(qblocks, t1 - t0, kResident);
+    hipLaunchKernelGGL(kern, dim3(qblocks * parts), dim3(G::kThreads), lds, s, (const uint16_t*)base, n, dp,
+                       (const uint16_t*)queries, nq, qsq, (const float*)qthr, t0, t1, n_tiles, mul, parts, qblocks,
                        dist, qcount, qcand);
     hip_check(hipGetLastError(), "launch bf_tile_kernel");
   };

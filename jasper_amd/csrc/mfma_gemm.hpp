@@ -57,19 +57,37 @@ __device__ __forceinline__ void gemm_load_lds16(const void* g, void* l) {
   __builtin_amdgcn_global_load_lds((gemm_glb_void*)g, (gemm_lds_void*)l, 16, 0, 0);
 }
 
+// How many parts to cut a walk of `tiles` tiles into, for `groups` rows of
+// work-groups each: the count whose last turn of `resident` work-groups is
+// fullest (a part's tiles set its turn's time).
+inline uint32_t gemm_parts(uint32_t groups, uint32_t tiles, uint32_t resident) {
+  uint32_t best = 1;
+  uint64_t cost = ~0ull;
+  for (uint32_t c = 1; c <= tiles; ++c) {
+    const uint64_t turns = ((uint64_t)groups * c + resident - 1) / resident;
+    if (turns > 4 && c > 1) break;
+    const uint64_t x = turns * ((tiles + c - 1) / c);
+    if (x < cost) {
+      cost = x;
+      best = c;
+    }
+  }
+  return best;
+}
+
 // Walks tiles 0 .. n_tiles - 1. `a_row0` / `a_last`: the work-group's first
 // row of A and the last valid one (rows past it read that row again);
-// tile_row(t): the first B row of tile t; `b_last` as a_last. nck: chunks per
-// row of either operand (its stride). zero: 16 bytes of zeros in global
+// tile_row(t): the first B row of tile t; `b_last` as a_last. a_stride,
+// b_stride: 16-byte chunks from row to row; nck: chunks multiplied. zero: 16 bytes of zeros in global
 // memory, read for chunks past the row in the last slice (both operands, so
 // that no value is multiplied by a stray one). slice(s, y): called with the B
 // fragments of each K step s of a slice; epi(t, acc): called with a tile's sums, lane l holding
 // column l % 32 of B tile b and rows 8*(i/4) + 4*(l/32) + i%4 of A tile a in
 // acc[a][b][i]. epi may use LDS outside [lds, lds + G::kLds).
 template <class G, class TileRow, class Slice, class Epi>
-__device__ __forceinline__ void gemm_walk(char* lds, const void* A, int64_t a_row0, int64_t a_last, const void* B,
-                                          int64_t b_last, uint32_t nck, const void* zero, uint32_t n_tiles,
-                                          TileRow tile_row, Slice slice, Epi epi) {
+__device__ __forceinline__ void gemm_walk(char* lds, const void* A, uint32_t a_stride, int64_t a_row0, int64_t a_last,
+                                          const void* B, uint32_t b_stride, int64_t b_last, uint32_t nck,
+                                          const void* zero, uint32_t n_tiles, TileRow tile_row, Slice slice, Epi epi) {
   if (n_tiles == 0) return;
   const uint32_t lane = threadIdx.x & 63u, wave = uniform(threadIdx.x >> 6);
   const uint32_t wm = wave % G::WAM, wn = wave / G::WAM;
@@ -85,7 +103,7 @@ __device__ __forceinline__ void gemm_walk(char* lds, const void* A, int64_t a_ro
   for (int j = 0; j < G::kLoadsA; ++j) {
     const uint32_t r = ((uint32_t)j * G::kWaves + wave) * kRowsPerLoad + lr;
     const int64_t row = min(a_row0 + (int64_t)r, a_last);
-    pa[j] = (const char*)A + (size_t)row * nck * 16 + chunk_of(r) * 16;
+    pa[j] = (const char*)A + (size_t)row * a_stride * 16 + chunk_of(r) * 16;
   }
   auto set_tile = [&](uint32_t t) {
     const int64_t row0 = tile_row(t);
@@ -93,7 +111,7 @@ __device__ __forceinline__ void gemm_walk(char* lds, const void* A, int64_t a_ro
     for (int j = 0; j < G::kLoadsB; ++j) {
       const uint32_t r = ((uint32_t)j * G::kWaves + wave) * kRowsPerLoad + lr;
       const int64_t row = min(row0 + (int64_t)r, b_last);
-      pb[j] = (const char*)B + (size_t)row * nck * 16 + chunk_of(r) * 16;
+      pb[j] = (const char*)B + (size_t)row * b_stride * 16 + chunk_of(r) * 16;
     }
   };
   auto issue = [&](uint32_t k, uint32_t buf) {
