@@ -4,19 +4,30 @@
 // At one bit per dimension the quantizer reduces to a closed form (the
 // multi-bit code is clamped to 0, so t_const does not matter): with
 // r = P^T x - P c, bit_i = [r_i >= 0] and two fp32 factors per vector
-// (f_add, f_rescale). The rotation P^T x is a GEMM; here it runs on the
-// matrix cores in fp32 (v_mfma_f32_16x16x4_f32), one wave per 16 vectors:
+// (f_add, f_rescale). The rotation P^T x is a GEMM. All residuals of a vector
+// stay in the registers of the four lanes that hold it; the factor sums are
+// reduced across those lanes with two xor shuffles.
+//
+// fp16 rows (rabitq_split_kernel): x is exact in fp16, and each fp32 entry of
+// P is the sum of three fp16 values (times its row's power of two), so the
+// fp32 product runs as three v_mfma_f32_16x16x32_f16 chains at 16 times the
+// fp32 matrix rate: every product is exact and the sums are fp32. An entry's
+// 24 bits split exactly unless it is under 2^-29 of its row's largest; the
+// rest is then below 2^-39 of that one, under the sums' own rounding. Where a
+// residual lies within the two products' rounding of zero, its tile (16
+// coordinates of 16 vectors) takes the fp32 product instead, so the code bytes
+// are that one's.
+// fp32 rows (rabitq_kernel): v_mfma_f32_16x16x4_f32, one wave per 16 vectors:
 // the MFMA's M side is 16 output coordinates, its N side 16 vectors, and the
 // four K slots of each MFMA take coordinates k = 32b + 8q + s (q = lane/16,
 // s = 0..7 across eight MFMAs), so each lane feeds the MFMA from one 32-byte
-// (fp16: 16-byte) run of its vector. All residuals of a vector stay in the
-// registers of the four lanes that hold it; the factor sums are reduced
-// across those lanes with two xor shuffles.
+// run of its vector.
 //
 // Node layout (rabitq_data_store<float>): code bytes = ceil(dim/8) rounded
 // up to 4, bits LSB-first, then f_add and f_rescale.
 #include "common.hpp"
 #include "graph.hpp"
+#include "mfma_gemm.hpp"
 #include "rabitq.hpp"
 
 #include <cmath>
@@ -25,81 +36,286 @@
 
 namespace jasper_amd {
 
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float float4v __attribute__((ext_vector_type(4)));
 
 uint32_t rabitq_code_bytes(uint32_t dim) { return ((dim + 7u) / 8u + 3u) / 4u * 4u; }
 
-// rc[i] = sum_k P[i + k*dim] c[k] (P times c: the centroid goes through
-// CUBLAS_OP_N, rotation.cuh:160-176).
-__global__ void rotate_centroid_kernel(const float* __restrict__ P, const float* __restrict__ c, uint32_t dim,
-                                       float* __restrict__ rc) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= dim) return;
-  float acc = 0.0f;
-  for (uint32_t k = 0; k < dim; ++k) acc = __builtin_fmaf(P[(size_t)i + (size_t)k * dim], c[k], acc);
-  rc[i] = acc;
-}
-
-// Pt[i][k] = P[k + i*dim] for i < dim, k < dim; zero padding to [mp][kp].
-__global__ void transpose_pad_kernel(const float* __restrict__ P, uint32_t dim, uint32_t mp, uint32_t kp,
-                                     float* __restrict__ pt) {
-  const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (uint64_t)mp * kp) return;
-  const uint32_t i = (uint32_t)(t / kp), k = (uint32_t)(t % kp);
-  pt[t] = (i < dim && k < dim) ? P[(size_t)k + (size_t)i * dim] : 0.0f;
-}
-
-template <bool F16>
-__device__ __forceinline__ void load_run8(const void* x, size_t row, uint32_t stride, uint32_t k, uint32_t dim,
-                                          bool ok, float (&v)[8]) {
-  if constexpr (F16) {
-    const uint16_t* xr = (const uint16_t*)x + row * stride;
-    if (ok && k + 8 <= stride) {
-      const uint4 w = *reinterpret_cast<const uint4*>(xr + k);
-      const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
+// Scratch of one call, written by one launch of rabitq_setup_kernel: the
+// rotated centroid rc[i] = sum_k P[i + k*dim] c[k] (P times c: the centroid
+// goes through CUBLAS_OP_N, rotation.cuh:160-176; zero without a centroid and
+// for i >= dim), and Pt[i][k] = P[k + i*dim], zero padded to [mp][kp]. For
+// fp16 rows (split) also three fp16 parts [3][mp][kp] of Pt[i][k] * 2^s_i;
+// inv[i] = 2^-s_i, where 2^s_i brings row i's largest entry to [2^14, 2^15);
+// and tol[i], which bounds the difference of the two products' sums i for a
+// vector of norm 1: the f32 MFMAs round kp / 4 times, the f16 ones 3 kp / 32
+// times, each by at most 2^-24 of sum |P_ik x_k| <= |P_i| |x|, and 8 more for
+// the sums inside an instruction.
+// Block i < mp: row i. Block mp: the centroid.
+__global__ __launch_bounds__(256) void rabitq_setup_kernel(const float* __restrict__ P, const float* __restrict__ c,
+                                                           uint32_t dim, uint32_t mp, uint32_t kp, bool split,
+                                                           float* __restrict__ rc, float* __restrict__ inv,
+                                                           float* __restrict__ tol, float* __restrict__ pt,
+                                                           _Float16* __restrict__ parts) {
+  const uint32_t i = blockIdx.x, t = threadIdx.x;
+  if (i == mp) {
+    if (t >= mp) return;
+    float acc = 0.0f;
+    if (c && t < dim)
+      for (uint32_t k = 0; k < dim; ++k) acc = __builtin_fmaf(P[(size_t)t + (size_t)k * dim], c[k], acc);
+    rc[t] = acc;
+    return;
+  }
+  const float v = i < dim && t < dim ? P[(size_t)t + (size_t)i * dim] : 0.0f;  // kp <= 256
+  if (t < kp) pt[(size_t)i * kp + t] = v;
+  if (!split) return;
+  __shared__ uint32_t top[4];
+  __shared__ float sq[4];
+  float s2 = v * v;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        v[2 * j] = h2f_lo(ws[j]);
-        v[2 * j + 1] = h2f_hi(ws[j]);
-      }
-    } else {
+  for (int x = 32; x >= 1; x >>= 1) s2 += __shfl_xor(s2, x, 64);
+  if ((t & 63u) == 0) sq[t >> 6] = s2;
+  uint32_t m = __builtin_bit_cast(uint32_t, fabsf(v));
 #pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = 0.0f;
-    }
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-      if (k + j >= dim) v[j] = 0.0f;
-  } else {
-    const float* xr = (const float*)x + row * stride;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = (ok && k + j < dim) ? xr[k + j] : 0.0f;
+  for (int x = 32; x >= 1; x >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, x, 64));
+  if ((t & 63u) == 0) top[t >> 6] = m;
+  __syncthreads();
+  m = max(max(top[0], top[1]), max(top[2], top[3]));
+  // the largest entry's exponent; rows of zeros, subnormals, infinities or
+  // NaN are taken as they are
+  const int e = (int)(m >> 23) - 127;
+  const int sh = m >> 23 == 0 || m >> 23 == 255 ? 0 : 14 - e;
+  const float w = __builtin_ldexpf(v, sh);
+  const _Float16 p1 = (_Float16)w;
+  const bool whole = fabsf((float)p1) < __builtin_inff();
+  const float r1 = whole ? w - (float)p1 : 0.0f;  // exact
+  const _Float16 p2 = (_Float16)r1;
+  const _Float16 p3 = (_Float16)(r1 - (float)p2);
+  if (t < kp) {
+    const size_t at = (size_t)i * kp + t, part = (size_t)mp * kp;
+    parts[at] = p1;
+    parts[part + at] = p2;
+    parts[2 * part + at] = p3;
+  }
+  if (t == 0) {
+    inv[i] = __builtin_ldexpf(1.0f, -sh);
+    const float rounds = (float)(kp / 4 + 3 * kp / 32 + 8) * 0x1p-24f;
+    tol[i] = rounds * sqrtf((sq[0] + sq[1]) + (sq[2] + sq[3])) * 1.01f;
   }
 }
 
+// The factors and the node of one vector, from the four lanes (q = 0..3) that
+// hold its residuals r_i at i = 16t + 4q + j in res[t][j] (zero for i >= dim).
+// rcv(t, j): the rotated centroid at i.
+// |r_i| / ||r|| is rounded as the correctly rounded quotient: y = RN(1/||r||),
+// then two residual corrections (five fp32 operations where the f64 division
+// took about twenty; it was most of the kernel's time). The corrections are
+// exact while nothing is near the exponent range's ends; a wave with a norm
+// outside [2^-60, 2^60] (zero, infinite and NaN ones included) divides in f64.
+template <int KT, class Rc>
+__device__ __forceinline__ void rabitq_emit(float4v (&res)[KT], float l2, uint32_t dim, uint32_t q, Rc rcv, int metric,
+                                            bool ok, uint32_t* __restrict__ node) {
+  l2 += __shfl_xor(l2, 16, 64);
+  l2 += __shfl_xor(l2, 32, 64);
+  const float l2_norm = sqrt_rn(l2);
+  const float y = (float)(1.0 / (double)l2_norm);
+  const bool plain = ballot(!(l2_norm >= 0x1p-60f && l2_norm <= 0x1p60f)) == 0;
+  float ipn = 0.0f, s_rx = 0.0f, s_cx = 0.0f, s_rc = 0.0f;
+  constexpr int KW = (KT + 1) / 2;
+  uint32_t word[KW];
+#pragma unroll
+  for (int w = 0; w < KW; ++w) word[w] = 0;
+#pragma unroll
+  for (int t = 0; t < KT; ++t) {
+    const float4v cv = rcv(t);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t i = 16u * t + 4u * q + j;
+      // only the last tile holds coordinates past dim (dim > 16 (KT - 1))
+      if (t < KT - 1 || i < dim) {
+        const float r = res[t][j];
+        const float c = cv[j];
+        float d;
+        if (plain) {
+          d = r * y;
+          d = __builtin_fmaf(__builtin_fmaf(-d, l2_norm, r), y, d);
+          d = __builtin_fmaf(__builtin_fmaf(-d, l2_norm, r), y, d);
+        } else {
+          d = div_rn(r, l2_norm);
+        }
+        ipn += 0.5f * fabsf(d);
+        const bool bit = r >= 0.0f;
+        const float xucb = bit ? 0.5f : -0.5f;
+        s_rx = __builtin_fmaf(r, xucb, s_rx);
+        s_cx = __builtin_fmaf(c, xucb, s_cx);
+        s_rc = __builtin_fmaf(r, c, s_rc);
+        word[t / 2] |= (bit ? 1u : 0u) << (16 * (t & 1) + j);
+      }
+    }
+  }
+#pragma unroll
+  for (int m = 16; m <= 32; m <<= 1) {
+    ipn += __shfl_xor(ipn, m, 64);
+    s_rx += __shfl_xor(s_rx, m, 64);
+    s_cx += __shfl_xor(s_cx, m, 64);
+    s_rc += __shfl_xor(s_rc, m, 64);
+  }
+  float ipn_inv = div_rn(1.0f, ipn);
+  if (isnan(ipn_inv)) ipn_inv = 1.0f;
+  if (s_rx == 0.0f) s_rx = __builtin_inff();
+  float f_add, f_rescale;
+  if (metric == kL2) {
+    f_add = l2 + div_rn(2.0f * l2 * s_cx, s_rx);
+    f_rescale = ipn_inv * -2.0f * l2_norm;
+  } else {
+    f_add = (1.0f - s_rc) + div_rn(l2 * s_cx, s_rx);
+    f_rescale = ipn_inv * -l2_norm;
+  }
+  // this lane's nibbles into their places (4q of each half word), then the
+  // four lanes' together; lane q writes dwords q, q + 4, ... of the node
+  uint32_t dw[KW + 2 + 3];
+#pragma unroll
+  for (int w = 0; w < KW; ++w) {
+    uint32_t x = word[w] << (4 * q);
+    x |= (uint32_t)__shfl_xor((int)x, 16, 64);
+    x |= (uint32_t)__shfl_xor((int)x, 32, 64);
+    dw[w] = x;
+  }
+  dw[KW] = __builtin_bit_cast(uint32_t, f_add);
+  dw[KW + 1] = __builtin_bit_cast(uint32_t, f_rescale);
+#pragma unroll
+  for (int w = KW + 2; w < KW + 5; ++w) dw[w] = 0;
+  uint32_t pick[4];
+#pragma unroll
+  for (uint32_t w = 0; w < 4; ++w) pick[w] = q == w ? ~0u : 0u;
+  if (ok) {
+#pragma unroll
+    for (int w = 0; w < KW + 2; w += 4) {
+      // (by masks: selects of array elements become an indexed array)
+      const uint32_t x = (dw[w] & pick[0]) | (dw[w + 1] & pick[1]) | (dw[w + 2] & pick[2]) | (dw[w + 3] & pick[3]);
+      if ((uint32_t)w + q < KW + 2) node[(uint32_t)w + q] = x;
+    }
+  }
+}
+
+// The values of the row chunk at coordinates k .. k + 7 that lie below dim;
+// zeros past it, whatever a row's padding holds.
+__device__ __forceinline__ uint4 keep_below(uint4 w, uint32_t k, uint32_t dim) {
+  uint32_t ws[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+  for (uint32_t j = 0; j < 4; ++j) {
+    if (k + 2 * j >= dim) ws[j] = 0;
+    else if (k + 2 * j + 1 >= dim) ws[j] &= 0xFFFFu;
+  }
+  return make_uint4(ws[0], ws[1], ws[2], ws[3]);
+}
+
+// What the fp16-row kernels keep in LDS beside P, [mp] each.
+struct RqTables {
+  const float *rc, *inv, *tol;
+};
+
+// One tile of 16 vectors from the split product's sums to its residuals, in
+// place; returns sum r^2 over this lane's coordinates. x2: this lane's part of
+// |x|^2. An output tile with a residual within `tol` of zero is taken again
+// from the fp32 product (about one in 130 at 128 dims). Redoing the vectors'
+// other output tiles with it cost 45 us more on 1M x 128.
+template <int KT>
+__device__ __forceinline__ float rabitq_residuals(float4v (&acc)[KT], float x2, const uint16_t* __restrict__ x, int64_t v,
+                                                  int64_t n, uint32_t stride, uint32_t dim,
+                                                  const float* __restrict__ pt, uint32_t col, uint32_t q,
+                                                  const RqTables& tab) {
+  constexpr uint32_t kp = 32 * ((KT + 1) / 2);
+  x2 += __shfl_xor(x2, 16, 64);
+  x2 += __shfl_xor(x2, 32, 64);
+  const float xn = sqrtf(x2) * 1.01f;
+  uint32_t q4 = 4 * q;
+  asm volatile("" : "+v"(q4));  // opaque: or the tables are held in registers for all tiles
+  uint32_t redo = 0;  // output tiles with a residual within its tolerance
+#pragma unroll
+  for (int t = 0; t < KT; ++t) {
+    const float4v cv = *reinterpret_cast<const float4v*>(tab.rc + 16 * t + q4);
+    const float4v iv = *reinterpret_cast<const float4v*>(tab.inv + 16 * t + q4);
+    const float4v tv = *reinterpret_cast<const float4v*>(tab.tol + 16 * t + q4);
+    bool near = false;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const bool in = t < KT - 1 || 16u * t + 4u * q + j < dim;
+      // (the scaling is exact: one rounding, that of the subtraction)
+      const float r = in ? __builtin_fmaf(acc[t][j], iv[j], -cv[j]) : 0.0f;
+      near = near || (in && !(fabsf(r) > tv[j] * xn));  // NaN included
+      acc[t][j] = r;
+    }
+    if (ballot(near && v < n)) redo |= 1u << t;
+  }
+  if (redo) {
+#pragma unroll
+    for (int t = 0; t < KT; ++t) {
+      if (!(redo >> t & 1u)) continue;
+      float4v a = {0.0f, 0.0f, 0.0f, 0.0f};
+      for (uint32_t b = 0; b < kp; b += 32) {
+        const uint32_t k = b + 8 * q;
+        uint4 w = make_uint4(0, 0, 0, 0);
+        if (v < n && k < dim) w = keep_below(*reinterpret_cast<const uint4*>(x + (size_t)v * stride + k), k, dim);
+        const float4* pr = reinterpret_cast<const float4*>(pt + (size_t)(16 * t + col) * kp + k);
+        const float4 p0 = pr[0], p1 = pr[1];
+        const float xv[8] = {h2f_lo(w.x), h2f_hi(w.x), h2f_lo(w.y), h2f_hi(w.y),
+                             h2f_lo(w.z), h2f_hi(w.z), h2f_lo(w.w), h2f_hi(w.w)};
+        const float pv[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
+#pragma unroll
+        for (int s = 0; s < 8; ++s) a = __builtin_amdgcn_mfma_f32_16x16x4f32(pv[s], xv[s], a, 0, 0, 0);
+      }
+      const float4v cv = *reinterpret_cast<const float4v*>(tab.rc + 16 * t + q4);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[t][j] = t < KT - 1 || 16u * t + 4u * q + j < dim ? a[j] - cv[j] : 0.0f;
+    }
+  }
+  float l2 = 0.0f;
+#pragma unroll
+  for (int t = 0; t < KT; ++t)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) l2 = __builtin_fmaf(acc[t][j], acc[t][j], l2);
+  return l2;
+}
+
+// |x|^2 over 8 values
+__device__ __forceinline__ float sq_add(half8 h, float s) {
+  typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+#pragma unroll
+  for (int e = 0; e < 8; e += 2) {
+    const half2v p = {h[e], h[e + 1]};
+    s = __builtin_amdgcn_fdot2(p, p, s, false);
+  }
+  return s;
+}
+
 // KT = number of 16-wide output tiles (mp = 16 * KT <= 256).
-template <int KT, bool F16>
-__global__ __launch_bounds__(256) void rabitq_kernel(const void* __restrict__ x, int64_t n, uint32_t stride,
+template <int KT>
+__global__ __launch_bounds__(256, 2) void rabitq_kernel(const float* __restrict__ x, int64_t n, uint32_t stride,
                                                      uint32_t dim, const float* __restrict__ pt, uint32_t kp,
                                                      const float* __restrict__ rc, int metric,
-                                                     uint8_t* __restrict__ out, uint32_t code_bytes) {
+                                                     uint32_t* __restrict__ out) {
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t wave = threadIdx.x >> 6;
   const uint32_t col = lane & 15u;  // vector within the tile
   const uint32_t q = lane >> 4;     // K slot / output quarter
-  const uint32_t node_bytes = code_bytes + 8;
+  constexpr uint32_t kNode = (KT + 1) / 2 + 2;  // dwords per node
   const int64_t tiles = (n + 15) / 16;
   for (int64_t tile = (int64_t)blockIdx.x * 4 + wave; tile < tiles; tile += (int64_t)gridDim.x * 4) {
     const int64_t v = tile * 16 + col;
     const bool ok = v < n;
     float4v acc[KT];
+    const float* xr = x + (size_t)(ok ? v : 0) * stride;
 #pragma unroll
     for (int t = 0; t < KT; ++t) acc[t] = {0.0f, 0.0f, 0.0f, 0.0f};
     for (uint32_t b = 0; b < kp; b += 32) {
       float xv[8];
-      load_run8<F16>(x, (size_t)(ok ? v : 0), stride, b + 8 * q, dim, ok, xv);
+      const uint32_t k = b + 8 * q;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) xv[j] = (ok && k + j < dim) ? xr[k + j] : 0.0f;
 #pragma unroll
       for (int t = 0; t < KT; ++t) {
-        const float4* pr = reinterpret_cast<const float4*>(pt + (size_t)(16 * t + col) * kp + b + 8 * q);
+        const float4* pr = reinterpret_cast<const float4*>(pt + (size_t)(16 * t + col) * kp + k);
         const float4 p0 = pr[0], p1 = pr[1];
         const float pv[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
 #pragma unroll
@@ -117,65 +333,197 @@ __global__ __launch_bounds__(256) void rabitq_kernel(const void* __restrict__ x,
         acc[t][j] = r;
         l2 = __builtin_fmaf(r, r, l2);
       }
-    l2 += __shfl_xor(l2, 16, 64);
-    l2 += __shfl_xor(l2, 32, 64);
-    const float l2_norm = sqrt_rn(l2);
-    float ipn = 0.0f, s_rx = 0.0f, s_cx = 0.0f, s_rc = 0.0f;
-    uint32_t nib[KT];
+    rabitq_emit<KT>(
+        acc, l2, dim, q, [&](int t) { return *reinterpret_cast<const float4v*>(rc + 16 * t + 4 * q); }, metric, ok,
+        out + (size_t)v * kNode);
+  }
+}
+
+// fp16 rows. A block stages the three parts of Pt in LDS once (rows one chunk
+// past a multiple of 256 bytes, so that the 16 rows of a fragment fall on
+// different banks) and its waves then walk tiles of 16 * NT vectors alone:
+// each fragment of P read from LDS serves NT MFMAs, and the next tile's rows
+// load while this tile's factors are summed. LDS bounds NT = 1 (98 KB per 16
+// vectors at 128 dims), so two where the registers hold them (KT <= 8: 128
+// VGPRs of sums and rows).
+// 1M x 128: 668 us (f32 MFMA, f64 divisions, byte stores) -> 268 us; 1M x 96:
+// 410 -> 174 us. Against 64 bits over 512M codes at 128 dims the code bits are
+// off in the same 12 places, f_rescale by 1.04e-7 (1.09e-7 before).
+template <int KT, int NT>
+__global__ __launch_bounds__(512, 2) void rabitq_split_kernel(const uint16_t* __restrict__ x, int64_t n,
+                                                              uint32_t stride, uint32_t dim,
+                                                              const _Float16* __restrict__ parts,
+                                                              const float* __restrict__ pt,
+                                                              const float* __restrict__ tables, int metric,
+                                                              uint32_t* __restrict__ out) {
+  constexpr uint32_t KS = (KT + 1) / 2, kp = 32 * KS, mp = 16 * KT;
+  constexpr uint32_t kRow = kp / 8 + 1;  // chunks per row of a part
+  extern __shared__ uint4 rq_lds[];
+  const uint4* pg = reinterpret_cast<const uint4*>(parts);
+  float* tabl = reinterpret_cast<float*>(rq_lds + 3 * mp * kRow);  // rc, inv, tol
+  const RqTables tab{tabl, tabl + mp, tabl + 2 * mp};
+  for (uint32_t e = threadIdx.x; e < 3 * mp * (kp / 8); e += 512) rq_lds[(e / (kp / 8)) * kRow + e % (kp / 8)] = pg[e];
+  for (uint32_t e = threadIdx.x; e < 3 * mp; e += 512) tabl[e] = tables[e];
+  __syncthreads();
+  const uint32_t lane = threadIdx.x & 63u, col = lane & 15u, q = lane >> 4;
+  const int64_t tiles = (n + 16 * NT - 1) / (16 * NT);
+  const int64_t step = (int64_t)gridDim.x * 8;
+  int64_t tile = (int64_t)blockIdx.x * 8 + uniform(threadIdx.x >> 6);
+  // lane: coordinates 32s + 8q .. + 7 of vector 16 u + col; zeros past the
+  // row's dim, whatever the padding holds
+  uint4 xf[NT][KS];
+  auto load = [&](int64_t tl) {
 #pragma unroll
-    for (int t = 0; t < KT; ++t) {
-      nib[t] = 0;
+    for (int u = 0; u < NT; ++u) {
+      const int64_t v = tl * (16 * NT) + 16 * u + col;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const uint32_t i = 16u * t + 4u * q + j;
-        if (i < dim) {
-          const float r = acc[t][j];
-          const float c = rc[i];
-          ipn += 0.5f * fabsf(div_rn(r, l2_norm));
-          const bool bit = r >= 0.0f;
-          const float xucb = bit ? 0.5f : -0.5f;
-          s_rx = __builtin_fmaf(r, xucb, s_rx);
-          s_cx = __builtin_fmaf(c, xucb, s_cx);
-          s_rc = __builtin_fmaf(r, c, s_rc);
-          nib[t] |= (bit ? 1u : 0u) << j;
+      for (uint32_t s = 0; s < KS; ++s) {
+        const uint32_t k = 32 * s + 8 * q;
+        xf[u][s] = v < n && k < dim ? *reinterpret_cast<const uint4*>(x + (size_t)v * stride + k)
+                                    : make_uint4(0, 0, 0, 0);
+      }
+    }
+  };
+  if (tile < tiles) load(tile);
+  for (; tile < tiles; tile += step) {
+    // opaque per tile: or the compiler reads every fragment of P, the same for
+    // all tiles, before the loop, and spills them
+    uint32_t frag = col * kRow + q;
+    asm volatile("" : "+v"(frag));
+    float4v acc[NT][KT];
+#pragma unroll
+    for (int u = 0; u < NT; ++u)
+#pragma unroll
+      for (int t = 0; t < KT; ++t) acc[u][t] = {0.0f, 0.0f, 0.0f, 0.0f};
+    float x2[NT], l2[NT];
+#pragma unroll
+    for (int u = 0; u < NT; ++u) x2[u] = 0.0f;
+#pragma unroll
+    for (uint32_t s = 0; s < KS; ++s) {
+      half8 xh[NT];
+#pragma unroll
+      for (int u = 0; u < NT; ++u) {
+        // (stride >= 8-padded dim, so a chunk past dim's own is never read)
+        uint4 w = xf[u][s];
+        if (s == KS - 1 && dim % 8 != 0) w = keep_below(w, 32 * s + 8 * q, dim);
+        __builtin_memcpy(&xh[u], &w, 16);
+        x2[u] = sq_add(xh[u], x2[u]);
+      }
+#pragma unroll
+      for (int t = 0; t < KT; ++t) {
+#pragma unroll
+        for (int part = 2; part >= 0; --part) {  // smallest part first
+          const uint4 w = rq_lds[frag + ((uint32_t)part * mp + 16 * t) * kRow + 4 * s];
+          half8 ph;
+          __builtin_memcpy(&ph, &w, 16);
+#pragma unroll
+          for (int u = 0; u < NT; ++u) acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph, xh[u], acc[u][t], 0, 0, 0);
         }
       }
     }
 #pragma unroll
-    for (int m = 16; m <= 32; m <<= 1) {
-      ipn += __shfl_xor(ipn, m, 64);
-      s_rx += __shfl_xor(s_rx, m, 64);
-      s_cx += __shfl_xor(s_cx, m, 64);
-      s_rc += __shfl_xor(s_rc, m, 64);
-    }
-    float ipn_inv = div_rn(1.0f, ipn);
-    if (isnan(ipn_inv)) ipn_inv = 1.0f;
-    if (s_rx == 0.0f) s_rx = __builtin_inff();
-    float f_add, f_rescale;
-    if (metric == kL2) {
-      f_add = l2 + div_rn(2.0f * l2 * s_cx, s_rx);
-      f_rescale = ipn_inv * -2.0f * l2_norm;
-    } else {
-      f_add = (1.0f - s_rc) + div_rn(l2 * s_cx, s_rx);
-      f_rescale = ipn_inv * -l2_norm;
-    }
-    // byte 2t + (q >> 1) = nibble of q even | nibble of q odd << 4; the
-    // shuffles run on every lane (lanes l and l ^ 16 hold the same vector)
-    uint32_t bytes[KT];
+    for (int u = 0; u < NT; ++u)
+      l2[u] = rabitq_residuals<KT>(acc[u], x2[u], x, tile * (16 * NT) + 16 * u + col, n, stride, dim, pt, col, q, tab);
+    if (tile + step < tiles) load(tile + step);
+    uint32_t q4 = 4 * q;
+    asm volatile("" : "+v"(q4));
 #pragma unroll
-    for (int t = 0; t < KT; ++t) bytes[t] = nib[t] | ((uint32_t)__shfl_xor((int)nib[t], 16, 64) << 4);
-    if (ok) {
-      uint8_t* node = out + (size_t)v * node_bytes;
-      if ((q & 1u) == 0) {
+    for (int u = 0; u < NT; ++u) {
+      const int64_t v = tile * (16 * NT) + 16 * u + col;
+      rabitq_emit<KT>(
+          acc[u], l2[u], dim, q, [&](int t) { return *reinterpret_cast<const float4v*>(tab.rc + 16 * t + q4); }, metric,
+          v < n, out + (size_t)v * (KS + 2));
+    }
+  }
+}
+
+// fp16 rows of more than 160 values: the parts of Pt exceed LDS, so a block
+// stages them one K step of 32 at a time (3 * mp * 64 bytes, double-buffered,
+// loaded straight into LDS) and its eight waves take the step together, each
+// for its own 16 vectors (32 would spill: 128 sums per lane at 256 values, and
+// the factors' temporaries). Read through the caches instead, by each wave, 500k x 256 took 1.7 times as long; this way 0.89 ms (1.22 on the f32 MFMA).
+// Chunk q of row r sits at slot q ^ (r / 2 % 4) (mfma_gemm.hpp).
+template <int KT>
+__global__ __launch_bounds__(512, 2) void rabitq_split_long_kernel(const uint16_t* __restrict__ x, int64_t n,
+                                                                   uint32_t stride, uint32_t dim,
+                                                                   const _Float16* __restrict__ parts,
+                                                                   const float* __restrict__ pt,
+                                                                   const float* __restrict__ tables, int metric,
+                                                                   uint32_t* __restrict__ out) {
+  constexpr uint32_t KS = (KT + 1) / 2, kp = 32 * KS, mp = 16 * KT, NT = 1;
+  constexpr uint32_t kLoads = 3 * KT;  // kilobytes per step
+  __shared__ uint4 slice[2][3 * mp * 4];
+  __shared__ __align__(16) float tabl[3 * mp];  // rc, inv, tol
+  for (uint32_t e = threadIdx.x; e < 3 * mp; e += 512) tabl[e] = tables[e];
+  const RqTables tab{tabl, tabl + mp, tabl + 2 * mp};
+  const uint32_t lane = threadIdx.x & 63u, wave = uniform(threadIdx.x >> 6), col = lane & 15u, q = lane >> 4;
+  auto issue = [&](uint32_t s, uint32_t buf) {
 #pragma unroll
-        for (int t = 0; t < KT; ++t) node[2u * t + (q >> 1)] = (uint8_t)bytes[t];
-      }
-      if (q == 0) {
-        for (uint32_t byte = 2u * KT; byte < code_bytes; ++byte) node[byte] = 0;
-        *reinterpret_cast<float*>(node + code_bytes) = f_add;
-        *reinterpret_cast<float*>(node + code_bytes + 4) = f_rescale;
+    for (uint32_t j = 0; j < (kLoads + 7) / 8; ++j) {
+      const uint32_t kb = j * 8 + wave;  // 16 rows of 4 chunks
+      if (kb < kLoads) {
+        const uint32_t r = kb * 16 + (lane >> 2), c = (lane & 3u) ^ ((r >> 1) & 3u);
+        gemm_load_lds16(parts + (size_t)r * kp + 32 * s + 8 * c, (char*)slice[buf] + kb * 1024);
       }
     }
+  };
+  const int64_t tiles = (n + 16 * NT - 1) / (16 * NT);
+  const int64_t turns = (tiles + (int64_t)gridDim.x * 8 - 1) / ((int64_t)gridDim.x * 8);  // the same for every wave
+  auto row_chunk = [&](int64_t tl, uint32_t u, uint32_t s) {
+    const int64_t v = tl * (16 * NT) + 16 * u + col;
+    const uint32_t k = 32 * s + 8 * q;
+    uint4 w = make_uint4(0, 0, 0, 0);
+    if (v < n && k < dim) w = *reinterpret_cast<const uint4*>(x + (size_t)v * stride + k);
+    if (s == KS - 1 && dim % 8 != 0) w = keep_below(w, k, dim);
+    return w;
+  };
+  issue(0, 0);
+  uint32_t buf = 0;
+  for (int64_t turn = 0; turn < turns; ++turn) {
+    const int64_t tile = (turn * gridDim.x + blockIdx.x) * 8 + wave;  // past the last: no rows
+    float4v acc[NT][KT];
+#pragma unroll
+    for (uint32_t u = 0; u < NT; ++u)
+#pragma unroll
+      for (int t = 0; t < KT; ++t) acc[u][t] = {0.0f, 0.0f, 0.0f, 0.0f};
+    uint4 xn[NT];
+    float x2 = 0.0f;
+#pragma unroll
+    for (uint32_t u = 0; u < NT; ++u) xn[u] = row_chunk(tile, u, 0);
+    for (uint32_t s = 0; s < KS; ++s) {
+      half8 xh[NT];
+#pragma unroll
+      for (uint32_t u = 0; u < NT; ++u) __builtin_memcpy(&xh[u], &xn[u], 16);
+      x2 = sq_add(xh[0], x2);
+      __builtin_amdgcn_s_waitcnt(0x70);  // vmcnt(0) lgkmcnt(0): this step's slice and rows are here
+      __syncthreads();                   // and every wave is done with the other buffer
+      if (s + 1 < KS) {
+        issue(s + 1, buf ^ 1u);
+#pragma unroll
+        for (uint32_t u = 0; u < NT; ++u) xn[u] = row_chunk(tile, u, s + 1);
+      } else if (turn + 1 < turns) {
+        issue(0, buf ^ 1u);
+      }
+      const char* pl = (const char*)slice[buf] + col * 64 + ((q ^ ((col >> 1) & 3u)) * 16);
+#pragma unroll
+      for (int t = 0; t < KT; ++t) {
+#pragma unroll
+        for (int part = 2; part >= 0; --part) {  // smallest part first
+          const half8 ph = *reinterpret_cast<const half8*>(pl + (part * mp + 16 * t) * 64);
+#pragma unroll
+          for (uint32_t u = 0; u < NT; ++u)
+            acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph, xh[u], acc[u][t], 0, 0, 0);
+        }
+      }
+      buf ^= 1u;
+    }
+    const int64_t v = tile * 16 + col;
+    const float l2 = rabitq_residuals<KT>(acc[0], x2, x, v, n, stride, dim, pt, col, q, tab);
+    uint32_t q4 = 4 * q;
+    asm volatile("" : "+v"(q4));
+    rabitq_emit<KT>(
+        acc[0], l2, dim, q, [&](int t) { return *reinterpret_cast<const float4v*>(tab.rc + 16 * t + q4); }, metric,
+        v < n, out + (size_t)v * (KS + 2));
   }
 }
 
@@ -187,27 +535,37 @@ void rabitq_quantize(const void* x, bool f16, int64_t n, uint32_t dim, uint32_t 
     throw std::invalid_argument("fp16 rows must be 16-byte aligned with a stride that is a multiple of 8");
   if (n <= 0) return;
   const uint32_t kp = (dim + 31u) & ~31u, mp = (dim + 15u) & ~15u, kt = mp / 16;
-  float* pt = nullptr;
-  float* rc = nullptr;
-  hip_check(hipMallocAsync((void**)&pt, (size_t)mp * kp * 4, s), "alloc rabitq rotation");
-  hip_check(hipMallocAsync((void**)&rc, (size_t)mp * 4, s), "alloc rotated centroid");
-  hip_check(hipMemsetAsync(rc, 0, (size_t)mp * 4, s), "clear rotated centroid");
-  const uint64_t total = (uint64_t)mp * kp;
-  hipLaunchKernelGGL(transpose_pad_kernel, dim3((uint32_t)((total + 255) / 256)), dim3(256), 0, s, P, dim, mp, kp, pt);
-  if (centroid)
-    hipLaunchKernelGGL(rotate_centroid_kernel, dim3((dim + 63) / 64), dim3(64), 0, s, P, centroid, dim, rc);
+  // one allocation: rc, inv and tol [mp], Pt, then its parts
+  float* tables = nullptr;
+  const size_t ptn = (size_t)mp * kp;
+  hip_check(hipMallocAsync((void**)&tables, (size_t)3 * mp * 4 + ptn * (f16 ? 10 : 4), s), "alloc rabitq rotation");
+  float* pt = tables + 3 * mp;  // 16-byte aligned: mp is a multiple of 16
+  _Float16* parts = (_Float16*)(pt + ptn);
+  hipLaunchKernelGGL(rabitq_setup_kernel, dim3(mp + 1), dim3(256), 0, s, P, centroid, dim, mp, kp, f16, tables,
+                     tables + mp, tables + 2 * mp, pt, parts);
   hip_check(hipGetLastError(), "launch rabitq set-up");
-  const int64_t tiles = (n + 15) / 16;
-  const uint32_t grid = (uint32_t)std::min<int64_t>((tiles + 3) / 4, 16384);
-  const uint32_t cb = rabitq_code_bytes(dim);
-  auto go = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, s, x, n, stride, dim, (const float*)pt, kp,
-                       (const float*)rc, metric, (uint8_t*)out, cb);
+  auto wide = [&](auto kern) {
+    const int64_t tiles = (n + 15) / 16;
+    const uint32_t grid = (uint32_t)std::min<int64_t>((tiles + 3) / 4, 16384);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, s, (const float*)x, n, stride, dim, (const float*)pt, kp,
+                       (const float*)tables, metric, (uint32_t*)out);
   };
-#define JA_RQ_CASE(K)                                        \
-  case K:                                                    \
-    if (f16) go(rabitq_kernel<K, true>);                     \
-    else go(rabitq_kernel<K, false>);                        \
+  auto split = [&](auto kern, int nt, size_t lds) {
+    if (lds > 64 * 1024)
+      hip_check(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
+                "rabitq LDS");
+    // one turn of resident blocks (two waves per SIMD are one block of eight)
+    const int64_t tiles = (n + 16 * nt - 1) / (16 * nt);
+    const uint32_t grid = (uint32_t)std::min<int64_t>((tiles + 7) / 8, 256);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(512), lds, s, (const uint16_t*)x, n, stride, dim, (const _Float16*)parts,
+                       (const float*)pt, (const float*)tables, metric, (uint32_t*)out);
+  };
+  const size_t staged = (size_t)3 * mp * (kp / 8 + 1) * 16 + (size_t)3 * mp * 4;
+#define JA_RQ_CASE(K)                                                                   \
+  case K:                                                                               \
+    if (!f16) wide(rabitq_kernel<K>);                                                   \
+    else if constexpr (K <= 10) split(rabitq_split_kernel<K, (K <= 8 ? 2 : 1)>, K <= 8 ? 2 : 1, staged); \
+    else split(rabitq_split_long_kernel<K>, 1, 0);                                      \
     break;
   switch (kt) {
     JA_RQ_CASE(1) JA_RQ_CASE(2) JA_RQ_CASE(3) JA_RQ_CASE(4) JA_RQ_CASE(5) JA_RQ_CASE(6) JA_RQ_CASE(7)
@@ -217,8 +575,7 @@ void rabitq_quantize(const void* x, bool f16, int64_t n, uint32_t dim, uint32_t 
   }
 #undef JA_RQ_CASE
   hip_check(hipGetLastError(), "launch rabitq_kernel");
-  (void)hipFreeAsync(pt, s);
-  (void)hipFreeAsync(rc, s);
+  (void)hipFreeAsync(tables, s);
 }
 
 }  // namespace jasper_amd

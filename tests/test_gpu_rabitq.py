@@ -74,3 +74,32 @@ def test_rabitq_default_rotation_and_sizes(jasper, oracle_lib):
     assert torch.isfinite(got.f_add).all() and (got.f_rescale < 0).all()
     empty = jasper.rabitq_quantize(x[:0])
     assert empty.nodes.shape == (0, 24)
+
+
+# fp16 rows: the smallest dims, a last output tile of one coordinate, the edge
+# between P held in LDS whole (up to 160) and staged per K step, partial tiles
+# of vectors; and a matrix whose columns differ by ten orders of magnitude,
+# each split against its own largest entry.
+@pytest.mark.parametrize("dim,n", [(1, 33), (16, 1), (17, 31), (144, 500), (160, 4097), (161, 47), (177, 300),
+                                   (240, 129)])
+@pytest.mark.parametrize("metric", ["l2", "ip"])
+def test_rabitq_split_edges(jasper, oracle_lib, dim, n, metric):
+    rng = np.random.default_rng(dim)
+    x = rng.normal(size=(n, dim)).astype(np.float32)
+    m, _ = oracle.rotation_matrix(dim, 5)
+    c = (rng.normal(size=dim) * 0.5).astype(np.float32)
+    _check(jasper, x, m, c, metric, f16=True)
+
+
+def test_rabitq_columns_of_any_scale(jasper, oracle_lib):
+    """r_i = sum_k P[k + i*dim] x_k for P's column i scaled by 10^(i % 11 - 5):
+    the signs of every column's outputs are those of the 64-bit product."""
+    dim, n = 96, 2000
+    rng = np.random.default_rng(3)
+    x = rng.normal(size=(n, dim)).astype(np.float16)
+    p = (rng.normal(size=(dim, dim)) * 10.0 ** (np.arange(dim) % 11 - 5)[:, None]).astype(np.float32)  # row i = column i
+    got = jasper.rabitq_quantize(torch.from_numpy(x).cuda(), rotation=torch.from_numpy(p).cuda())
+    r = x.astype(np.float64) @ p.astype(np.float64).T
+    clear = np.abs(r) > 1e-5 * np.sqrt((p.astype(np.float64) ** 2).sum(1))[None, :]
+    bits = got.bits().cpu().numpy()
+    assert np.array_equal(bits[clear], (r >= 0)[clear].astype(np.uint8))
