@@ -65,6 +65,7 @@ struct SearchArgs {
   // integers too, with the union spanning at most smax, take the packed form
   uint32_t gint;
   int32_t glo, ghi, smax;
+  uint32_t hash_bytes;  // the seen cache in LDS (teams: what follows it)
 };
 
 // Seen cache: returns true when v is recorded, else records it (replacing
@@ -256,6 +257,14 @@ constexpr int search_waves_per_simd() {
                : CPL == 0 ? 4 : (CPL <= 4 && METRIC == kL2) ? JASPER_SEARCH_WAVES_L2 : 1;
 }
 
+// LDS order between the lanes of the wave that owns a query. In a team (the
+// work-group holds other waves) that wave alone waits, without a barrier.
+template <bool TEAM>
+__device__ __forceinline__ void search_sync() {
+  if constexpr (TEAM) lds_wave_sync();
+  else wave_sync();
+}
+
 // Merge of the sorted new keys t (nt of them, one per lane) into B held one
 // key per lane (b, cnt entries, bw <= 64): B ascending against the new keys
 // reversed, the lane-wise minima are a bitonic sequence holding the 64
@@ -290,6 +299,7 @@ __device__ __forceinline__ bool merge_regs(uint64_t& b, uint64_t t, uint32_t nt,
 // of [lb0, ncnt) run from the top down, so a chunk reads only entries that
 // are not yet overwritten (its own reads precede its writes). Returns false
 // when every new key was a repeat or a member of B (B unchanged).
+template <bool TEAM = false>
 __device__ __forceinline__ bool merge_general(uint64_t* B, uint64_t* T, uint32_t* TAG, uint64_t t, uint32_t nt,
                                               uint32_t& cnt, uint32_t& hint, uint32_t bw, uint32_t lane) {
   const uint64_t prev = __shfl_up(t, 1, 64);
@@ -304,16 +314,16 @@ __device__ __forceinline__ bool merge_general(uint64_t* B, uint64_t* T, uint32_t
   const uint32_t nk = (uint32_t)__builtin_popcountll(km);
   if (nk == 0) return false;
   const uint32_t ti = mbcnt(km);
-  wave_sync();
+  search_sync<(TEAM > 0)>();
   if (keep) T[ti] = t;
-  wave_sync();
+  search_sync<(TEAM > 0)>();
   const uint32_t lb0 = uniform((uint32_t)__shfl((int)lb, (int)__builtin_ctzll(km), 64));
   const uint32_t ncnt = min(cnt + nk, bw);
   const bool placed = keep && ti + lb < ncnt;
   if (placed) TAG[ti + lb] = 0x100u | ti;
   // kept keys that land inside the clipped list (the others fall past it)
   const uint32_t np = (uint32_t)__builtin_popcountll(ballot(placed));
-  wave_sync();
+  search_sync<(TEAM > 0)>();
   uint32_t above = 0;  // kept keys above the current chunk
   for (int32_t o0 = (int32_t)(lb0 + ((ncnt - 1u - lb0) & ~63u)); o0 >= (int32_t)lb0; o0 -= 64) {
     const uint32_t o = (uint32_t)o0 + lane;
@@ -332,17 +342,106 @@ __device__ __forceinline__ bool merge_general(uint64_t* B, uint64_t* T, uint32_t
   if (placed) TAG[ti + lb] = 0u;
   hint = uniform(min(hint, lb0));
   cnt = uniform(ncnt);
-  wave_sync();
+  search_sync<(TEAM > 0)>();
   return true;
 }
 
-// BYTES: the graph keeps byte rows (CPL 4, L2, no measurement mode)
-template <int CPL, int METRIC, bool STATS, bool BYTES = false>
-__global__ __launch_bounds__(64, (search_waves_per_simd<CPL, METRIC, BYTES>())) void beam_search_kernel(
+// Teams: with few queries in a launch the chip is mostly idle and a query's
+// time is its hops' one after another; most of a hop is then reading and
+// summing the new neighbours' rows, 16 (or 32) at a time by one wave, above
+// all where rows are longer than 32 chunks and stream through the registers
+// in batches that each wait out a memory latency. A work-group of TEAM waves
+// then serves a query: wave 0 searches, and a hop's rows go round the waves, a
+// row per quad, each quad summing in the one-wave kernel's order (the same
+// bits). For streamed rows the query row is in LDS and a row's chunks come in
+// batches of kTeamChunks per lane, the next batch in flight while one is
+// summed. A hop of at most kTeamAlone new neighbours is one pass of the
+// searching wave, which scores it alone (no barriers).
+constexpr uint32_t kTeamAlone = 16;
+constexpr int kTeamChunks = 6;  // four waves per SIMD without spills (8: 23 spilled, 1.2x slower)
+
+// The quad lane partial of a streamed row against the query row in LDS, in
+// the order of stream_partial_l2 / stream_partial_ip. A batch's query chunks
+// are read together, before the sums: left to itself the compiler reads each
+// right before its use and waits for LDS once per chunk.
+template <int METRIC>
+__device__ __forceinline__ float team_partial(const uint4* q, const uint4* row, uint32_t ql, uint32_t nchunks,
+                                              uint32_t nlimit) {
+  constexpr uint32_t kStep = 4u * kTeamChunks;
+  const uint32_t nck = METRIC == kL2 ? nlimit : (nlimit + 7u) / 8u;
+  float acc = 0.0f;
+  uint4 xa[kTeamChunks], xb[kTeamChunks];
+  auto load = [&](uint32_t c, uint4 (&x)[kTeamChunks]) {
+#pragma unroll
+    for (int u = 0; u < kTeamChunks; ++u) {
+      const uint32_t cc = c + 4u * (uint32_t)u;
+      x[u] = row[cc < nchunks ? cc : 0u];
+    }
+  };
+  auto add = [&](uint32_t c, const uint4 (&x)[kTeamChunks]) {
+    if constexpr (METRIC == kL2) {
+      uint4 qv[kTeamChunks];
+#pragma unroll
+      for (int u = 0; u < kTeamChunks; ++u) {
+        const uint32_t cc = c + 4u * (uint32_t)u;
+        qv[u] = q[cc < nchunks ? cc : 0u];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (c - ql + kStep <= nlimit) {  // (uniform) every lane's chunks lie inside the row
+#pragma unroll
+        for (int u = 0; u < kTeamChunks; ++u) l2_chunk(qv[u], x[u], acc);
+      } else {
+#pragma unroll
+        for (int u = 0; u < kTeamChunks; ++u)
+          if (c + 4u * (uint32_t)u < nlimit) l2_chunk(qv[u], x[u], acc);
+      }
+    } else {
+      // quad lane s holds chunk c - ql + 4u + s: each in turn to all four
+      // lanes, which take elements ql and ql + 4 of it
+      const uint16_t* qh = reinterpret_cast<const uint16_t*>(q);
+#pragma unroll
+      for (int u = 0; u < kTeamChunks; ++u) {
+        const uint32_t src[4] = {x[u].x, x[u].y, x[u].z, x[u].w};
+        const uint32_t c0 = c - ql + 4u * (uint32_t)u;
+        if (c0 >= nck) break;  // (uniform)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          uint32_t w[4];
+#pragma unroll
+          for (int k = 0; k < 4; ++k)
+            w[k] = s == 0 ? quad_bcast<0>(src[k]) : s == 1 ? quad_bcast<1>(src[k])
+                 : s == 2 ? quad_bcast<2>(src[k]) : quad_bcast<3>(src[k]);
+          const uint32_t w0 = (ql >> 1) == 0 ? w[0] : w[1], w1 = (ql >> 1) == 0 ? w[2] : w[3];
+          const float v0 = (ql & 1u) ? h2f_hi(w0) : h2f_lo(w0), v1 = (ql & 1u) ? h2f_hi(w1) : h2f_lo(w1);
+          const uint32_t e = 8u * (c0 + (uint32_t)s) + ql;
+          if (e < nlimit) acc = __builtin_fmaf(h2f_lo(qh[e]), v0, acc);
+          if (e + 4u < nlimit) acc = __builtin_fmaf(h2f_lo(qh[e + 4u]), v1, acc);
+        }
+      }
+    }
+  };
+  load(ql, xa);
+  for (uint32_t c0 = 0; c0 < nck; c0 += 2 * kStep) {
+    if (c0 + kStep < nck) load(c0 + kStep + ql, xb);
+    __builtin_amdgcn_sched_barrier(0);
+    add(c0 + ql, xa);
+    if (c0 + kStep >= nck) break;
+    if (c0 + 2 * kStep < nck) load(c0 + 2 * kStep + ql, xa);
+    __builtin_amdgcn_sched_barrier(0);
+    add(c0 + kStep + ql, xb);
+  }
+  return acc;
+}
+
+// BYTES: the graph keeps byte rows (CPL 4, L2, no measurement mode). TEAM:
+// waves per query (0: one, without a team's barriers).
+template <int CPL, int METRIC, bool STATS, bool BYTES = false, int TEAM = 0>
+__global__ __launch_bounds__(TEAM ? 64 * TEAM : 64, (TEAM ? 4 : search_waves_per_simd<CPL, METRIC, BYTES>())) void beam_search_kernel(
     SearchArgs a) {
+  static_assert(!TEAM || (!STATS && !BYTES), "the measurement mode and byte rows take one wave");
   static_assert(!BYTES || (CPL == 4 && METRIC == kL2 && !STATS), "byte rows: L2 rows of 112 or 128 values");
   extern __shared__ uint64_t smem[];
-  const uint32_t lane = threadIdx.x;
+  const uint32_t lane = threadIdx.x & 63u;
   const uint32_t qid = blockIdx.x;
   const uint32_t bw = a.bw;
   uint64_t* B = smem;                                     // [bw] the candidate list
@@ -350,14 +449,24 @@ __global__ __launch_bounds__(64, (search_waves_per_simd<CPL, METRIC, BYTES>())) 
   uint32_t* cand = reinterpret_cast<uint32_t*>(T + 64);   // [64] new neighbour ids
   uint32_t* TAG = cand + 64;                              // [bw] merge position tags
   uint32_t* H = TAG + bw;                                 // seen cache
-  {
-    // 32-bit words of the cache: empty = all ones (ids) or zero (tags)
-    const uint32_t words = a.tag_bits ? (1u << a.hash_bits) / 2u : 1u << a.hash_bits;
-    const uint32_t fill = a.tag_bits ? 0u : kInvalid32;
-    for (uint32_t i = lane; i < words; i += 64) H[i] = fill;
-    for (uint32_t i = lane; i < bw; i += 64) TAG[i] = 0u;  // no position marked
+  // team: the new neighbours' count (kTeamDone ends the helpers) and their
+  // distances, then the query row, past the seen cache
+  constexpr uint32_t kTeamDone = ~0u;
+  volatile uint32_t* team_n = nullptr;
+  float* team_d = nullptr;
+  uint4* team_q = nullptr;
+  if constexpr (TEAM > 0) {
+    char* past = reinterpret_cast<char*>(H) + a.hash_bytes;
+    team_q = reinterpret_cast<uint4*>(past);
+    team_d = reinterpret_cast<float*>(team_q + (CPL == 0 ? a.nchunks : 0u));
+    team_n = reinterpret_cast<volatile uint32_t*>(team_d + 64);
+    if constexpr (CPL == 0) {
+      const uint4* src = a.use_range ? a.vecs + (size_t)(a.q_start + qid) * a.nchunks
+                                     : a.queries + (size_t)qid * a.nchunks;
+      for (uint32_t c = threadIdx.x; c < a.nchunks; c += 64 * TEAM) team_q[c] = src[c];
+      __syncthreads();
+    }
   }
-
   const uint32_t ql = lane & 3u, qg = lane >> 2;
   const uint4* qrow = a.use_range ? a.vecs + (size_t)(a.q_start + qid) * a.nchunks
                                   : a.queries + (size_t)qid * a.nchunks;
@@ -390,6 +499,43 @@ __global__ __launch_bounds__(64, (search_waves_per_simd<CPL, METRIC, BYTES>())) 
     }
   }
 
+  // a hop's rows: candidate j by wave j % TEAM, a row per quad and pass
+  auto team_score = [&](uint32_t nm) {
+    if constexpr (TEAM > 0) {
+      for (uint32_t j = qg * TEAM + (threadIdx.x >> 6), first = 0; first < nm; first += 16 * TEAM, j += 16 * TEAM) {
+        const uint32_t v = cand[j < nm ? j : 0u];
+        float d;
+        if constexpr (CPL == 0) {
+          d = quad_finish<METRIC>(team_partial<METRIC>(team_q, a.vecs + (size_t)v * a.nchunks, ql, a.nchunks, nlimit));
+        } else {
+          RowFrag<CPL> x;
+          load_row_frag<CPL>(a.vecs + (size_t)v * a.nchunks, ql, a.nchunks, true, x);
+          d = score<CPL, METRIC>(a, qf, x, ql, nlimit, intx);
+        }
+        if (ql == 0 && j < nm) team_d[j] = d;
+      }
+    }
+  };
+  if constexpr (TEAM) {
+    if (uniform(threadIdx.x >> 6) != 0u) {  // the helpers: until the searching wave ends
+      while (true) {
+        __syncthreads();  // a hop's candidates are listed
+        const uint32_t nm = uniform(*team_n);
+        if (nm == kTeamDone) return;
+        team_score(nm);
+        __syncthreads();  // their distances are written
+      }
+    }
+  }
+
+  {
+    // 32-bit words of the cache: empty = all ones (ids) or zero (tags)
+    const uint32_t words = a.tag_bits ? (1u << a.hash_bits) / 2u : 1u << a.hash_bits;
+    const uint32_t fill = a.tag_bits ? 0u : kInvalid32;
+    for (uint32_t i = lane; i < words; i += 64) H[i] = fill;
+    for (uint32_t i = lane; i < bw; i += 64) TAG[i] = 0u;  // no position marked
+  }
+
   // B = [(medoid, d(q, medoid))]; at bw <= 64 B lives in registers, one key
   // per lane (`b`), and is written to LDS only for the merge's general path
   // and the epilogue
@@ -410,14 +556,14 @@ __global__ __launch_bounds__(64, (search_waves_per_simd<CPL, METRIC, BYTES>())) 
       d = score<CPL, METRIC>(a, qf, x, ql, nlimit, intx);
     }
     if (lane == 0) b = make_key(d, a.medoid);
-    wave_sync();  // hash table initialised
+    search_sync<(TEAM > 0)>();  // hash table initialised
     if (lane == 0) {
       B[0] = make_key(d, a.medoid);
       seen_test_insert(a, H, a.medoid);
       if constexpr (STATS) atomicOr(&a.seen_bits[(size_t)qid * a.seen_words + (a.medoid >> 5)], 1u << (a.medoid & 31u));
     }
   }
-  wave_sync();
+  search_sync<(TEAM > 0)>();
   uint32_t st_hops = 0, st_deg = 0, st_scored = 1, st_pred = 0;
 
   uint32_t hint = 0, vc = 0, loop = 0;
@@ -457,7 +603,7 @@ __global__ __launch_bounds__(64, (search_waves_per_simd<CPL, METRIC, BYTES>())) 
       if (p < 0) break;
       pk = B[p] | 1ull;
       next_u = uniform(p2 >= 0 ? key_id(B[p2]) : kInvalid32);
-      wave_sync();
+      search_sync<(TEAM > 0)>();
       if (lane == 0) {
         B[p] = pk;
         if (a.visited) a.visited[(size_t)qid * a.max_result + vc] = pk;
@@ -505,7 +651,7 @@ __global__ __launch_bounds__(64, (search_waves_per_simd<CPL, METRIC, BYTES>())) 
       st_scored += nm;
     }
     if (isnew) cand[mbcnt(newm)] = v;
-    wave_sync();
+    search_sync<(TEAM > 0)>();
 
     // ---- score the new neighbours (4 lanes per vector). Once B is full,
     //      a key ranked above B's last cannot enter: B's bw distinct ranks
@@ -516,7 +662,17 @@ __global__ __launch_bounds__(64, (search_waves_per_simd<CPL, METRIC, BYTES>())) 
     uint64_t thr = ~0ull;
     if (cnt == bw) thr = key_rank(regb ? readlane64(b, (int)(bw - 1u)) : B[bw - 1u]);
     uint32_t nt = 0, base = 0;
-    if (bytes) {
+    if (TEAM && nm > kTeamAlone) {
+      if (lane == 0) *team_n = nm;
+      __syncthreads();
+      team_score(nm);
+      __syncthreads();
+      const uint64_t key = make_key(lane < nm ? team_d[lane] : 0.0f, lane < nm ? cand[lane] : 0u);
+      const bool w = lane < nm && key_rank(key) < thr;
+      const uint64_t m = ballot(w);
+      if (w) T[mbcnt(m)] = key;
+      nt = (uint32_t)__builtin_popcountll(m);
+    } else if (bytes) {
       if constexpr (BYTES) {
         if (u8q) {
           for (; base + 16 < nm; base += 32)
@@ -543,7 +699,7 @@ __global__ __launch_bounds__(64, (search_waves_per_simd<CPL, METRIC, BYTES>())) 
       lds_wave_sync();
       continue;
     }
-    wave_sync();
+    search_sync<(TEAM > 0)>();
 
     // ---- sort the new keys, merge them into B
     uint64_t t = lane < nt ? T[lane] : kEmptyKey;
@@ -556,17 +712,21 @@ __global__ __launch_bounds__(64, (search_waves_per_simd<CPL, METRIC, BYTES>())) 
       // B to LDS for the general path
       if (lane < cnt) B[lane] = b;
       hint = 0;
-      wave_sync();
+      search_sync<(TEAM > 0)>();
     }
-    if (!merge_general(B, T, TAG, t, nt, cnt, hint, bw, lane)) {
+    if (!merge_general<(TEAM > 0)>(B, T, TAG, t, nt, cnt, hint, bw, lane)) {
       lds_wave_sync();
       continue;
     }
     if (regb) b = lane < cnt ? B[lane] : kEmptyKey;
   }
+  if constexpr (TEAM) {  // every way out of the loop leads here
+    if (lane == 0) *team_n = kTeamDone;
+    __syncthreads();
+  }
   if (regb) {
     if (lane < cnt) B[lane] = b;
-    wave_sync();
+    search_sync<(TEAM > 0)>();
   }
 
   // ---- output: first k valid, non-deleted entries, then padding
@@ -650,13 +810,13 @@ size_t beam_search_lds_bytes(const Graph& g, const SearchRequest& r) {
          std::max<size_t>(((size_t)1 << hb) * entry, 4);
 }
 
-template <int CPL, int METRIC, bool STATS, bool BYTES = false>
+template <int CPL, int METRIC, bool STATS, bool BYTES = false, int TEAM = 0>
 static void launch_one(const SearchArgs& a, dim3 grid, size_t lds, hipStream_t stream) {
-  auto kern = beam_search_kernel<CPL, METRIC, STATS, BYTES>;
+  auto kern = beam_search_kernel<CPL, METRIC, STATS, BYTES, TEAM>;
   if (lds > 64 * 1024)
     hip_check(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
               "set LDS size");
-  hipLaunchKernelGGL(kern, grid, dim3(64), lds, stream, a);
+  hipLaunchKernelGGL(kern, grid, dim3(TEAM ? 64 * TEAM : 64), lds, stream, a);
 }
 
 void launch_beam_search(const Graph& g, const SearchRequest& r, hipStream_t stream) {
@@ -742,7 +902,44 @@ void launch_beam_search(const Graph& g, const SearchRequest& r, hipStream_t stre
   const size_t lds = beam_search_lds_bytes(g, r);
   const uint32_t cpl = (a.nchunks + 3) / 4;
   const dim3 grid(r.nq);
-  if (a.vecs8 && !stats && g.metric == kL2 && cpl == 4) {
+  a.hash_bytes = (uint32_t)std::max<size_t>(((size_t)1 << a.hash_bits) * (seen_tag_bits(g.n, a.hash_bits) ? 2 : 4), 4);
+  const bool bytes = a.vecs8 && !stats && g.metric == kL2 && cpl == 4;
+  const size_t team_lds = ((lds + 15) & ~(size_t)15) + (cpl > 8 ? (size_t)a.nchunks * 16 : 0) + 64 * 4 + 16;
+  // Teams while every query's waves are resident: 1,024 queries of four waves
+  // at four per SIMD; two waves to 2,048, to 3,072 where the registers allow
+  // six per SIMD (L2 rows of up to 128 values), to 4,096 for streamed rows,
+  // which gain from two waves even in turns. Against one wave per query, bw 64:
+  //   four waves, 1 / 1,000 queries: 128 Gaussian values 1.36x / 1.34x, 200
+  //   values 1.51x / 1.37x, 960 values 2.4x / 1.8x; 96 values by inner product
+  //   1.12x / 1.00x, 384 1.4x / 1.7x; at 2,000 they lose (0.80x on 128 values)
+  //   two waves, 2,000 / 3,000 / 4,000 queries: 128 values 1.06x / 1.05x /
+  //   0.79x, 200 values 1.07x / 0.93x; 960 values 1.14x / 1.10x / 1.15x, 384 by
+  //   inner product 1.66x / 1.29x / 1.33x
+  // Byte rows stay with one wave (1.00x at bw 64, 0.97x at 200): a hop's rows
+  // are one pass of it already.
+  const uint32_t two = cpl > 8 ? 4096u : cpl <= 4 && g.metric == kL2 ? 3072u : 2048u;
+  const uint32_t team = r.nq <= 1024u ? 4u : r.nq <= two ? 2u : 0u;
+  if (team && !bytes && !stats && team_lds <= 160 * 1024) {
+    a.hash_bytes += (uint32_t)(((lds + 15) & ~(size_t)15) - lds);
+#define JA_TEAM(C)                                                                              \
+  case C:                                                                                       \
+    if (g.metric == kL2) {                                                                      \
+      if (team == 4) launch_one<C, kL2, false, false, 4>(a, grid, team_lds, stream);            \
+      else launch_one<C, kL2, false, false, 2>(a, grid, team_lds, stream);                      \
+    } else {                                                                                    \
+      if (team == 4) launch_one<C, kIP, false, false, 4>(a, grid, team_lds, stream);            \
+      else launch_one<C, kIP, false, false, 2>(a, grid, team_lds, stream);                      \
+    }                                                                                           \
+    break;
+    switch (cpl > 8 ? 0u : cpl) {
+      JA_TEAM(0) JA_TEAM(1) JA_TEAM(2) JA_TEAM(3) JA_TEAM(4) JA_TEAM(5) JA_TEAM(6) JA_TEAM(7) JA_TEAM(8)
+      default: throw std::logic_error("unreachable chunks-per-lane case");
+    }
+#undef JA_TEAM
+    hip_check(hipGetLastError(), "launch beam_search_kernel");
+    return;
+  }
+  if (bytes) {
     launch_one<4, kL2, false, true>(a, grid, lds, stream);
     hip_check(hipGetLastError(), "launch beam_search_kernel");
     return;

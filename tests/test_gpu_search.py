@@ -315,3 +315,26 @@ def test_search_host_resident_graph_matches_oracle(jasper, oracle_lib, tmp_path)
         rid, rd = oracle.beam_search(g, q, k=10, beam_width=bw)
         msg = compare_search(ids, d, rid, rd)
         assert msg is None, f"bw={bw}: {msg}"
+
+
+# Launches of few queries run four waves per query (up to 1,024 queries), then
+# two (to 2,048 .. 4,096), larger ones a wave per query: the same bits each way,
+# at every chunk count of a row (streamed ones: part of a batch, whole batches,
+# a last chunk alone), integer rows included.
+@pytest.mark.parametrize("distance,dim,R", [("l2", 8, 64), ("l2", 40, 32), ("ip", 96, 64), ("l2", 128, 64),
+                                            ("ip", 200, 64), ("l2", 256, 64), ("l2", 257, 64), ("l2", 392, 64),
+                                            ("ip", 264, 64), ("ip", 600, 64), ("l2", 960, 64)])
+def test_team_matches_one_wave(jasper, distance, dim, R):
+    rng = np.random.default_rng(dim)
+    base = rng.normal(size=(3000, dim)).astype(np.float16)
+    if dim == 256:
+        base = rng.integers(0, 300, size=(3000, dim)).astype(np.float16)  # integers, no byte rows
+    q = base[rng.choice(3000, size=40, replace=False)] + np.float16(0.25 if dim != 256 else 1)
+    g = jasper.Graph.build(torch.from_numpy(base).cuda(), n_neighbors=R, distance=distance)
+    few = torch.from_numpy(q).cuda()
+    for bw in (16, 64, 150):
+        ids, d = g.search(few.repeat(105, 1), k=10, beam_width=bw)  # 4,200 queries: one wave each
+        for times in (1, 30):
+            idt, dt = g.search(few.repeat(times, 1), k=10, beam_width=bw)
+            assert torch.equal(ids[:40 * times], idt), f"bw={bw}, {40 * times} queries"
+            assert torch.equal(d[:40 * times].view(torch.int32), dt.view(torch.int32)), f"bw={bw}, {40 * times} queries"
