@@ -700,7 +700,7 @@ def run_bruteforce(args, torch, jasper_amd, datasets, dev, log):
                 {"workload": f"config 2 ground truth: {args.nq} queries x {args.n} x 128 fp16, L2, k=10",
                  "queries_per_s": args.nq / (wall / 1000.0)},
                 {"bound": "mfma", "achieved": tf, "peak": 2500.0, "unit": "TFLOP/s", "frac": tf / 2500.0,
-                 "traffic": None, "kernel": "bruteforce_knn (sample scan + bf_filter_kernel + bf_select_kernel)", "kernel_ms": ev,
+                 "traffic": None, "kernel": "bruteforce_knn (rounds of bf_stream_kernel and bf_trim_kernel)", "kernel_ms": ev,
                  "algorithmic_flop_per_launch": flop})
     print(json.dumps(res), flush=True)
     return 0

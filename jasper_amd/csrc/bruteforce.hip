@@ -7,9 +7,8 @@
 // products are exact in fp32, accumulation in fp32); the squared norms are
 // fp32 sums in element order. Ties are ordered by (distance, id).
 //
-// One-pass path, used for small bases (under 16,384 rows; under four samples,
-// 262,144 rows at k = 10, where rows hold up to 128 values), for the threshold
-// sample of the two-pass path and for queries that overflow the other paths:
+// One-pass path, used for small bases (the line is in bruteforce_knn) and for
+// queries that the rounds path leaves over:
 // bf_scan_kernel: one wave owns 32 queries and one chunk of the base. It
 // holds the A fragments of its queries in registers and walks the chunk 32
 // vectors at a time (one 32x32 output tile, K over the padded dim), loading
@@ -21,9 +20,7 @@
 // wave per query merges the chunk lists. Rows longer than 32 K steps (512
 // values, config 4's 960) take the same kernel with the query and base
 // fragments read per slice of 8 K steps.
-// The two-pass path for large bases of rows of up to 128 values is described
-// before bf_filter_kernel, the rounds path for longer rows before
-// bf_tile_kernel.
+// The rounds path for larger bases is described before bf_tile_kernel.
 #include "bruteforce.hpp"
 #include "common.hpp"
 #include "graph.hpp"
@@ -34,6 +31,7 @@
 #include <cstdlib>
 #include <numeric>
 #include <stdexcept>
+#include <type_traits>
 
 namespace jasper_amd {
 
@@ -325,313 +323,9 @@ __global__ __launch_bounds__(64) void bf_merge_kernel(const uint64_t* __restrict
   }
 }
 
-// ----------------------------------------------------------- two-pass path
-// For large bases the exact top-k is found in two passes over a GEMM:
-//  1. the one-pass kernels above on a sample (the first rows of the base:
-//     kBfSample, or more when k * n is large) give
-//     each query the k-th smallest distance T_q of that sample. The true
-//     k-th smallest over the whole base is <= T_q (the sample's k nearest are
-//     k base rows), so every true neighbour has d <= T_q;
-//  2. bf_filter_kernel computes every distance (same arithmetic) and appends
-//     the keys with d <= T_q to a per-query list in HBM (about k * n / sample
-//     entries per query), with no per-query state in the loop, so its
-//     work-groups share one base tile in LDS across 256 (or 128) queries;
-//  3. bf_select_kernel sorts each list by (distance, id) and writes the top k.
-// A query whose list would exceed kBfCandCap is flagged and redone with the
-// one-pass kernels (only its 32-query tile runs). Results are identical to
-// the one-pass path: the same distances, the same (distance, id) order.
-constexpr int64_t kBfSample = 65536;  // smallest sample (larger for large k * n)
-constexpr uint32_t kBfCandCap = 1024;
-constexpr uint32_t kBfLocal = 16;  // candidates a filter work-group stages per query before appending to HBM
-
-// Appends a candidate key to query q's list (a rare path, kept out of line
-// so that its address arithmetic does not occupy registers in the loop).
-__device__ __noinline__ void bf_append(uint32_t* qcount, uint64_t* qcand, uint32_t q, uint64_t key) {
-  const uint32_t slot = atomicAdd(&qcount[q], 1u);
-  if (slot < kBfCandCap) qcand[(size_t)q * kBfCandCap + slot] = key;
-}
-
-// Cooperative base-tile staging of bf_filter_kernel: thread element i is
-// (row srow[i], chunk scol[i]) of the ROWS-row tile starting at v0.
-// (native vector registers: a uint4 struct copied under a condition stays in
-// private memory)
-// offb[i]: the element's byte offset in a whole tile (srow[i] * nck +
-// scol[i] chunks), so a whole tile's loads add a per-thread constant to a
-// uniform base and need no address arithmetic; the chunk's last, partial
-// tile clamps its rows to the chunk.
-template <int PER, int ROWS, int METRIC>
-__device__ __forceinline__ void bf_gload(const uint4* base4, const float* vsq, int64_t v0, int64_t v_begin,
-                                         int64_t v_end, uint32_t nck, uint32_t nel, uint32_t tid,
-                                         const uint32_t (&srow)[PER], const uint32_t (&scol)[PER],
-                                         const uint32_t (&offb)[PER], u32x4 (&stage)[PER], float& svs) {
-  if (v0 + ROWS <= v_end) {
-    const char* tb = reinterpret_cast<const char*>(base4 + (size_t)v0 * nck);
-#pragma unroll
-    for (int i = 0; i < PER; ++i) stage[i] = *reinterpret_cast<const u32x4*>(tb + offb[i]);
-    if constexpr (METRIC == kL2) svs = vsq[v0 + (tid & (uint32_t)(ROWS - 1))];
-    return;
-  }
-#pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    // elements past the tile re-read chunk 0 of the first row and are not stored
-    const bool in = tid + 256u * (uint32_t)i < nel;
-    const int64_t vv = v0 + (in ? srow[i] : 0u);
-    stage[i] = *reinterpret_cast<const u32x4*>(base4 + (size_t)(vv < v_end ? vv : v_begin) * nck + (in ? scol[i] : 0u));
-  }
-  if constexpr (METRIC == kL2) {
-    const int64_t vv = v0 + (tid & (uint32_t)(ROWS - 1));
-    svs = vsq[vv < v_end ? vv : v_begin];
-  }
-}
-
-// The filter's cheap test reads ||v||^2 shrunk by 2^-20 (see bf_filter_kernel).
+constexpr uint32_t kBfCandCap = 1024;  // keys a query's list holds between rounds
+// The tests' cheap form reads ||v||^2 shrunk by 2^-20 (bf_tile_kernel).
 constexpr float kBfVsShrink = 1.0f - 0x1p-20f;
-
-template <int PER, int ROWS>
-__device__ __forceinline__ void bf_sstore(uint4* tile, float* tvs, uint32_t buf, uint32_t rs, uint32_t nel,
-                                          uint32_t tid, const uint32_t (&srow)[PER], const uint32_t (&scol)[PER],
-                                          const u32x4 (&stage)[PER], float svs) {
-#pragma unroll
-  for (int i = 0; i < PER; ++i)
-    if (tid + 256u * (uint32_t)i < nel)
-      *reinterpret_cast<u32x4*>(tile + buf * ROWS * rs + srow[i] * rs + scol[i]) = stage[i];
-  if (tid < (uint32_t)ROWS) {
-    tvs[buf * ROWS + tid] = svs;
-    tvs[2 * ROWS + buf * ROWS + tid] = svs * kBfVsShrink;
-  }
-}
-
-// TILES: 32-query tiles per wave; SUB: 32-row base tiles per step (one
-// barrier per SUB tiles, SUB independent matrix-core chains per query tile).
-// Two waves per SIMD: the pipelined loop's two accumulator sets fit 256
-// registers at up to 128 values per row (config 2, 1M x 128, 5.38 ms ->
-// 4.98 ms against one wave). Longer rows take the rounds path.
-template <int KS, int TILES, int SUB, int METRIC>
-__global__ __launch_bounds__(256, 2) void bf_filter_kernel(const uint16_t* __restrict__ base, int64_t n, uint32_t dp,
-                                                        const uint16_t* __restrict__ queries, int64_t nq,
-                                                        const float* __restrict__ vsq, const float* __restrict__ qsq,
-                                                        const float* __restrict__ qthr, uint32_t thr_stride,
-                                                        int64_t chunk, uint32_t qblocks,
-                                                        uint32_t* __restrict__ qcount,
-                                                        uint64_t* __restrict__ qcand) {
-  // XCD-aware work order: work-groups are dealt to the 8 XCDs round-robin
-  // by id, so work-group p runs on XCD p % 8. Logical item L = (the items of
-  // the XCDs before it) + p / 8, with query block L % qblocks and base chunk
-  // L / qblocks: the query blocks of one chunk run on one XCD together and
-  // read its base tiles through that XCD's L2 (dealt round-robin they would
-  // fetch every tile into all eight L2s).
-  const uint32_t G = gridDim.x, p = blockIdx.x, xcd = p & 7u, per = G >> 3, extra = G & 7u;
-  const uint32_t L = xcd * per + min(xcd, extra) + (p >> 3);
-  const uint32_t qblock = L % qblocks, cblock = L / qblocks;
-  // LDS: two base tiles of ROWS rows, row stride nck + 1 chunks (the extra
-  // chunk is zero: it is the K slot past the row when dp % 16 == 8, and it
-  // staggers the rows across banks); two sets of ROWS squared norms (and
-  // their shrunk copies); per wave and query tile the 32 query norms,
-  // thresholds and cheap-test bounds.
-  //
-  // L2 scores first take a cheap conservative test: y = fl(2 q.v - vs')
-  // >= c_q, with vs' = fl(||v||^2 (1 - 2^-20)) and c_q <= (||q||^2 - T_q) -
-  // 2^-19 (||q||^2 + T_q). Whenever the exact score d = fl(fl(||q||^2 +
-  // ||v||^2) - 2 q.v) satisfies d <= T_q (T_q >= 0), y passes: with u =
-  // 2^-24 and |2 q.v| <= (||q||^2 + ||v||^2)(1 + 128u), d <= T_q gives
-  // 2 q.v - ||v||^2 >= ||q||^2 - T_q - (||q||^2 + ||v||^2 + 2 T_q) u, and y
-  // exceeds 2 q.v - ||v||^2 by at least 11.9 u ||v||^2 - 2.1 u ||q||^2. Only
-  // a 32 x 32 block in which some lane's test passes computes the exact
-  // scores and their appends; the others cost one fma and one compare per
-  // score.
-  constexpr int ROWS = 32 * SUB;
-  extern __shared__ uint4 bf_tile[];
-  const uint32_t nck = dp / 8, rs = nck + 1;
-  float* tvs = reinterpret_cast<float*>(bf_tile + 2 * ROWS * rs);  // [2][ROWS] norms, then [2][ROWS] shrunk
-  float* sqs = tvs + 4 * ROWS;         // [4 waves][TILES][32]
-  float* sth = sqs + 4 * TILES * 32;   // [4 waves][TILES][32]
-  float* scr = sth + 4 * TILES * 32;   // [4 waves][TILES][32] c_q of the cheap test
-  // per wave and query row: a count and kBfLocal staged candidate keys
-  // (wave-private; flushed to the query's HBM list once, at the end)
-  uint32_t* lcnt = reinterpret_cast<uint32_t*>(scr + 4 * TILES * 32);  // [4 waves][TILES * 32]
-  uint64_t* lbuf = reinterpret_cast<uint64_t*>(lcnt + 4 * TILES * 32); // [4 waves][TILES * 32][kBfLocal]
-  const uint32_t tid = threadIdx.x, w = tid >> 6, lane = tid & 63u, am = lane & 31u, ah = lane >> 5;
-  const int64_t qbase = (int64_t)qblock * (128 * TILES) + (int64_t)w * (32 * TILES);
-  for (uint32_t r = lane; r < 32u * TILES; r += 64) lcnt[w * TILES * 32 + r] = 0u;
-  const int64_t v_begin = (int64_t)cblock * chunk;
-  const int64_t v_end = min(n, v_begin + chunk);
-  const uint4* base4 = reinterpret_cast<const uint4*>(base);
-
-  for (uint32_t r = tid; r < 2u * ROWS; r += 256) bf_tile[(r / ROWS) * ROWS * rs + (r % ROWS) * rs + nck] =
-      make_uint4(0, 0, 0, 0);
-  uint4 af[TILES][KS];
-#pragma unroll
-  for (int t = 0; t < TILES; ++t) {
-    const int64_t aq = qbase + 32 * t + am;
-#pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      const uint32_t c = (uint32_t)s * 2 + ah;
-      af[t][s] = (aq < nq && c < nck) ? reinterpret_cast<const uint4*>(queries + (size_t)aq * dp)[c]
-                                      : make_uint4(0, 0, 0, 0);
-    }
-    if (ah == 0) {
-      // a NaN threshold passes nothing (rows past the last query)
-      const float qn = (METRIC == kL2 && aq < nq) ? qsq[aq] : 0.0f;
-      const float th = aq < nq ? qthr[(size_t)aq * thr_stride] : __builtin_nanf("");
-      sqs[(w * TILES + t) * 32 + am] = qn;
-      sth[(w * TILES + t) * 32 + am] = th;
-      // c_q in double, pushed below its own rounding to fp32
-      const double c = ((double)qn - (double)th) - ((double)qn + fabs((double)th)) * 0x1p-19;
-      scr[(w * TILES + t) * 32 + am] = (float)(c - fabs(c) * 0x1p-22);
-    }
-  }
-
-  // cooperative tile loads: thread element i is (row srow[i], chunk scol[i])
-  constexpr int kPer = (ROWS * 2 * KS + 255) / 256;
-  const uint32_t nel = ROWS * nck;
-  uint32_t srow[kPer], scol[kPer], offb[kPer];
-#pragma unroll
-  for (int i = 0; i < kPer; ++i) {
-    const uint32_t e = tid + 256u * (uint32_t)i;
-    srow[i] = e / nck;
-    scol[i] = e % nck;
-    offb[i] = e < nel ? e * 16u : 0u;  // srow * nck + scol chunks; past the tile: chunk 0 of the first row
-  }
-  // base tiles: tile i is in LDS buffer i % 2 while tile i + 1 waits in
-  // registers and tile i + 2 is loading, so a load has two steps of work to
-  // hide behind
-  u32x4 sta[kPer], stb[kPer];
-  float sva = 0.0f, svb = 0.0f;
-  if (v_begin < v_end) {
-    bf_gload<kPer, ROWS, METRIC>(base4, vsq, v_begin, v_begin, v_end, nck, nel, tid, srow, scol, offb, sta, sva);
-    bf_sstore<kPer, ROWS>(bf_tile, tvs, 0u, rs, nel, tid, srow, scol, sta, sva);
-    bf_gload<kPer, ROWS, METRIC>(base4, vsq, v_begin + ROWS, v_begin, v_end, nck, nel, tid, srow, scol, offb, stb, svb);
-  }
-  __syncthreads();
-  // every load issued so far (query fragments, first tiles) completes here:
-  // otherwise the loop's first MFMA waits for all outstanding loads on every
-  // iteration, the prefetched tile included
-  __builtin_amdgcn_s_waitcnt(0);
-  // the cheap test's c_q of this lane's 16 rows per query tile (rows 8g +
-  // 4ah + j), held in registers for the whole loop
-  float cq[TILES][16];
-#pragma unroll
-  for (int t = 0; t < TILES; ++t)
-#pragma unroll
-    for (int g = 0; g < 4; ++g)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) cq[t][4 * g + j] = scr[(w * TILES + t) * 32 + 8 * g + 4 * ah + j];
-  // One tile's products: the chains of every (query tile, base sub-tile)
-  // interleaved; each accumulates over s in order, as bf_scan_kernel does
-  // (the distances must match it bit for bit). The tile's norms are taken
-  // into registers with it, so its LDS buffer is free once the MFMAs are
-  // issued.
-  auto mma = [&](uint32_t buf, float16v (&accs)[TILES][SUB], float (&vs)[SUB], float (&vsm)[SUB]) {
-#pragma unroll
-    for (int t = 0; t < TILES; ++t)
-#pragma unroll
-      for (int u = 0; u < SUB; ++u) accs[t][u] = float16v{};
-#pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      uint4 b[SUB];
-#pragma unroll
-      for (int u = 0; u < SUB; ++u) b[u] = bf_tile[buf * ROWS * rs + (32u * u + am) * rs + (uint32_t)s * 2 + ah];
-#pragma unroll
-      for (int t = 0; t < TILES; ++t)
-#pragma unroll
-        for (int u = 0; u < SUB; ++u)
-          accs[t][u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(u4_as_h8(af[t][s]), u4_as_h8(b[u]), accs[t][u], 0, 0, 0);
-    }
-#pragma unroll
-    for (int u = 0; u < SUB; ++u) {
-      vs[u] = tvs[buf * ROWS + 32u * u + am];
-      vsm[u] = tvs[2 * ROWS + buf * ROWS + 32u * u + am];
-    }
-  };
-  // One tile's tests and appends.
-  auto epi = [&](int64_t v0, const float16v (&accs)[TILES][SUB], const float (&vs)[SUB], const float (&vsm)[SUB]) {
-#pragma unroll
-    for (int u = 0; u < SUB; ++u) {
-      const int64_t v = v0 + 32 * u + am;
-      const bool vok = v < v_end;
-#pragma unroll
-      for (int t = 0; t < TILES; ++t) {
-        const float16v acc = accs[t][u];
-        if constexpr (METRIC == kL2) {
-          uint64_t any = 0;  // lanes with a passing score, one compare mask per score
-#pragma unroll
-          for (int i = 0; i < 16; ++i) any |= ballot(__builtin_fmaf(2.0f, acc[i], -vsm[u]) >= cq[t][i]);
-          if (any == 0) continue;
-        }
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          // rows 8g + 4ah + j, j = 0..3
-          const uint32_t row0 = 8u * (uint32_t)g + 4u * ah;
-          const float4 q4 = *reinterpret_cast<const float4*>(sqs + (w * TILES + t) * 32 + row0);
-          const float4 t4 = *reinterpret_cast<const float4*>(sth + (w * TILES + t) * 32 + row0);
-          const float qsv[4] = {q4.x, q4.y, q4.z, q4.w}, thv[4] = {t4.x, t4.y, t4.z, t4.w};
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            float d;
-            if constexpr (METRIC == kL2) d = __builtin_fmaf(-2.0f, acc[4 * g + j], qsv[j] + vs[u]);
-            else d = -__half2float(__float2half_rn(acc[4 * g + j]));
-            if (vok && d <= thv[j]) {
-              if constexpr (METRIC == kL2) d = d < 0.0f ? 0.0f : d;
-              // staged in LDS (an LDS atomic); a full stage appends to HBM
-              const uint32_t r = (uint32_t)(32 * t + j) + row0;
-              const uint64_t key = bf_key(d, (uint32_t)v);
-              const uint32_t slot = atomicAdd(&lcnt[w * TILES * 32 + r], 1u);
-              if (slot < kBfLocal) lbuf[(size_t)(w * TILES * 32 + r) * kBfLocal + slot] = key;
-              else bf_append(qcount, qcand, (uint32_t)qbase + r, key);
-            }
-          }
-        }
-      }
-    }
-  };
-  // Software pipeline over tiles of ROWS rows: tile i + 1's MFMAs are
-  // issued before tile i's tests, so the matrix cores work while the VALU
-  // runs the tests. Invariant at the loop head: tile v0's products are in
-  // accA, tile v0 + ROWS is in LDS buffer 1 and tile v0 + 2 ROWS is loading
-  // into sta. A tile's LDS buffer is overwritten only after the barrier
-  // that follows its MFMAs' reads. Loads and stores are unconditional
-  // inside the loop (rows past the chunk are clamped reads, stored but
-  // never scored): with a conditional store the compiler cannot prove the
-  // staging registers free at the loop head and waits there for every load
-  // in flight, the prefetch included.
-  float16v accA[TILES][SUB], accB[TILES][SUB];
-  float vsA[SUB], vsmA[SUB], vsB[SUB], vsmB[SUB];
-  if (v_begin < v_end) {
-    mma(0u, accA, vsA, vsmA);
-    bf_sstore<kPer, ROWS>(bf_tile, tvs, 1u, rs, nel, tid, srow, scol, stb, svb);
-    bf_gload<kPer, ROWS, METRIC>(base4, vsq, v_begin + 2 * ROWS, v_begin, v_end, nck, nel, tid, srow, scol, offb, sta,
-                                 sva);
-  }
-  __syncthreads();
-  for (int64_t v0 = v_begin; v0 < v_end; v0 += 2 * ROWS) {
-    const bool more1 = v0 + ROWS < v_end;
-    if (more1) mma(1u, accB, vsB, vsmB);
-    epi(v0, accA, vsA, vsmA);
-    if (!more1) break;
-    // tile v0 + 2 ROWS into buffer 0, tile v0 + 3 ROWS loads into stb
-    bf_sstore<kPer, ROWS>(bf_tile, tvs, 0u, rs, nel, tid, srow, scol, sta, sva);
-    bf_gload<kPer, ROWS, METRIC>(base4, vsq, v0 + 3 * ROWS, v_begin, v_end, nck, nel, tid, srow, scol, offb, stb, svb);
-    __syncthreads();
-    const bool more2 = v0 + 2 * ROWS < v_end;
-    if (more2) mma(0u, accA, vsA, vsmA);
-    epi(v0 + ROWS, accB, vsB, vsmB);
-    if (!more2) break;
-    // tile v0 + 3 ROWS into buffer 1, tile v0 + 4 ROWS loads into sta
-    bf_sstore<kPer, ROWS>(bf_tile, tvs, 1u, rs, nel, tid, srow, scol, stb, svb);
-    bf_gload<kPer, ROWS, METRIC>(base4, vsq, v0 + 4 * ROWS, v_begin, v_end, nck, nel, tid, srow, scol, offb, sta, sva);
-    __syncthreads();
-  }
-  // flush the staged candidates: one HBM slot reservation per query row
-  lds_wave_sync();
-  for (uint32_t r = lane; r < 32u * TILES; r += 64) {
-    const int64_t q = qbase + r;
-    const uint32_t c = min(lcnt[w * TILES * 32 + r], kBfLocal);
-    if (q >= nq || c == 0) continue;
-    const uint32_t at = atomicAdd(&qcount[q], c);
-    for (uint32_t i = 0; i < c && at + i < kBfCandCap; ++i)
-      qcand[(size_t)q * kBfCandCap + at + i] = lbuf[(size_t)(w * TILES * 32 + r) * kBfLocal + i];
-  }
-}
 
 // ------------------------------------------------------------ rounds path
 // The base is scored in rounds over its tiles, in an order that spreads every
@@ -657,13 +351,22 @@ __device__ __forceinline__ void lds_block_sync() {
 // One round over the order's tiles [t0, t1) with the product loop of
 // mfma_gemm.hpp: G::TM queries per work-group, tiles of G::TN base rows, n_ch
 // work-groups per query block taking contiguous parts of the round. The work
-// order is XCD-aware as in bf_filter_kernel: the query blocks of one part run
-// on one XCD and share its L2's copy of the tiles. The base rows' squared
+// order is XCD-aware: work-groups are dealt to the 8 XCDs round-robin by id, so
+// work-group p takes item p / 8 of XCD p % 8's share, and the query blocks of one
+// part run on one XCD and share its L2's copy of the tiles. The base rows' squared
 // norms are summed from the fragments the products read (v_dot2, in the
 // shadow of the MFMAs; each of the WAM waves that read the same fragments
 // takes one K step of a slice), so the base is read once, without a pass of
 // its own for the norms. dense: round 0, every distance to its own slot of
 // dist [nq][kBfFirst] (NaN for rows past the base).
+// L2 scores first take a cheap conservative test: y = fl(2 q.v - vs') >= c_q,
+// with vs' = fl(||v||^2 (1 - 2^-20)) and c_q <= (||q||^2 - T_q) - 2^-19
+// (||q||^2 + |T_q|). Whenever the exact score d = fl(fl(||q||^2 + ||v||^2) -
+// 2 q.v) satisfies d <= T_q, y passes: with u = 2^-24, d <= T_q gives 2 q.v -
+// ||v||^2 >= ||q||^2 - T_q - (||q||^2 + ||v||^2 + 2 |T_q|) u for the same
+// computed q.v and norms, and vs' leaves 14 u ||v||^2, c_q 32 u (||q||^2 +
+// |T_q|) of room. Only a 32 x 32 block in which some lane's test passes
+// computes exact scores, and of its 16 rows per lane those that passed.
 template <class G>
 struct BfTileLds {
   static constexpr uint32_t kLocal = 11;  // keys staged per query
@@ -703,8 +406,8 @@ __global__ __launch_bounds__(G::kThreads, 2) void bf_tile_kernel(
     const float th = q >= nq ? __builtin_nanf("") : dense ? __builtin_inff() : qthr[q];
     sqs[r] = qn;
     sth[r] = th;
-    // L2: the bound of bf_filter_kernel. IP: fp16(q.v) >= -T_q needs q.v >=
-    // -T_q less half an fp16 step; a whole step (or the subnormal step) here.
+    // IP: fp16(q.v) >= -T_q needs q.v >= -T_q less half an fp16 step; a whole
+    // step (or the subnormal step) here.
     const double t = (double)th;
     const double c = METRIC == kL2 ? ((double)qn - t) - ((double)qn + fabs(t)) * 0x1p-19
                                    : -t - fabs(t) * 0x1p-10 - 0x1p-24;
@@ -815,6 +518,249 @@ __global__ __launch_bounds__(G::kThreads, 2) void bf_tile_kernel(
           }
         }
       });
+  if (dense) return;
+  // flush the staged keys: one reservation in the query's list
+  __syncthreads();
+  for (uint32_t r = threadIdx.x; r < (uint32_t)G::TM; r += G::kThreads) {
+    const uint32_t c = min(lcnt[r], kLocal);
+    if (qbase + r >= nq || c == 0) continue;
+    const uint32_t at = atomicAdd(&qcount[qbase + r], c);
+    for (uint32_t i = 0; i < c && at + i < kBfCandCap; ++i)
+      qcand[(size_t)(qbase + r) * kBfCandCap + at + i] = lbuf[(size_t)r * kLocal + i];
+  }
+}
+
+// Rows of up to 128 values: the whole row fits registers, so a wave holds the
+// fragments of 64 queries (64 VGPRs at 128 values) and only the base goes
+// through LDS: 64-row tiles, loaded straight into it two tiles ahead of use
+// (three buffers), each read by the block's four waves (2 x 2 MFMA tiles per
+// wave: 64 bytes of LDS per cycle and CU at the matrix cores' rate, of 128).
+// Two blocks per CU, so one's tests run beside the other's products.
+// L2's cheap test costs 9 VALU instructions per 32 x 32 scores instead of 32:
+// the products start from -c_q / 2 in place of zero and the largest of a
+// lane's 16 sums is compared with ||v||^2 / 2. A block of scores that passes
+// is multiplied again from zero for its exact sums (the
+// scan's, bit for bit). The test's sums carry at most 136 roundings
+// (8 chains of 16 products and the start) of at most (|c_q| + ||q||^2 +
+// ||v||^2) / 2 each, the exact ones as many: with u = 2^-24, c_q <= ||q||^2 -
+// T_q less 2048 u (||q||^2 + |T_q|) and ||v||^2 taken 1024 u smaller leave
+// room for 2 * 136 u (|c_q| + ||q||^2 + ||v||^2) and the distance's own three.
+// IP compares each sum with its bound (its error has no bound without norms).
+// 10k x 1M x 128, k = 10, L2, the whole call: 4.71 ms with thresholds from a
+// scan of 65,536 rows and 32 queries per wave, 3.3 ms this way (the last round
+// 1,014 TFLOP/s); k = 100 by inner product at 96 values 40 -> 6.1 ms.
+template <int KS>
+struct BfStream {
+  static constexpr int TM = 256, TN = 64, kWaves = 4, kThreads = 256, kBuffers = 3;
+  static constexpr uint32_t kLocal = 11;                      // keys staged per query
+  static constexpr int kLoads = (2 * KS + 3) / 4;             // per wave and tile: 1 KB each (nck = 2 KS or one less)
+  static size_t bytes(uint32_t nck) {
+    return (size_t)kBuffers * (TN * nck * 16 + TN * 4) + (size_t)TM * (8 * kLocal + 4 * 4);
+  }
+};
+
+template <class G, int KS, int METRIC>
+__global__ __launch_bounds__(256, 2) void bf_stream_kernel(
+    const uint16_t* __restrict__ base, int64_t n, uint32_t dp, const uint16_t* __restrict__ queries, int64_t nq,
+    const float* __restrict__ qsq, const float* __restrict__ vsq, const float* __restrict__ qthr, uint32_t t0,
+    uint32_t t1, uint32_t n_tiles, uint32_t mul, uint32_t n_ch, uint32_t qblocks, float* __restrict__ dense,
+    uint32_t* __restrict__ qcount, uint64_t* __restrict__ qcand) {
+  extern __shared__ uint4 bf_stream_lds[];
+  constexpr uint32_t kLocal = G::kLocal;
+  const uint32_t nck = dp / 8, tile_bytes = G::TN * nck * 16;
+  char* rows = reinterpret_cast<char*>(bf_stream_lds);                                   // [3][TN][nck]
+  float* norms = reinterpret_cast<float*>(rows + (size_t)G::kBuffers * tile_bytes);     // [3][TN]
+  uint64_t* lbuf = reinterpret_cast<uint64_t*>(norms + G::kBuffers * G::TN);            // [TM][kLocal]
+  float* sqs = reinterpret_cast<float*>(lbuf + (size_t)G::TM * kLocal);                 // [TM] query norms
+  float* sth = sqs + G::TM;                                                             // [TM] thresholds
+  float* scr = sth + G::TM;                                                             // [TM] the products' start
+  uint32_t* lcnt = reinterpret_cast<uint32_t*>(scr + G::TM);                            // [TM]
+  const uint32_t W = gridDim.x, p = blockIdx.x, xcd = p & 7u, per = W >> 3, extra = W & 7u;
+  const uint32_t L = xcd * per + min(xcd, extra) + (p >> 3);
+  const uint32_t qblock = L % qblocks, ch = L / qblocks;
+  const uint32_t total = t1 - t0, each = total / n_ch, more = total % n_ch;
+  const uint32_t first = t0 + ch * each + min(ch, more), count = each + (ch < more ? 1u : 0u);
+  const int64_t qbase = (int64_t)qblock * G::TM;
+  for (uint32_t r = threadIdx.x; r < (uint32_t)G::TM; r += G::kThreads) {
+    const int64_t q = qbase + r;
+    // a NaN threshold passes nothing (rows past the last query)
+    const float qn = (METRIC == kL2 && q < nq) ? qsq[q] : 0.0f;
+    const float th = q >= nq ? __builtin_nanf("") : dense ? __builtin_inff() : qthr[q];
+    sqs[r] = qn;
+    sth[r] = th;
+    const double t = (double)th;
+    if (METRIC == kL2) {
+      const double c = ((double)qn - t) - ((double)qn + fabs(t)) * 0x1p-13;
+      scr[r] = dense ? 0.0f : (float)(-0.5 * c);
+    } else {
+      const double c = -t - fabs(t) * 0x1p-10 - 0x1p-24;
+      scr[r] = (float)(c - fabs(c) * 0x1p-22);
+    }
+    lcnt[r] = 0u;
+  }
+  const uint32_t lane = threadIdx.x & 63u, wave = uniform(threadIdx.x >> 6), am = lane & 31u, ah = lane >> 5;
+  // a row's chunk c sits at slot (c + f(r)) mod nck, which spreads eight
+  // consecutive rows' equal chunks over the banks: row starts repeat every
+  // 8 / g rows (mod 128 bytes), g = gcd(nck, 8)
+  const uint32_t g8 = nck & (0u - nck), g = min(g8, 8u), gshift = 3u - (uint32_t)__builtin_ctz(g);
+  auto turn = [&](uint32_t r) { return (r >> gshift) & (g - 1u); };
+  uint32_t off[G::kLoads], lrow[G::kLoads];  // this lane's piece of load j: byte offset in a whole tile, row
+#pragma unroll
+  for (int j = 0; j < G::kLoads; ++j) {
+    const uint32_t e = min((uint32_t)j * G::kWaves + wave, nck - 1u) * 64u + lane;  // (the last kilobyte again)
+    const uint32_t r = e / nck, slot = e % nck, f = turn(r) % nck;
+    const uint32_t c = slot >= f ? slot - f : slot + nck - f;
+    lrow[j] = r;
+    off[j] = (r * nck + c) * 16u;
+  }
+  auto issue = [&](uint32_t tile, uint32_t buf) {
+    const int64_t v0 = (int64_t)tile * G::TN;
+    const char* tb = reinterpret_cast<const char*>(base) + (size_t)v0 * nck * 16;
+    const bool whole = v0 + G::TN <= n;
+#pragma unroll
+    for (int j = 0; j < G::kLoads; ++j) {
+      uint32_t o = off[j];
+      if (!whole && v0 + lrow[j] >= n) o -= (uint32_t)(v0 + lrow[j] - (n - 1)) * nck * 16u;  // the last row again
+      const uint32_t kb = min((uint32_t)j * G::kWaves + wave, nck - 1u);
+      gemm_load_lds16(tb + o, rows + (size_t)buf * tile_bytes + kb * 1024u);
+    }
+    if constexpr (METRIC == kL2)
+      __builtin_amdgcn_global_load_lds((gemm_glb_void*)(vsq + min(v0 + (int64_t)lane, n - 1)),
+                                       (gemm_lds_void*)(norms + buf * G::TN), 4, 0, 0);
+  };
+  half8 af[2][KS];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const int64_t aq = qbase + 64 * wave + 32 * t + am;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const uint32_t c = (uint32_t)s * 2 + ah;
+      af[t][s] = u4_as_h8((aq < nq && c < nck) ? reinterpret_cast<const uint4*>(queries + (size_t)aq * dp)[c]
+                                               : make_uint4(0, 0, 0, 0));
+    }
+  }
+  const uint32_t fr = turn(am) % nck, fr32 = turn(am + 32u) % nck;
+  const bool odd = (nck & 1u) != 0;
+  auto frag = [&](uint32_t buf, int u, int s) {
+    const uint32_t f = u ? fr32 : fr;
+    uint32_t slot = (uint32_t)s * 2 + ah + f;
+    slot = slot >= nck ? slot - nck : slot;
+    slot = slot >= nck ? 0u : slot;  // (the K slot past an odd row)
+    half8 b = *reinterpret_cast<const half8*>(rows + (size_t)buf * tile_bytes + ((32u * u + am) * nck + slot) * 16u);
+    if (s == KS - 1 && odd && ah) b = half8{};
+    return b;
+  };
+  __syncthreads();
+  float16v start[2];  // L2: -c_q / 2 of this lane's rows; IP: the bounds themselves
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) start[t][i] = scr[64 * wave + 32 * t + 8 * (i >> 2) + 4 * ah + (i & 3)];
+  uint32_t next = bf_tile_at(first, mul, n_tiles), here = next;
+  auto advance = [&](uint32_t x) {
+    x += mul;
+    return x >= n_tiles ? x - n_tiles : x;
+  };
+  uint32_t nb = 0, cb = 0;
+  for (uint32_t k = 0; k < 2 && k < count; ++k) {
+    issue(next, nb);
+    next = advance(next);
+    nb = nb == 2 ? 0 : nb + 1;
+  }
+  for (uint32_t it = 0; it < count; ++it) {
+    // this tile's loads have landed (the next one's may be in flight), and
+    // every wave is done with the buffer that the one after goes to
+    constexpr int kInFlight = G::kLoads + (METRIC == kL2 ? 1 : 0);
+    if (it + 1 < count) __builtin_amdgcn_s_waitcnt(kInFlight | 0x70);
+    else __builtin_amdgcn_s_waitcnt(0x70);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (it + 2 < count) {
+      issue(next, nb);
+      next = advance(next);
+      nb = nb == 2 ? 0 : nb + 1;
+    }
+    float16v acc[2][2];
+    half8 b[2][2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) b[0][u] = frag(cb, u, 0);
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      if (s + 1 < KS) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) b[(s + 1) & 1][u] = frag(cb, u, s + 1);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+          acc[t][u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+              af[t][s], b[s & 1][u], s ? acc[t][u] : METRIC == kL2 ? start[t] : float16v{}, 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int64_t v = (int64_t)here * G::TN + 32 * u + am;
+      const float vn = METRIC == kL2 ? norms[cb * G::TN + 32 * u + am] : 0.0f;
+      const float half = 0.5f * (vn * (1.0f - 0x1p-14f));
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        bool hit;
+        if constexpr (METRIC == kL2) {
+          float m = acc[t][u][0];
+#pragma unroll
+          for (int i = 1; i < 16; ++i) m = fmaxf(m, acc[t][u][i]);
+          hit = m >= half;
+        } else {
+          hit = false;
+#pragma unroll
+          for (int i = 0; i < 16; ++i) hit = hit || acc[t][u][i] >= start[t][i];
+        }
+        if (ballot(hit) == 0 && !dense) continue;
+        float16v sum = {};
+        if constexpr (METRIC == kL2) {
+#pragma unroll
+          for (int s = 0; s < KS; ++s)
+            sum = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[t][s], frag(cb, u, s), sum, 0, 0, 0);
+        } else {
+          sum = acc[t][u];
+        }
+        // rows r0 + 8g + j of this lane; opaque, or the compiler forms every
+        // row's addresses once for the whole walk and spills
+        uint32_t r0 = 64 * wave + 32 * t + 4 * ah;
+        asm volatile("" : "+v"(r0));
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          // most of a passing block's 16 rows have no passing score
+          if (!dense && ballot(METRIC == kL2 ? acc[t][u][i] >= half : acc[t][u][i] >= start[t][i]) == 0) continue;
+          const uint32_t r = r0 + 8 * (i >> 2) + (i & 3);
+          float d;
+          if constexpr (METRIC == kL2) d = __builtin_fmaf(-2.0f, sum[i], sqs[r] + vn);
+          else d = -__half2float(__float2half_rn(sum[i]));
+          const bool pass = v < n && d <= sth[r];
+          if constexpr (METRIC == kL2) d = d < 0.0f ? 0.0f : d;
+          if (dense) {
+            const int64_t q = qbase + r;
+            if (q < nq)
+              dense[(size_t)q * kBfFirst + (first + it) * G::TN + 32 * u + am] = pass ? d : __builtin_nanf("");
+          } else if (pass) {
+            const uint64_t key = bf_key(d, (uint32_t)v);
+            const uint32_t s = atomicAdd(&lcnt[r], 1u);
+            if (s < kLocal) lbuf[(size_t)r * kLocal + s] = key;
+            else {
+              const size_t q = (size_t)qbase + r;
+              const uint32_t at = atomicAdd(&qcount[q], 1u);
+              if (at < kBfCandCap) qcand[q * kBfCandCap + at] = key;
+            }
+          }
+        }
+      }
+    }
+    here = advance(here);
+    cb = cb == 2 ? 0 : cb + 1;
+  }
   if (dense) return;
   // flush the staged keys: one reservation in the query's list
   __syncthreads();
@@ -1006,36 +952,6 @@ __global__ void bf_clear_kernel(uint8_t* __restrict__ flags, int64_t n, uint32_t
   if (i == 0) *word = 0;
 }
 
-// Per query: sort the candidate list by (distance, id) and write the best k;
-// a list that overflowed flags the query (and its 32-query tile) for the
-// one-pass kernels.
-__global__ __launch_bounds__(64) void bf_select_kernel(const uint32_t* __restrict__ qcount,
-                                                       const uint64_t* __restrict__ qcand, int64_t nq, uint32_t k,
-                                                       int32_t* __restrict__ out_ids, float* __restrict__ out_d,
-                                                       uint8_t* __restrict__ q_flags, uint8_t* __restrict__ tile_flags) {
-  __shared__ uint64_t buf[kBfCandCap];
-  const int64_t q = blockIdx.x;
-  const uint32_t lane = threadIdx.x;
-  const uint32_t cnt = qcount[q];
-  if (cnt > kBfCandCap) {
-    if (lane == 0) {
-      q_flags[q] = 1;
-      tile_flags[q >> 5] = 1;
-    }
-    return;
-  }
-  const uint32_t N = max(pow2_ceil(cnt), 2u);
-  const uint64_t* src = qcand + (size_t)q * kBfCandCap;
-  for (uint32_t i = lane; i < N; i += 64) buf[i] = i < cnt ? src[i] : ~0ull;
-  wave_sync();
-  lds_bitonic_sort(buf, N);
-  for (uint32_t i = lane; i < k; i += 64) {
-    const uint64_t key = i < N ? buf[i] : ~0ull;
-    out_ids[(size_t)q * k + i] = key == ~0ull ? -1 : (int32_t)(uint32_t)key;
-    out_d[(size_t)q * k + i] = key == ~0ull ? FLT_MAX : ord_to_dist((uint32_t)(key >> 32));
-  }
-}
-
 // The one-pass path (scan + merge) over base rows [0, n), for all queries or
 // only the flagged ones.
 static void bf_one_pass(const void* base, int64_t n, uint32_t dp, const void* queries, int64_t nq, uint32_t k,
@@ -1045,8 +961,8 @@ static void bf_one_pass(const void* base, int64_t n, uint32_t dp, const void* qu
   // chunks: each a multiple of 64 vectors (a whole number of 32-vector steps)
   // about 2,048 work-groups (single waves): longer chunks spend fewer of
   // their steps filling and compacting the buffers before the threshold
-  // settles (config 2's 65,536-row sample: 8,192 work-groups 6.24 ms per
-  // ground-truth call, 4,096 5.62, 2,048 5.44, 1,024 5.77);
+  // settles (65,536 x 128 rows, 10k queries: 8,192 work-groups took 0.80 ms
+  // longer, 4,096 0.18, 1,024 0.33);
   // JASPER_BF_SCAN_WGS overrides it (tuning)
   const int64_t qtiles = (nq + 31) / 32;
   static const int64_t target = [] {
@@ -1064,8 +980,8 @@ static void bf_one_pass(const void* base, int64_t n, uint32_t dp, const void* qu
   // every row's threshold reloaded) once it holds more than cap - kBfStep
   // keys, so at k = 10 the 48 slots of k + kBfStep compacted each query
   // after every 6 or so new candidates; 64 allow 22 between compactions
-  // and keep all of config 2's 1,878 work-groups resident (18.4 KB of LDS
-  // each): its 65,536-row sample scan 0.90 -> 0.77 ms
+  // and keep the 1,878 work-groups of 10k queries resident (18.4 KB of LDS
+  // each): 65,536 x 128 rows 0.90 -> 0.77 ms
   const uint32_t cap = std::max<uint32_t>((k + kBfStep + 7u) & ~7u, 64u);
   const size_t lds = ((size_t)32 * cap + kBfScratch) * 8;
   auto go = [&](auto kern) {
@@ -1094,90 +1010,25 @@ static void bf_one_pass(const void* base, int64_t n, uint32_t dp, const void* qu
   (void)hipFreeAsync(lists, s);
 }
 
-template <int KS, int SUB, int METRIC>
-static void launch_filter_sub(const void* base, int64_t n, uint32_t dp, const void* queries, int64_t nq,
-                              const float* vsq, const float* qsq, const float* qthr, uint32_t thr_stride,
-                              uint32_t* qcount, uint64_t* qcand, hipStream_t s) {
-  // one 32-query tile per wave: two (208 VGPRs) and three (272) measured
-  // 7.48 and 11.7 ms against 7.15 ms on config 2's 10k x 1M ground truth
-  constexpr int TILES = 1;
-  const int64_t qblocks = (nq + 128 * TILES - 1) / (128 * TILES);
-  // about 2,500 work-groups in a 1-D grid that the kernel maps to (query
-  // block, chunk) so that one chunk's query blocks share an XCD
-  int64_t want = std::max<int64_t>(1, 2560 / qblocks);
-  want = std::min<int64_t>(want, (n + 31) / 32);
-  const int64_t chunk = ((n + want - 1) / want + 31) / 32 * 32;
-  const uint32_t n_chunks = (uint32_t)((n + chunk - 1) / chunk);
-  const uint32_t rs = dp / 8 + 1;
-  const size_t lds = (size_t)2 * 32 * SUB * rs * 16 + 4 * 32 * SUB * 4 + (size_t)3 * 4 * TILES * 32 * 4 +
-                     (size_t)4 * TILES * 32 * (4 + 8 * kBfLocal);
-  auto kern = bf_filter_kernel<KS, TILES, SUB, METRIC>;
-  if (lds > 64 * 1024)
-    hip_check(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), "LDS");
-  hipLaunchKernelGGL(kern, dim3((uint32_t)qblocks * n_chunks), dim3(256), lds, s, (const uint16_t*)base, n, dp,
-                     (const uint16_t*)queries, nq, vsq, qsq, qthr, thr_stride, chunk, (uint32_t)qblocks, qcount,
-                     qcand);
-  hip_check(hipGetLastError(), "launch bf_filter_kernel");
-}
-
-template <int KS, int METRIC>
-static void launch_filter(const void* base, int64_t n, uint32_t dp, const void* queries, int64_t nq,
-                          const float* vsq, const float* qsq, const float* qthr, uint32_t thr_stride,
-                          uint32_t* qcount, uint64_t* qcand, hipStream_t s) {
-  // 64-row steps (two 32-row tiles, two chains per wave): 6.25 ms against
-  // 6.73 ms with 32-row steps on config 2's ground truth; JASPER_BF_SUB=1
-  // selects the latter (tuning)
-  static const int sub = [] {
-    const char* e = std::getenv("JASPER_BF_SUB");
-    return e ? std::atoi(e) : 2;
-  }();
-  if (sub == 1)
-    launch_filter_sub<KS, 1, METRIC>(base, n, dp, queries, nq, vsq, qsq, qthr, thr_stride, qcount, qcand, s);
-  else
-    launch_filter_sub<KS, 2, METRIC>(base, n, dp, queries, nq, vsq, qsq, qthr, thr_stride, qcount, qcand, s);
-}
-
-template <int METRIC>
-static void dispatch_filter(uint32_t ks, const void* base, int64_t n, uint32_t dp, const void* queries, int64_t nq,
-                            const float* vsq, const float* qsq, const float* qthr, uint32_t thr_stride,
-                            uint32_t* qcount, uint64_t* qcand, hipStream_t s) {
-  switch (ks) {
-#define JA_F(K) \
-  case K: launch_filter<K, METRIC>(base, n, dp, queries, nq, vsq, qsq, qthr, thr_stride, qcount, qcand, s); break;
-    JA_F(1) JA_F(2) JA_F(3) JA_F(4) JA_F(5) JA_F(6) JA_F(7) JA_F(8)
-#undef JA_F
-    default: throw std::invalid_argument("bruteforce_knn: unsupported dim");
-  }
-}
-
 // Scores the whole base in rounds and writes the results; flags (cleared by
-// the caller) name the queries that are left to the one-pass kernels.
-template <class G>
-static void bf_rounds(const void* base, int64_t n, uint32_t dp, const void* queries, int64_t nq, uint32_t k,
-                      int metric, const float* qsq, float* qthr, float* dense, uint32_t* qcount, uint64_t* qcand,
-                      uint8_t* q_flags, uint8_t* tile_flags, int32_t* out_ids, float* out_d, hipStream_t s) {
+// the caller) name the queries that are left to the one-pass kernels. G: the
+// tiles; round(parts, t0, t1, mul, dist): launches one round.
+template <class G, class Round>
+static void bf_rounds(int64_t n, int64_t nq, uint32_t k, float* dense, uint32_t* qcount, uint64_t* qcand, float* qthr,
+                      uint8_t* q_flags, uint8_t* tile_flags, int32_t* out_ids, float* out_d, hipStream_t s,
+                      Round round) {
   const uint32_t n_tiles = (uint32_t)((n + G::TN - 1) / G::TN);
   const uint32_t qblocks = (uint32_t)((nq + G::TM - 1) / G::TM);
   uint32_t mul = std::max<uint32_t>(1u, (uint32_t)(0.6180339887 * n_tiles));
   while (std::gcd(mul, n_tiles) != 1u) ++mul;
-  constexpr size_t lds = BfTileLds<G>::bytes;
   // work-groups the chip holds at once: eight waves per CU (two per SIMD)
   constexpr uint32_t kResident = 256u * (8 / G::kWaves);
-  auto go = [&](auto kern, uint32_t t0, uint32_t t1, float* dist) {
-    hip_check(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), "LDS");
-    const uint32_t parts = gemm_parts(qblocks, t1 - t0, kResident);
-    hipLaunchKernelGGL(kern, dim3(qblocks * parts), dim3(G::kThreads), lds, s, (const uint16_t*)base, n, dp,
-                       (const uint16_t*)queries, nq, qsq, (const float*)qthr, t0, t1, n_tiles, mul, parts, qblocks,
-                       dist, qcount, qcand);
-    hip_check(hipGetLastError(), "launch bf_tile_kernel");
-  };
   constexpr uint32_t kFirstTiles = kBfFirst / G::TN;
   static_assert(kFirstTiles * G::TN == kBfFirst, "round 0 is whole tiles");
   uint32_t t0 = 0, t1 = kFirstTiles;  // n >= 4 kBfFirst
   while (true) {
-    float* dist = t0 == 0 ? dense : nullptr;
-    if (metric == kL2) go(bf_tile_kernel<G, kL2>, t0, t1, dist);
-    else go(bf_tile_kernel<G, kIP>, t0, t1, dist);
+    round(gemm_parts(qblocks, t1 - t0, kResident), qblocks, t0, t1, n_tiles, mul, t0 == 0 ? dense : nullptr);
+    hip_check(hipGetLastError(), "launch a brute-force round");
     const bool last = t1 == n_tiles;
     auto trim = [&](auto kern, uint32_t threads) {
       hipLaunchKernelGGL(kern, dim3((uint32_t)nq), dim3(threads), 0, s, (const float*)dense, mul, n_tiles, qcount,
@@ -1187,10 +1038,12 @@ static void bf_rounds(const void* base, int64_t n, uint32_t dp, const void* quer
     if (t0 == 0) trim(bf_trim_kernel<G::TN>, 256);
     else trim(bf_trim_kernel<0>, 64);
     if (last) break;
-    // the last two rounds grow fourfold (few candidates where most rows
-    // are), earlier ones 16-fold where a list holds 16 k keys with room
+    // fourfold: about 3 k candidates per query and round, few where most rows
+    // are. With few queries, where a round is mostly its launches, one step of
+    // 16 (a list holds 16 k keys with room at k <= 32); with 10k queries it
+    // cost 0.25 ms more in exact scores than the round it saves
     t0 = t1;
-    const uint64_t grow = k <= 32 && (uint64_t)t1 * 64 <= n_tiles ? 16 : 4;
+    const uint64_t grow = k <= 32 && nq <= 1024 && (uint64_t)t1 * 64 <= n_tiles ? 16 : 4;
     t1 = (uint32_t)std::min<uint64_t>(n_tiles, (uint64_t)t1 * grow);
   }
 }
@@ -1215,20 +1068,70 @@ static void bf_in_rounds(const void* base, int64_t n, uint32_t dim, uint32_t dp,
   hip_check(hipMallocAsync((void**)&flags, (size_t)(nq + ntiles), s), "alloc overflow flags");
   hipLaunchKernelGGL(bf_clear_kernel, dim3((uint32_t)((nq + ntiles + 255) / 256)), dim3(256), 0, s, flags,
                      nq + ntiles, qcount + nq);
+  const uint32_t* flagged = qcount + nq;
+  const uint16_t* base16 = (const uint16_t*)base;
+  const uint16_t* queries16 = (const uint16_t*)queries;
   if (metric == kL2) {
     hip_check(hipMallocAsync((void**)&qsq, (size_t)nq * 4, s), "alloc query norms");
     hip_check(hipMallocAsync((void**)&vsq, (size_t)n * 4, s), "alloc base norms");
-    hipLaunchKernelGGL(bf_query_sqnorm_kernel, dim3((uint32_t)((nq + 3) / 4)), dim3(256), 0, s,
-                       (const uint16_t*)queries, nq, dp, qsq);
   }
-  // 256 queries per work-group at 991 TFLOP/s or 128 at 850 (mfma_gemm.hpp),
-  // whichever finishes the padded queries first
-  const uint64_t by256 = (uint64_t)((nq + 255) / 256) * 256 * 850, by128 = (uint64_t)((nq + 127) / 128) * 128 * 991;
-  auto rounds = by256 <= by128 ? bf_rounds<GemmTile<2, 4, 4, 2, 8>> : bf_rounds<GemmTile<2, 4, 2, 2, 4>>;
-  rounds(base, n, dp, queries, nq, k, metric, qsq, qthr, dense, qcount, qcand, flags, flags + nq, out_ids, out_d, s);
-  if (metric == kL2) {
-    hipLaunchKernelGGL(row_sqnorm_kernel, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, s, (const uint16_t*)base, n,
-                       dp, dim, vsq, (const uint32_t*)(qcount + nq));
+  auto norms = [&](const uint16_t* x, int64_t rows, float* out, const uint32_t* wanted) {
+    hipLaunchKernelGGL(row_sqnorm_kernel, dim3((uint32_t)((rows + 255) / 256)), dim3(256), 0, s, x, rows, dp, dim, out,
+                       wanted);
+  };
+  if (dp <= 128) {
+    if (metric == kL2) {
+      norms(queries16, nq, qsq, nullptr);
+      norms(base16, n, vsq, nullptr);
+    }
+    auto go = [&](auto tag) {
+      constexpr int KS = decltype(tag)::value;
+      using G = BfStream<KS>;
+      const size_t lds = G::bytes(dp / 8);
+      auto kern = metric == kL2 ? bf_stream_kernel<G, KS, kL2> : bf_stream_kernel<G, KS, kIP>;
+      if (lds > 64 * 1024)
+        hip_check(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), "LDS");
+      bf_rounds<G>(n, nq, k, dense, qcount, qcand, qthr, flags, flags + nq, out_ids, out_d, s,
+                   [&](uint32_t parts, uint32_t qblocks, uint32_t t0, uint32_t t1, uint32_t n_tiles, uint32_t mul,
+                       float* dist) {
+                     hipLaunchKernelGGL(kern, dim3(qblocks * parts), dim3(G::kThreads), lds, s, base16, n, dp,
+                                        queries16, nq, (const float*)qsq, (const float*)vsq, (const float*)qthr, t0,
+                                        t1, n_tiles, mul, parts, qblocks, dist, qcount, qcand);
+                   });
+    };
+    switch ((dp + 15) / 16) {
+      case 1: go(std::integral_constant<int, 1>{}); break;
+      case 2: go(std::integral_constant<int, 2>{}); break;
+      case 3: go(std::integral_constant<int, 3>{}); break;
+      case 4: go(std::integral_constant<int, 4>{}); break;
+      case 5: go(std::integral_constant<int, 5>{}); break;
+      case 6: go(std::integral_constant<int, 6>{}); break;
+      case 7: go(std::integral_constant<int, 7>{}); break;
+      default: go(std::integral_constant<int, 8>{}); break;
+    }
+  } else {
+    if (metric == kL2)
+      hipLaunchKernelGGL(bf_query_sqnorm_kernel, dim3((uint32_t)((nq + 3) / 4)), dim3(256), 0, s, queries16, nq, dp,
+                         qsq);
+    auto go = [&](auto tile) {
+      using G = decltype(tile);
+      constexpr size_t lds = BfTileLds<G>::bytes;
+      auto kern = metric == kL2 ? bf_tile_kernel<G, kL2> : bf_tile_kernel<G, kIP>;
+      hip_check(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), "LDS");
+      bf_rounds<G>(n, nq, k, dense, qcount, qcand, qthr, flags, flags + nq, out_ids, out_d, s,
+                   [&](uint32_t parts, uint32_t qblocks, uint32_t t0, uint32_t t1, uint32_t n_tiles, uint32_t mul,
+                       float* dist) {
+                     hipLaunchKernelGGL(kern, dim3(qblocks * parts), dim3(G::kThreads), lds, s, base16, n, dp,
+                                        queries16, nq, (const float*)qsq, (const float*)qthr, t0, t1, n_tiles, mul,
+                                        parts, qblocks, dist, qcount, qcand);
+                   });
+    };
+    // 256 queries per work-group at 991 TFLOP/s or 128 at 850 (mfma_gemm.hpp),
+    // whichever finishes the padded queries first
+    const uint64_t by256 = (uint64_t)((nq + 255) / 256) * 256 * 850, by128 = (uint64_t)((nq + 127) / 128) * 128 * 991;
+    if (by256 <= by128) go(GemmTile<2, 4, 4, 2, 8>{});
+    else go(GemmTile<2, 4, 2, 2, 4>{});
+    if (metric == kL2) norms(base16, n, vsq, flagged);  // for the flagged queries, if there are any
   }
   bf_one_pass(base, n, dp, queries, nq, k, metric, vsq, qsq, out_ids, out_d, flags + nq, flags, s);
   (void)hipFreeAsync(qthr, s);
@@ -1248,12 +1151,22 @@ void bruteforce_knn(const void* base, int64_t n, uint32_t dim, uint32_t dp, cons
   if (n <= 0) throw std::invalid_argument("empty base");
   if (n > 0x7FFFFFFFll) throw std::invalid_argument("too many base vectors");
   if (nq > 0x7FFFFFFFll) throw std::invalid_argument("too many queries");
-  // rows of more than 128 values: rounds (1M x 256, 3,750 queries, k = 10:
-  // 5.1 ms with the two passes below, 3.4 ms; 1M x 480, 2,000 queries, k =
-  // 100: 26.6 and 3.8 ms). Below 4 kBfFirst rows the one-pass kernels: round 0
-  // alone would be a quarter of the base.
-  if (dp > 128 && n >= 4 * (int64_t)kBfFirst) {
-    bf_in_rounds(base, n, dim, dp, queries, nq, k, metric, out_ids, out_d, s);
+  // Rounds from 16,384 rows on (round 0 alone is 4,096). At small k, bases
+  // that the one-pass kernels scan before the rounds' launches and trims are
+  // done stay with them: below 65,536 rows of up to 128 values (20,000 x 128,
+  // k = 1, 10k queries: 0.36 ms in one pass, 0.47 in rounds; 65,536 rows 0.77
+  // and 0.60) and below 262,144 of up to 256 (100,000 x 136, k = 1, 7,000
+  // queries: 0.63 and 0.75; 1M x 256, k = 10, 3,750: 5.1 and 3.4). Longer rows
+  // (40,000 x 384, k = 10, 2,000 queries: 0.58 and 0.31) and larger k (50,000
+  // x 64, k = 32: 3.1 and 0.8), where the scan's buffers are compacted ever
+  // more often, do not.
+  const int64_t scanned = k > 16 || dp > 256 ? 0 : dp > 128 ? 262144 : 65536;
+  if (n >= std::max<int64_t>(4 * (int64_t)kBfFirst, scanned)) {
+    // the scratch is 24 KB per query: 1.6 GB for a block of queries
+    constexpr int64_t kBlock = 65536;
+    for (int64_t q = 0; q < nq; q += kBlock)
+      bf_in_rounds(base, n, dim, dp, (const uint16_t*)queries + (size_t)q * dp, std::min(kBlock, nq - q), k, metric,
+                   out_ids + (size_t)q * k, out_d + (size_t)q * k, s);
     return;
   }
   float* vsq = nullptr;
@@ -1266,43 +1179,7 @@ void bruteforce_knn(const void* base, int64_t n, uint32_t dim, uint32_t dp, cons
     hipLaunchKernelGGL(row_sqnorm_kernel, dim3((uint32_t)((nq + 255) / 256)), dim3(256), 0, s,
                        (const uint16_t*)queries, nq, dp, dim, qsq, nullptr);
   }
-  // the two-pass path: a sample
-  // large enough that a query's filtered list (about k * n / sample keys)
-  // stays near half of kBfCandCap
-  const int64_t sample = std::max<int64_t>(kBfSample, ((int64_t)2 * k * n / kBfCandCap + 63) / 64 * 64);
-  if (n < 4 * sample || dp > 128) {
-    bf_one_pass(base, n, dp, queries, nq, k, metric, vsq, qsq, out_ids, out_d, nullptr, nullptr, s);
-  } else {
-    // 1. thresholds from the sample rows [0, sample)
-    int32_t* sid = nullptr;
-    float* sd = nullptr;
-    uint32_t* qcount = nullptr;
-    uint64_t* qcand = nullptr;
-    uint8_t* flags = nullptr;  // [nq] query flags, then [ceil(nq / 32)] tile flags
-    const int64_t ntiles = (nq + 31) / 32;
-    hip_check(hipMallocAsync((void**)&sid, (size_t)nq * k * 4, s), "alloc sample ids");
-    hip_check(hipMallocAsync((void**)&sd, (size_t)nq * k * 4, s), "alloc sample dists");
-    hip_check(hipMallocAsync((void**)&qcount, (size_t)nq * 4, s), "alloc candidate counts");
-    hip_check(hipMallocAsync((void**)&qcand, (size_t)nq * kBfCandCap * 8, s), "alloc candidate lists");
-    hip_check(hipMallocAsync((void**)&flags, (size_t)(nq + ntiles), s), "alloc overflow flags");
-    hip_check(hipMemsetAsync(qcount, 0, (size_t)nq * 4, s), "clear candidate counts");
-    hip_check(hipMemsetAsync(flags, 0, (size_t)(nq + ntiles), s), "clear overflow flags");
-    bf_one_pass(base, sample, dp, queries, nq, k, metric, vsq, qsq, sid, sd, nullptr, nullptr, s);
-    // 2. every distance against the thresholds (the k-th sample distance)
-    const uint32_t ks = (dp + 15) / 16;
-    if (metric == kL2) dispatch_filter<kL2>(ks, base, n, dp, queries, nq, vsq, qsq, sd + (k - 1), k, qcount, qcand, s);
-    else dispatch_filter<kIP>(ks, base, n, dp, queries, nq, vsq, qsq, sd + (k - 1), k, qcount, qcand, s);
-    // 3. select, and redo overflowed queries in one pass
-    hipLaunchKernelGGL(bf_select_kernel, dim3((uint32_t)nq), dim3(64), 0, s, (const uint32_t*)qcount,
-                       (const uint64_t*)qcand, nq, k, out_ids, out_d, flags, flags + nq);
-    hip_check(hipGetLastError(), "launch bf_select_kernel");
-    bf_one_pass(base, n, dp, queries, nq, k, metric, vsq, qsq, out_ids, out_d, flags + nq, flags, s);
-    (void)hipFreeAsync(sid, s);
-    (void)hipFreeAsync(sd, s);
-    (void)hipFreeAsync(qcount, s);
-    (void)hipFreeAsync(qcand, s);
-    (void)hipFreeAsync(flags, s);
-  }
+  bf_one_pass(base, n, dp, queries, nq, k, metric, vsq, qsq, out_ids, out_d, nullptr, nullptr, s);
   if (vsq) (void)hipFreeAsync(vsq, s);
   if (qsq) (void)hipFreeAsync(qsq, s);
 }

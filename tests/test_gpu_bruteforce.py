@@ -158,12 +158,16 @@ def test_two_pass_overflow_falls_back(jasper, oracle_lib):
     assert np.array_equal(ids, rid)
 
 
-# rounds path (rows of more than 128 values, 16,384 rows and more): one query
-# block and its edges (128 / 256 queries), a partial last tile of base rows, a
-# partial last slice of a row (dims that are no multiple of 64), k = 1 and the
-# largest; values small enough that every sum is an exact integer.
-@pytest.mark.parametrize("dim,n,nq,k", [(136, 16384, 1, 10), (200, 20001, 129, 128), (256, 66001, 256, 1),
-                                        (520, 17001, 257, 33), (960, 30003, 100, 100)])
+# rounds path: one query block and its edges (128 / 256 queries), a partial last
+# tile of base rows, a partial last slice of a row (dims that are no multiple of
+# 64) and short rows of every kind (one chunk, odd and even chunk counts, 128
+# values), k = 1 and the largest; values small enough that every sum is an
+# exact integer.
+@pytest.mark.parametrize("dim,n,nq,k", [(136, 16384, 1, 17), (200, 20001, 129, 128), (264, 66001, 256, 1),
+                                        (520, 17001, 257, 33), (960, 30003, 100, 100),
+                                        (8, 16384, 70, 17), (24, 65536, 3, 1), (40, 65601, 257, 10),
+                                        (64, 17001, 256, 128), (96, 20063, 1, 32), (113, 30001, 65, 20),
+                                        (128, 70007, 129, 10)])
 @pytest.mark.parametrize("distance", ["l2", "ip"])
 def test_rounds_integer_exact(jasper, oracle_lib, dim, n, nq, k, distance):
     rng = np.random.default_rng(dim + n)
