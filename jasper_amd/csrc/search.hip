@@ -819,6 +819,35 @@ static void launch_one(const SearchArgs& a, dim3 grid, size_t lds, hipStream_t s
   hipLaunchKernelGGL(kern, grid, dim3(TEAM ? 64 * TEAM : 64), lds, stream, a);
 }
 
+// Waves per query for a launch of nq queries; 0: one, without a team. Times of
+// a team against one wave, 50,000 rows, beams of 32 to 512:
+//  - Nodes of 16 edges have no hop for a team (kTeamAlone), and its waves only
+//    take the room of other queries' (2,200 to 4,000 queries of 960 values:
+//    1.3 to 1.7 times as long).
+//  - The 16 rows a wave scores in one pass bound a useful team: two waves at 32
+//    edges (128 values, L2: 0.97 to 1.01; four 1.01 to 1.06; 960 values, one
+//    query: 0.70 to 0.79, four 0.72 to 0.81), four at 64 (128 values 0.76 to
+//    0.88, 960 values 0.41 to 0.58). Inner products of 129 to 256 values gain
+//    from two only (0.85 to 0.93; four 0.89 to 1.20).
+//  - Every query's waves stay resident: 1,024 queries of four waves at four
+//    per SIMD, 2,048 of two; 3,072 where the registers allow six per SIMD (L2
+//    rows of up to 128 values: 0.95 to 1.00 there, 1.24 to 1.6 at 3,500).
+//  - Past that a launch takes a second turn, and two waves pay only where they
+//    gain that much: streamed rows by inner product (2,200 to 4,000 queries:
+//    0.64 to 0.94), and by L2 rows of 768 values or more while the second turn
+//    is at least half full (three quarters at 32 edges: less to gain): 0.77 to
+//    1.03 then, up to 1.4 at 2,200 queries. Streamed L2 rows of 260 to 512
+//    values lose there (260: 1.05 to 1.6).
+static uint32_t team_waves(const Graph& g, uint32_t nq, uint32_t cpl) {
+  if (g.R <= kTeamAlone) return 0;
+  const bool l2 = g.metric == kL2, streamed = cpl > 8;
+  const bool four = g.R > 2 * kTeamAlone && (l2 || cpl <= 4 || streamed);
+  if (nq <= 1024u) return four ? 4u : 2u;
+  if (nq <= (l2 && cpl <= 4 ? 3072u : 2048u)) return 2;
+  if (!streamed || nq > 4096u) return 0;
+  return !l2 || (g.dp >= 768 && nq >= (four ? 3072u : 3584u)) ? 2u : 0u;
+}
+
 void launch_beam_search(const Graph& g, const SearchRequest& r, hipStream_t stream) {
   if (r.nq == 0) return;
   if (r.beam_width == 0) throw std::invalid_argument("beam_width must be positive");
@@ -903,22 +932,11 @@ void launch_beam_search(const Graph& g, const SearchRequest& r, hipStream_t stre
   const uint32_t cpl = (a.nchunks + 3) / 4;
   const dim3 grid(r.nq);
   a.hash_bytes = (uint32_t)std::max<size_t>(((size_t)1 << a.hash_bits) * (seen_tag_bits(g.n, a.hash_bits) ? 2 : 4), 4);
+  // byte rows take one wave (a team 1.00x at bw 64, 0.97x at 200): a hop's rows
+  // are one or two passes of it already
   const bool bytes = a.vecs8 && !stats && g.metric == kL2 && cpl == 4;
   const size_t team_lds = ((lds + 15) & ~(size_t)15) + (cpl > 8 ? (size_t)a.nchunks * 16 : 0) + 64 * 4 + 16;
-  // Teams while every query's waves are resident: 1,024 queries of four waves
-  // at four per SIMD; two waves to 2,048, to 3,072 where the registers allow
-  // six per SIMD (L2 rows of up to 128 values), to 4,096 for streamed rows,
-  // which gain from two waves even in turns. Against one wave per query, bw 64:
-  //   four waves, 1 / 1,000 queries: 128 Gaussian values 1.36x / 1.34x, 200
-  //   values 1.51x / 1.37x, 960 values 2.4x / 1.8x; 96 values by inner product
-  //   1.12x / 1.00x, 384 1.4x / 1.7x; at 2,000 they lose (0.80x on 128 values)
-  //   two waves, 2,000 / 3,000 / 4,000 queries: 128 values 1.06x / 1.05x /
-  //   0.79x, 200 values 1.07x / 0.93x; 960 values 1.14x / 1.10x / 1.15x, 384 by
-  //   inner product 1.66x / 1.29x / 1.33x
-  // Byte rows stay with one wave (1.00x at bw 64, 0.97x at 200): a hop's rows
-  // are one pass of it already.
-  const uint32_t two = cpl > 8 ? 4096u : cpl <= 4 && g.metric == kL2 ? 3072u : 2048u;
-  const uint32_t team = r.nq <= 1024u ? 4u : r.nq <= two ? 2u : 0u;
+  const uint32_t team = team_waves(g, r.nq, cpl);
   if (team && !bytes && !stats && team_lds <= 160 * 1024) {
     a.hash_bytes += (uint32_t)(((lds + 15) & ~(size_t)15) - lds);
 #define JA_TEAM(C)                                                                              \

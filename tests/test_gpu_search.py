@@ -338,3 +338,28 @@ def test_team_matches_one_wave(jasper, distance, dim, R):
             idt, dt = g.search(few.repeat(times, 1), k=10, beam_width=bw)
             assert torch.equal(ids[:40 * times], idt), f"bw={bw}, {40 * times} queries"
             assert torch.equal(d[:40 * times].view(torch.int32), dt.view(torch.int32)), f"bw={bw}, {40 * times} queries"
+
+
+# Extra waves per query must not cost other queries their room: nodes of 16
+# edges leave a second wave nothing to do, and 2,200 queries of two waves do
+# not fit the chip at once. Where the launch rule overlooked that, they took
+# 1.6 times as long as 2,000; as single waves they take about 1.05 times.
+@pytest.mark.parametrize("dim,R", [(264, 16), (264, 32), (960, 16)])
+def test_a_few_more_queries_take_little_longer(jasper, dim, R):
+    rng = np.random.default_rng(dim + R)
+    base = rng.normal(size=(20_000, dim)).astype(np.float16)
+    g = jasper.Graph.build(torch.from_numpy(base).cuda(), n_neighbors=R, distance="l2")
+    q = torch.from_numpy(rng.normal(size=(2200, dim)).astype(np.float16)).cuda()
+
+    def once(nq):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        g.search(q[:nq], k=10, beam_width=128)
+        b.record()
+        torch.cuda.synchronize()
+        return a.elapsed_time(b)
+
+    times = [(once(2000), once(2200)) for _ in range(8)]
+    ratio = min(t[1] for t in times) / min(t[0] for t in times)
+    print(f"2,200 queries against 2,000: {ratio:.2f}")
+    assert ratio <= 1.3
