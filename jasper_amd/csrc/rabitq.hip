@@ -12,11 +12,11 @@
 // P is the sum of three fp16 values (times its row's power of two), so the
 // fp32 product runs as three v_mfma_f32_16x16x32_f16 chains at 16 times the
 // fp32 matrix rate: every product is exact and the sums are fp32. An entry's
-// 24 bits split exactly unless it is under 2^-29 of its row's largest; the
-// rest is then below 2^-39 of that one, under the sums' own rounding. Where a
-// residual lies within the two products' rounding of zero, its tile (16
-// coordinates of 16 vectors) takes the fp32 product instead, so the code bytes
-// are that one's.
+// 24 bits split exactly down to 2^-15 of its row's largest; of a smaller one
+// less than 2^-39 of the largest is lost, under the sums' own rounding. Where a
+// residual lies within the two products' rounding of zero (the bound is
+// counted at rabitq_setup_kernel), its tile (16 coordinates of 16 vectors)
+// takes the fp32 product instead, so the code bytes are that one's.
 // fp32 rows (rabitq_kernel): v_mfma_f32_16x16x4_f32, one wave per 16 vectors:
 // the MFMA's M side is 16 output coordinates, its N side 16 vectors, and the
 // four K slots of each MFMA take coordinates k = 32b + 8q + s (q = lane/16,
@@ -41,16 +41,29 @@ typedef float float4v __attribute__((ext_vector_type(4)));
 
 uint32_t rabitq_code_bytes(uint32_t dim) { return ((dim + 7u) / 8u + 3u) / 4u * 4u; }
 
+// w_s of the bound below.
+__device__ __forceinline__ float rabitq_weight(uint32_t steps, uint32_t s) { return (float)(64u * (steps - s) + 4u); }
+
 // Scratch of one call, written by one launch of rabitq_setup_kernel: the
 // rotated centroid rc[i] = sum_k P[i + k*dim] c[k] (P times c: the centroid
 // goes through CUBLAS_OP_N, rotation.cuh:160-176; zero without a centroid and
 // for i >= dim), and Pt[i][k] = P[k + i*dim], zero padded to [mp][kp]. For
 // fp16 rows (split) also three fp16 parts [3][mp][kp] of Pt[i][k] * 2^s_i;
 // inv[i] = 2^-s_i, where 2^s_i brings row i's largest entry to [2^14, 2^15);
-// and tol[i], which bounds the difference of the two products' sums i for a
-// vector of norm 1: the f32 MFMAs round kp / 4 times, the f16 ones 3 kp / 32
-// times, each by at most 2^-24 of sum |P_ik x_k| <= |P_i| |x|, and 8 more for
-// the sums inside an instruction.
+// and tol[i], which times a vector's xw (rabitq_residuals) bounds the difference
+// of the two products' sums i. An MFMA is taken to add its products one after
+// the other in any order, each sum rounded to nearest. A sum rounded in K step s
+// (32 coordinates) is at most A_s, the sum of |P_ik x_k| over the steps to s; the
+// fp32 chain rounds 32 of them per step, and so does the fp16 chain of the
+// first parts. The two others' sums are 2^-11 of it, so all their roundings
+// count as less than one A, and so does what the split lost; the fp32 chain's
+// rounded products and joining the two fp16 sums are one each:
+//   u (sum_s 64 A_s + 4 A) = u sum_s w_s a_s,  w_s = 64 (steps - s) + 4,
+// a_s = A_s - A_{s-1} <= |P_is| |x_s|, which by Cauchy-Schwarz is at most
+// u sqrt(sum_s w_s |P_is|^2) sqrt(sum_s w_s |x_s|^2) = tol[i] xw, u = 2^-24 (1%
+// on each factor for its own rounding). Rows whose largest entry is outside
+// [2^-60, 2^60] are always taken from the fp32 product: nearer the ends of the
+// exponent range its products underflow or its sums overflow.
 // Block i < mp: row i. Block mp: the centroid.
 __global__ __launch_bounds__(256) void rabitq_setup_kernel(const float* __restrict__ P, const float* __restrict__ c,
                                                            uint32_t dim, uint32_t mp, uint32_t kp, bool split,
@@ -71,10 +84,6 @@ __global__ __launch_bounds__(256) void rabitq_setup_kernel(const float* __restri
   if (!split) return;
   __shared__ uint32_t top[4];
   __shared__ float sq[4];
-  float s2 = v * v;
-#pragma unroll
-  for (int x = 32; x >= 1; x >>= 1) s2 += __shfl_xor(s2, x, 64);
-  if ((t & 63u) == 0) sq[t >> 6] = s2;
   uint32_t m = __builtin_bit_cast(uint32_t, fabsf(v));
 #pragma unroll
   for (int x = 32; x >= 1; x >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, x, 64));
@@ -86,6 +95,10 @@ __global__ __launch_bounds__(256) void rabitq_setup_kernel(const float* __restri
   const int e = (int)(m >> 23) - 127;
   const int sh = m >> 23 == 0 || m >> 23 == 255 ? 0 : 14 - e;
   const float w = __builtin_ldexpf(v, sh);
+  float s2 = t < kp ? rabitq_weight(kp / 32, t / 32) * w * w : 0.0f;  // (w: no underflow at any scale)
+#pragma unroll
+  for (int x = 32; x >= 1; x >>= 1) s2 += __shfl_xor(s2, x, 64);
+  if ((t & 63u) == 0) sq[t >> 6] = s2;
   const _Float16 p1 = (_Float16)w;
   const bool whole = fabsf((float)p1) < __builtin_inff();
   const float r1 = whole ? w - (float)p1 : 0.0f;  // exact
@@ -97,10 +110,12 @@ __global__ __launch_bounds__(256) void rabitq_setup_kernel(const float* __restri
     parts[part + at] = p2;
     parts[2 * part + at] = p3;
   }
+  __syncthreads();
   if (t == 0) {
-    inv[i] = __builtin_ldexpf(1.0f, -sh);
-    const float rounds = (float)(kp / 4 + 3 * kp / 32 + 8) * 0x1p-24f;
-    tol[i] = rounds * sqrtf((sq[0] + sq[1]) + (sq[2] + sq[3])) * 1.01f;
+    const float scale = __builtin_ldexpf(1.0f, -sh);
+    inv[i] = scale;
+    const bool ends = m != 0 && (e < -60 || e > 60);
+    tol[i] = ends ? __builtin_inff() : 0x1p-24f * 1.01f * sqrtf((sq[0] + sq[1]) + (sq[2] + sq[3])) * scale;
   }
 }
 
@@ -217,9 +232,10 @@ struct RqTables {
 
 // One tile of 16 vectors from the split product's sums to its residuals, in
 // place; returns sum r^2 over this lane's coordinates. x2: this lane's part of
-// |x|^2. An output tile with a residual within `tol` of zero is taken again
-// from the fp32 product (about one in 130 at 128 dims). Redoing the vectors'
-// other output tiles with it cost 45 us more on 1M x 128.
+// sum_s w_s |x_s|^2. An output tile with a residual within its bound of zero is
+// taken again from the fp32 product (about one in 50 at 128 dims, one in 17 at
+// 256). Redoing the vectors' other output tiles with it cost more: 45 us of
+// 1M x 128 when one in 130 was taken again.
 template <int KT>
 __device__ __forceinline__ float rabitq_residuals(float4v (&acc)[KT], float x2, const uint16_t* __restrict__ x, int64_t v,
                                                   int64_t n, uint32_t stride, uint32_t dim,
@@ -228,7 +244,7 @@ __device__ __forceinline__ float rabitq_residuals(float4v (&acc)[KT], float x2, 
   constexpr uint32_t kp = 32 * ((KT + 1) / 2);
   x2 += __shfl_xor(x2, 16, 64);
   x2 += __shfl_xor(x2, 32, 64);
-  const float xn = sqrtf(x2) * 1.01f;
+  const float xw = sqrtf(x2) * 1.01f;
   uint32_t q4 = 4 * q;
   asm volatile("" : "+v"(q4));  // opaque: or the tables are held in registers for all tiles
   uint32_t redo = 0;  // output tiles with a residual within its tolerance
@@ -243,7 +259,7 @@ __device__ __forceinline__ float rabitq_residuals(float4v (&acc)[KT], float x2, 
       const bool in = t < KT - 1 || 16u * t + 4u * q + j < dim;
       // (the scaling is exact: one rounding, that of the subtraction)
       const float r = in ? __builtin_fmaf(acc[t][j], iv[j], -cv[j]) : 0.0f;
-      near = near || (in && !(fabsf(r) > tv[j] * xn));  // NaN included
+      near = near || (in && !(fabsf(r) > tv[j] * xw));  // NaN included
       acc[t][j] = r;
     }
     if (ballot(near && v < n)) redo |= 1u << t;
@@ -252,8 +268,8 @@ __device__ __forceinline__ float rabitq_residuals(float4v (&acc)[KT], float x2, 
   if (redo) {
     // the fp32 product of output tile t, the loads of up to HS K steps issued
     // together: they meet cold caches (1 to 2 us a round trip; Pt is another
-    // XCD's write). One step after the other, 10,000 x 256 took 131 us, this way 73;
-    // 1M x 256 1.54 -> 1.36 ms. More steps than that spill beside 64 sums.
+    // XCD's write). One step after the other, 10,000 x 256 took 131 us, this way 78;
+    // 1M x 256 1.54 -> 1.40 ms. More steps than that spill beside 64 sums.
     constexpr uint32_t KS = kp / 32, HS = KS <= 5 ? KS : 4;
     const uint16_t* row = x + (size_t)(v < n ? v : 0) * stride;
     do {
@@ -364,13 +380,13 @@ __global__ __launch_bounds__(256, 2) void rabitq_kernel(const float* __restrict_
 // fp16 rows. A block stages the three parts of Pt in LDS once (rows one chunk
 // past a multiple of 256 bytes, so that the 16 rows of a fragment fall on
 // different banks) and its waves then walk tiles of 16 * NT vectors alone:
-// each fragment of P read from LDS serves NT MFMAs, and the next tile's rows
+// each fragment of P read from LDS serves NT MFMAs (the small parts of P over
+// all of K first, as the bound above counts them), and the next tile's rows
 // load while this tile's factors are summed. LDS bounds NT = 1 (98 KB per 16
 // vectors at 128 dims), so two where the registers hold them (KT <= 8: 128
 // VGPRs of sums and rows).
-// 1M x 128: 668 us (f32 MFMA, f64 divisions, byte stores) -> 268 us; 1M x 96:
-// 410 -> 174 us. Against 64 bits over 512M codes at 128 dims the code bits are
-// off in the same 12 places, f_rescale by 1.04e-7 (1.09e-7 before).
+// 1M x 128: 614 us (f32 MFMA, f64 divisions, byte stores) -> 221 us; 1M x 96:
+// 378 -> 158 us, 1M x 160: 1.02 -> 0.36 ms.
 template <int KT, int NT>
 __global__ __launch_bounds__(512, 2) void rabitq_split_kernel(const uint16_t* __restrict__ x, int64_t n,
                                                               uint32_t stride, uint32_t dim,
@@ -421,25 +437,34 @@ __global__ __launch_bounds__(512, 2) void rabitq_split_kernel(const uint16_t* __
 #pragma unroll
     for (int u = 0; u < NT; ++u) x2[u] = 0.0f;
 #pragma unroll
-    for (uint32_t s = 0; s < KS; ++s) {
-      half8 xh[NT];
+    for (int u = 0; u < NT; ++u)
 #pragma unroll
-      for (int u = 0; u < NT; ++u) {
+      for (uint32_t s = 0; s < KS; ++s) {
         // (stride >= 8-padded dim, so a chunk past dim's own is never read)
-        uint4 w = xf[u][s];
-        if (s == KS - 1 && dim % 8 != 0) w = keep_below(w, 32 * s + 8 * q, dim);
-        __builtin_memcpy(&xh[u], &w, 16);
-        x2[u] = sq_add(xh[u], x2[u]);
+        if (s == KS - 1 && dim % 8 != 0) xf[u][s] = keep_below(xf[u][s], 32 * s + 8 * q, dim);
+        half8 xh;
+        __builtin_memcpy(&xh, &xf[u][s], 16);
+        x2[u] = __builtin_fmaf(rabitq_weight(KS, s), sq_add(xh, 0.0f), x2[u]);
       }
+    // the small parts' sums first, then the first parts' on top of them
 #pragma unroll
-      for (int t = 0; t < KT; ++t) {
+    for (int first = 0; first < 2; ++first) {
 #pragma unroll
-        for (int part = 2; part >= 0; --part) {  // smallest part first
-          const uint4 w = rq_lds[frag + ((uint32_t)part * mp + 16 * t) * kRow + 4 * s];
-          half8 ph;
-          __builtin_memcpy(&ph, &w, 16);
+      for (uint32_t s = 0; s < KS; ++s) {
 #pragma unroll
-          for (int u = 0; u < NT; ++u) acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph, xh[u], acc[u][t], 0, 0, 0);
+        for (int t = 0; t < KT; ++t) {
+#pragma unroll
+          for (int part = first ? 0 : 2; part >= (first ? 0 : 1); --part) {
+            const uint4 w = rq_lds[frag + ((uint32_t)part * mp + 16 * t) * kRow + 4 * s];
+            half8 ph;
+            __builtin_memcpy(&ph, &w, 16);
+#pragma unroll
+            for (int u = 0; u < NT; ++u) {
+              half8 xh;
+              __builtin_memcpy(&xh, &xf[u][s], 16);
+              acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph, xh, acc[u][t], 0, 0, 0);
+            }
+          }
         }
       }
     }
@@ -462,8 +487,9 @@ __global__ __launch_bounds__(512, 2) void rabitq_split_kernel(const uint16_t* __
 // fp16 rows of more than 160 values: the parts of Pt exceed LDS, so a block
 // stages them one K step of 32 at a time (3 * mp * 64 bytes, double-buffered,
 // loaded straight into LDS) and its eight waves take the step together, each
-// for its own 16 vectors (32 would spill: 128 sums per lane at 256 values, and
-// the factors' temporaries). Read through the caches instead, by each wave, 500k x 256 took 1.7 times as long; this way 0.89 ms (1.22 on the f32 MFMA).
+// for its own 16 vectors, the first parts' sums beside the two others' (128 per
+// lane at 256 values). Read through the caches instead, by each wave, 500k x 256
+// took 1.7 times as long. 1M x 256: 2.24 ms on the f32 MFMA, 1.40 this way.
 // Chunk q of row r sits at slot q ^ (r / 2 % 4) (mfma_gemm.hpp).
 template <int KT>
 __global__ __launch_bounds__(512, 2) void rabitq_split_long_kernel(const uint16_t* __restrict__ x, int64_t n,
@@ -472,7 +498,7 @@ __global__ __launch_bounds__(512, 2) void rabitq_split_long_kernel(const uint16_
                                                                    const float* __restrict__ pt,
                                                                    const float* __restrict__ tables, int metric,
                                                                    uint32_t* __restrict__ out) {
-  constexpr uint32_t KS = (KT + 1) / 2, kp = 32 * KS, mp = 16 * KT, NT = 1;
+  constexpr uint32_t KS = (KT + 1) / 2, kp = 32 * KS, mp = 16 * KT;
   constexpr uint32_t kLoads = 3 * KT;  // kilobytes per step
   __shared__ uint4 slice[2][3 * mp * 4];
   __shared__ __align__(16) float tabl[3 * mp];  // rc, inv, tol
@@ -489,10 +515,10 @@ __global__ __launch_bounds__(512, 2) void rabitq_split_long_kernel(const uint16_
       }
     }
   };
-  const int64_t tiles = (n + 16 * NT - 1) / (16 * NT);
+  const int64_t tiles = (n + 15) / 16;
   const int64_t turns = (tiles + (int64_t)gridDim.x * 8 - 1) / ((int64_t)gridDim.x * 8);  // the same for every wave
-  auto row_chunk = [&](int64_t tl, uint32_t u, uint32_t s) {
-    const int64_t v = tl * (16 * NT) + 16 * u + col;
+  auto row_chunk = [&](int64_t tl, uint32_t s) {
+    const int64_t v = tl * 16 + col;
     const uint32_t k = 32 * s + 8 * q;
     uint4 w = make_uint4(0, 0, 0, 0);
     if (v < n && k < dim) w = *reinterpret_cast<const uint4*>(x + (size_t)v * stride + k);
@@ -503,26 +529,20 @@ __global__ __launch_bounds__(512, 2) void rabitq_split_long_kernel(const uint16_
   uint32_t buf = 0;
   for (int64_t turn = 0; turn < turns; ++turn) {
     const int64_t tile = (turn * gridDim.x + blockIdx.x) * 8 + wave;  // past the last: no rows
-    float4v acc[NT][KT];
+    float4v acc[KT], low[KT];  // sums of the first parts, and of the two others
 #pragma unroll
-    for (uint32_t u = 0; u < NT; ++u)
-#pragma unroll
-      for (int t = 0; t < KT; ++t) acc[u][t] = {0.0f, 0.0f, 0.0f, 0.0f};
-    uint4 xn[NT];
+    for (int t = 0; t < KT; ++t) acc[t] = low[t] = {0.0f, 0.0f, 0.0f, 0.0f};
     float x2 = 0.0f;
-#pragma unroll
-    for (uint32_t u = 0; u < NT; ++u) xn[u] = row_chunk(tile, u, 0);
+    uint4 xn = row_chunk(tile, 0);
     for (uint32_t s = 0; s < KS; ++s) {
-      half8 xh[NT];
-#pragma unroll
-      for (uint32_t u = 0; u < NT; ++u) __builtin_memcpy(&xh[u], &xn[u], 16);
-      x2 = sq_add(xh[0], x2);
+      half8 xh;
+      __builtin_memcpy(&xh, &xn, 16);
+      x2 = __builtin_fmaf(rabitq_weight(KS, s), sq_add(xh, 0.0f), x2);
       __builtin_amdgcn_s_waitcnt(0x70);  // vmcnt(0) lgkmcnt(0): this step's slice and rows are here
       __syncthreads();                   // and every wave is done with the other buffer
       if (s + 1 < KS) {
         issue(s + 1, buf ^ 1u);
-#pragma unroll
-        for (uint32_t u = 0; u < NT; ++u) xn[u] = row_chunk(tile, u, s + 1);
+        xn = row_chunk(tile, s + 1);
       } else if (turn + 1 < turns) {
         issue(0, buf ^ 1u);
       }
@@ -532,19 +552,20 @@ __global__ __launch_bounds__(512, 2) void rabitq_split_long_kernel(const uint16_
 #pragma unroll
         for (int part = 2; part >= 0; --part) {  // smallest part first
           const half8 ph = *reinterpret_cast<const half8*>(pl + (part * mp + 16 * t) * 64);
-#pragma unroll
-          for (uint32_t u = 0; u < NT; ++u)
-            acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph, xh[u], acc[u][t], 0, 0, 0);
+          float4v& sum = part ? low[t] : acc[t];
+          sum = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph, xh, sum, 0, 0, 0);
         }
       }
       buf ^= 1u;
     }
     const int64_t v = tile * 16 + col;
-    const float l2 = rabitq_residuals<KT>(acc[0], x2, x, v, n, stride, dim, pt, col, q, tab);
+#pragma unroll
+    for (int t = 0; t < KT; ++t) acc[t] += low[t];
+    const float l2 = rabitq_residuals<KT>(acc, x2, x, v, n, stride, dim, pt, col, q, tab);
     uint32_t q4 = 4 * q;
     asm volatile("" : "+v"(q4));
     rabitq_emit<KT>(
-        acc[0], l2, dim, q, [&](int t) { return *reinterpret_cast<const float4v*>(tab.rc + 16 * t + q4); }, metric,
+        acc, l2, dim, q, [&](int t) { return *reinterpret_cast<const float4v*>(tab.rc + 16 * t + q4); }, metric,
         v < n, out + (size_t)v * (KS + 2));
   }
 }

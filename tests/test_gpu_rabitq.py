@@ -105,6 +105,31 @@ def test_rabitq_columns_of_any_scale(jasper, oracle_lib):
     assert np.array_equal(bits[clear], (r >= 0)[clear].astype(np.uint8))
 
 
+# The code bits of fp16 rows are those of the fp32 product, also where nearly
+# every output is a small rest of large sums (so that the two products' rounding
+# decides its sign unless it is taken again): pairs that cancel, and a first half
+# that the second half cancels; at any scale of the matrix's columns.
+@pytest.mark.parametrize("dim", [24, 128, 160, 176, 256])
+@pytest.mark.parametrize("scale", [1e-36, 1e-25, 1.0, 1e25])
+@pytest.mark.parametrize("halves", [False, True])
+def test_rabitq_cancelling_sums_take_the_fp32_bits(jasper, dim, scale, halves):
+    rng = np.random.default_rng(dim)
+    n, h = 4000, dim // 2
+    pos = np.abs(rng.normal(size=(n, h))) + 0.1 if halves else rng.normal(size=(n, h))
+    col = np.abs(rng.normal(size=(dim, h))) + 0.1 if halves else rng.normal(size=(dim, h))  # row i = column i
+    near = col * (1 + rng.normal(size=(dim, h)) * 2.0**-19)
+    x, p = np.empty((n, dim)), np.empty((dim, dim))
+    at = (slice(0, h), slice(h, dim)) if halves else (slice(0, dim, 2), slice(1, dim, 2))
+    x[:, at[0]], x[:, at[1]] = pos, -pos
+    p[:, at[0]], p[:, at[1]] = col, near
+    rows = torch.from_numpy(x.astype(np.float16)).cuda()
+    matrix = torch.from_numpy((p * scale).astype(np.float32)).cuda()
+    got = jasper.rabitq_quantize(rows, rotation=matrix)
+    ref = jasper.rabitq_quantize(rows.float(), rotation=matrix)
+    assert 0.2 < got.bits().float().mean() < 0.8
+    assert torch.equal(got.codes, ref.codes), f"{(got.bits() != ref.bits()).sum()} of {n * dim} bits"
+
+
 @pytest.mark.parametrize("dim", [200, 256])
 def test_short_calls_on_fp16_rows_take_no_longer_than_on_fp32_rows(jasper, dim):
     """10,000 rows are one turn of the chip, in which a tile that takes the fp32
