@@ -4,8 +4,10 @@
 // Arithmetic as the reference computes it: L2 = (||q||^2 + ||v||^2) - 2 q.v in
 // fp32, clamped at 0; IP = -(q.v) where the fp16 matmul's result is rounded to
 // fp16 before the negation. q.v comes from v_mfma_f32_32x32x16_f16 (fp16
-// products are exact in fp32, accumulation in fp32); the squared norms are
-// fp32 sums in element order. Ties are ordered by (distance, id).
+// products are exact in fp32, accumulation in fp32, K ascending on every path);
+// the squared norms are fp32 sums, in element order for rows of up to 128 values
+// and in the order of bf_long_sqnorm_kernel for longer ones. So a pair's
+// distance is the same bits in every call. Ties are ordered by (distance, id).
 //
 // One-pass path, used for small bases (the line is in bruteforce_knn) and for
 // queries that the rounds path leaves over:
@@ -62,9 +64,7 @@ __device__ __forceinline__ half8 u4_as_h8(uint4 v) {
 // two rows of a wave share a bank when they read the same column.
 constexpr uint32_t kSqnRows = 256, kSqnChunk = 64, kSqnStride = kSqnChunk * 2 + 8;  // bytes
 __global__ __launch_bounds__(kSqnRows) void row_sqnorm_kernel(const uint16_t* __restrict__ x, int64_t n,
-                                                              uint32_t dp, uint32_t dim, float* __restrict__ out,
-                                                              const uint32_t* __restrict__ wanted) {
-  if (wanted && !*wanted) return;  // the norms are for queries left over, and there are none
+                                                              uint32_t dp, uint32_t dim, float* __restrict__ out) {
   __shared__ __align__(16) uint8_t tile[kSqnRows * kSqnStride];  // 34,816 bytes
   const uint32_t t = threadIdx.x;
   const int64_t r0 = (int64_t)blockIdx.x * kSqnRows;
@@ -98,6 +98,40 @@ __global__ __launch_bounds__(kSqnRows) void row_sqnorm_kernel(const uint16_t* __
     __syncthreads();
   }
   if (i < n) out[i] = s;
+}
+
+// ||x||^2 per row of more than 128 values, in the order that bf_tile_kernel sums
+// it from its fragments: chunk c (8 values) to sum c mod 8, sums 2w and 2w + 1
+// joined to part w, and the parts added from 0 to 3. Every path takes long rows'
+// norms in this order, so that a pair's distance does not depend on the call it
+// is computed in. Eight lanes per row, one per sum (128 contiguous bytes).
+__global__ __launch_bounds__(256) void bf_long_sqnorm_kernel(const uint16_t* __restrict__ x, int64_t n, uint32_t dp,
+                                                             float* __restrict__ out,
+                                                             const uint32_t* __restrict__ wanted) {
+  if (wanted && !*wanted) return;  // the norms are for queries left over, and there are none
+  const int64_t row = (int64_t)blockIdx.x * 32 + (threadIdx.x >> 3);
+  const uint32_t lane = threadIdx.x & 63u, j = lane & 7u;
+  float s = 0.0f;
+  if (row < n)
+    for (uint32_t c = j; c < dp / 8; c += 8)
+      s = gemm_sq_add(u4_as_h8(reinterpret_cast<const uint4*>(x + (size_t)row * dp)[c]), s);
+  const float part = s + __shfl_xor(s, 1, 64);
+  float sum = 0.0f;
+#pragma unroll
+  for (uint32_t w = 0; w < 4; ++w) sum += __shfl(part, (int)((lane & ~7u) + 2 * w), 64);
+  if (row < n && j == 0) out[row] = sum;
+}
+
+// ||x||^2 of every row. wanted (long rows): nothing is computed if it is zero.
+static void bf_sqnorms(const void* x, int64_t n, uint32_t dp, uint32_t dim, float* out, const uint32_t* wanted,
+                       hipStream_t s) {
+  if (dp > 128)
+    hipLaunchKernelGGL(bf_long_sqnorm_kernel, dim3((uint32_t)((n + 31) / 32)), dim3(256), 0, s, (const uint16_t*)x, n,
+                       dp, out, wanted);
+  else
+    hipLaunchKernelGGL(row_sqnorm_kernel, dim3((uint32_t)((n + kSqnRows - 1) / kSqnRows)), dim3(kSqnRows), 0, s,
+                       (const uint16_t*)x, n, dp, dim, out);
+  hip_check(hipGetLastError(), "launch row norms");
 }
 
 // Sort key: order-preserving distance bits (high) and id (low).
@@ -355,9 +389,9 @@ __device__ __forceinline__ void lds_block_sync() {
 // work-group p takes item p / 8 of XCD p % 8's share, and the query blocks of one
 // part run on one XCD and share its L2's copy of the tiles. The base rows' squared
 // norms are summed from the fragments the products read (v_dot2, in the
-// shadow of the MFMAs; each of the WAM waves that read the same fragments
-// takes one K step of a slice), so the base is read once, without a pass of
-// its own for the norms. dense: round 0, every distance to its own slot of
+// shadow of the MFMAs, in the order of bf_long_sqnorm_kernel; the WAM waves that
+// read the same fragments share the K steps), so the base is read once, without
+// a pass of its own for the norms. dense: round 0, every distance to its own slot of
 // dist [nq][kBfFirst] (NaN for rows past the base).
 // L2 scores first take a cheap conservative test: y = fl(2 q.v - vs') >= c_q,
 // with vs' = fl(||v||^2 (1 - 2^-20)) and c_q <= (||q||^2 - T_q) - 2^-19
@@ -373,7 +407,7 @@ struct BfTileLds {
   // after the loop's buffers, per query: staged keys, norm, threshold, the
   // cheap test's bound, a count; then the norms' parts. 256 x 256: 161,792
   // of 163,840 bytes
-  static constexpr size_t bytes = G::kLds + (size_t)G::TM * (8 * kLocal + 4 * 4) + (size_t)G::WAM * G::TN * 4;
+  static constexpr size_t bytes = G::kLds + (size_t)G::TM * (8 * kLocal + 4 * 4) + (size_t)4 * G::TN * 4;
 };
 
 template <class G, int METRIC>
@@ -382,7 +416,10 @@ __global__ __launch_bounds__(G::kThreads, 2) void bf_tile_kernel(
     const float* __restrict__ qsq, const float* __restrict__ qthr, uint32_t t0, uint32_t t1, uint32_t n_tiles,
     uint32_t mul, uint32_t n_ch, uint32_t qblocks, float* __restrict__ dense, uint32_t* __restrict__ qcount,
     uint64_t* __restrict__ qcand) {
-  static_assert(G::KC / 2 == G::WAM, "one K step of a slice per wave that shares a column");
+  // K step j's squares go to part j mod 4 of the norm: the waves that share a
+  // column take one step of each slice (four waves) or every other slice (two)
+  static_assert((G::KC == 8 && G::WAM == 4) || (G::KC == 4 && G::WAM == 2), "every K step is some wave's");
+  constexpr int kParts = 4 / G::WAM;  // of a wave
   extern __shared__ uint4 bf_tile_lds[];
   constexpr uint32_t kLocal = BfTileLds<G>::kLocal;
   char* lds = reinterpret_cast<char*>(bf_tile_lds);
@@ -391,7 +428,7 @@ __global__ __launch_bounds__(G::kThreads, 2) void bf_tile_kernel(
   float* sth = sqs + G::TM;                                              // [TM] thresholds
   float* scr = sth + G::TM;                                              // [TM] the cheap test's c_q
   uint32_t* lcnt = reinterpret_cast<uint32_t*>(scr + G::TM);             // [TM]
-  float* part = reinterpret_cast<float*>(lcnt + G::TM);                  // [WAM][TN] parts of the rows' norms
+  float* part = reinterpret_cast<float*>(lcnt + G::TM);                  // [4][TN] parts of the rows' norms
   const uint32_t W = gridDim.x, p = blockIdx.x, xcd = p & 7u, per = W >> 3, extra = W & 7u;
   const uint32_t L = xcd * per + min(xcd, extra) + (p >> 3);
   const uint32_t qblock = L % qblocks, ch = L / qblocks;
@@ -417,9 +454,11 @@ __global__ __launch_bounds__(G::kThreads, 2) void bf_tile_kernel(
   __syncthreads();
   const uint32_t lane = threadIdx.x & 63u, wave = uniform(threadIdx.x >> 6), am = lane & 31u, ah = lane >> 5;
   const uint32_t wm = wave % G::WAM, wn = wave / G::WAM;
-  float vs[G::WTN];  // this lane's part of its columns' squared norms
+  float vs[kParts][G::WTN];  // this lane's parts of its columns' squared norms
 #pragma unroll
-  for (int b = 0; b < G::WTN; ++b) vs[b] = 0.0f;
+  for (int e = 0; e < kParts; ++e)
+#pragma unroll
+    for (int b = 0; b < G::WTN; ++b) vs[e][b] = 0.0f;
   // the tiles being loaded and being tested
   uint32_t next = bf_tile_at(first, mul, n_tiles), here = next;
   gemm_walk<G>(
@@ -430,16 +469,11 @@ __global__ __launch_bounds__(G::kThreads, 2) void bf_tile_kernel(
         next -= next >= n_tiles ? n_tiles : 0u;
         return row;
       },
-      [&](int step, const gemm_half8 (&y)[G::WTN]) {
-        if (METRIC == kL2 && (uint32_t)step == wm) {
-          typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+      [&](uint32_t k, int step, const gemm_half8 (&y)[G::WTN]) {
+        if (METRIC == kL2 && (G::WAM == 4 ? (uint32_t)step : k & 1u) == wm) {
+          float(&part_vs)[G::WTN] = vs[G::WAM == 4 ? 0 : step];
 #pragma unroll
-          for (int b = 0; b < G::WTN; ++b)
-#pragma unroll
-            for (int e = 0; e < 8; e += 2) {
-              const half2v h = {y[b][e], y[b][e + 1]};
-              vs[b] = __builtin_amdgcn_fdot2(h, h, vs[b], false);
-            }
+          for (int b = 0; b < G::WTN; ++b) part_vs[b] = gemm_sq_add(y[b], part_vs[b]);
         }
       },
       [&](uint32_t t, const gemm_acc (&acc)[G::WTM][G::WTN]) {
@@ -452,16 +486,18 @@ __global__ __launch_bounds__(G::kThreads, 2) void bf_tile_kernel(
         if constexpr (METRIC == kL2) {
           // the last tile's readers are past the barriers of this tile's slices
 #pragma unroll
-          for (int b = 0; b < G::WTN; ++b) {
-            vs[b] += __shfl_xor(vs[b], 32, 64);
-            if (ah == 0) part[wm * G::TN + wn * G::WTN * 32 + 32 * b + am] = vs[b];
-            vs[b] = 0.0f;
-          }
+          for (int e = 0; e < kParts; ++e)
+#pragma unroll
+            for (int b = 0; b < G::WTN; ++b) {
+              const float x = vs[e][b] + __shfl_xor(vs[e][b], 32, 64);
+              if (ah == 0) part[(wm * kParts + e) * G::TN + wn * G::WTN * 32 + 32 * b + am] = x;
+              vs[e][b] = 0.0f;
+            }
           lds_block_sync();
 #pragma unroll
           for (int b = 0; b < G::WTN; ++b)
 #pragma unroll
-            for (int w = 0; w < G::WAM; ++w) vn[b] += part[w * G::TN + wn * G::WTN * 32 + 32 * b + am];
+            for (int w = 0; w < 4; ++w) vn[b] += part[w * G::TN + wn * G::WTN * 32 + 32 * b + am];
         }
 #pragma unroll
         for (int a = 0; a < G::WTM; ++a) {
@@ -773,24 +809,6 @@ __global__ __launch_bounds__(256, 2) void bf_stream_kernel(
   }
 }
 
-// ||x||^2 per row, a wave per row (the rounds path's query norms: few rows,
-// so the lanes share a row's sum instead of a row each).
-__global__ __launch_bounds__(256) void bf_query_sqnorm_kernel(const uint16_t* __restrict__ x, int64_t n, uint32_t dp,
-                                                              float* __restrict__ out) {
-  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const uint32_t lane = threadIdx.x & 63u;
-  if (row >= n) return;
-  float s = 0.0f;
-  for (uint32_t c = lane; c < dp / 8; c += 64) {
-    const half8 h = u4_as_h8(reinterpret_cast<const uint4*>(x + (size_t)row * dp)[c]);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) s = __builtin_fmaf((float)h[e], (float)h[e], s);
-  }
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) s += __shfl_xor(s, m, 64);
-  if (lane == 0) out[row] = s;
-}
-
 // After a round, a work-group per query: finds the query's k-th key and keeps
 // the k smallest in the list (in any order), their k-th distance as the
 // threshold. The k-th is found by bits, from the top: a key's word takes a 0
@@ -1075,15 +1093,9 @@ static void bf_in_rounds(const void* base, int64_t n, uint32_t dim, uint32_t dp,
     hip_check(hipMallocAsync((void**)&qsq, (size_t)nq * 4, s), "alloc query norms");
     hip_check(hipMallocAsync((void**)&vsq, (size_t)n * 4, s), "alloc base norms");
   }
-  auto norms = [&](const uint16_t* x, int64_t rows, float* out, const uint32_t* wanted) {
-    hipLaunchKernelGGL(row_sqnorm_kernel, dim3((uint32_t)((rows + 255) / 256)), dim3(256), 0, s, x, rows, dp, dim, out,
-                       wanted);
-  };
+  if (metric == kL2) bf_sqnorms(queries, nq, dp, dim, qsq, nullptr, s);
   if (dp <= 128) {
-    if (metric == kL2) {
-      norms(queries16, nq, qsq, nullptr);
-      norms(base16, n, vsq, nullptr);
-    }
+    if (metric == kL2) bf_sqnorms(base, n, dp, dim, vsq, nullptr, s);
     auto go = [&](auto tag) {
       constexpr int KS = decltype(tag)::value;
       using G = BfStream<KS>;
@@ -1110,9 +1122,6 @@ static void bf_in_rounds(const void* base, int64_t n, uint32_t dim, uint32_t dp,
       default: go(std::integral_constant<int, 8>{}); break;
     }
   } else {
-    if (metric == kL2)
-      hipLaunchKernelGGL(bf_query_sqnorm_kernel, dim3((uint32_t)((nq + 3) / 4)), dim3(256), 0, s, queries16, nq, dp,
-                         qsq);
     auto go = [&](auto tile) {
       using G = decltype(tile);
       constexpr size_t lds = BfTileLds<G>::bytes;
@@ -1131,7 +1140,7 @@ static void bf_in_rounds(const void* base, int64_t n, uint32_t dim, uint32_t dp,
     const uint64_t by256 = (uint64_t)((nq + 255) / 256) * 256 * 850, by128 = (uint64_t)((nq + 127) / 128) * 128 * 991;
     if (by256 <= by128) go(GemmTile<2, 4, 4, 2, 8>{});
     else go(GemmTile<2, 4, 2, 2, 4>{});
-    if (metric == kL2) norms(base16, n, vsq, flagged);  // for the flagged queries, if there are any
+    if (metric == kL2) bf_sqnorms(base, n, dp, dim, vsq, flagged, s);  // for the flagged queries, if there are any
   }
   bf_one_pass(base, n, dp, queries, nq, k, metric, vsq, qsq, out_ids, out_d, flags + nq, flags, s);
   (void)hipFreeAsync(qthr, s);
@@ -1174,10 +1183,8 @@ void bruteforce_knn(const void* base, int64_t n, uint32_t dim, uint32_t dp, cons
   if (metric == kL2) {
     hip_check(hipMallocAsync((void**)&vsq, (size_t)n * 4, s), "alloc base norms");
     hip_check(hipMallocAsync((void**)&qsq, (size_t)nq * 4, s), "alloc query norms");
-    hipLaunchKernelGGL(row_sqnorm_kernel, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, s, (const uint16_t*)base,
-                       n, dp, dim, vsq, nullptr);
-    hipLaunchKernelGGL(row_sqnorm_kernel, dim3((uint32_t)((nq + 255) / 256)), dim3(256), 0, s,
-                       (const uint16_t*)queries, nq, dp, dim, qsq, nullptr);
+    bf_sqnorms(base, n, dp, dim, vsq, nullptr, s);
+    bf_sqnorms(queries, nq, dp, dim, qsq, nullptr, s);
   }
   bf_one_pass(base, n, dp, queries, nq, k, metric, vsq, qsq, out_ids, out_d, nullptr, nullptr, s);
   if (vsq) (void)hipFreeAsync(vsq, s);

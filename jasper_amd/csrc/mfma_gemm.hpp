@@ -57,6 +57,17 @@ __device__ __forceinline__ void gemm_load_lds16(const void* g, void* l) {
   __builtin_amdgcn_global_load_lds((gemm_glb_void*)g, (gemm_lds_void*)l, 16, 0, 0);
 }
 
+// s plus the squares of 8 values (v_dot2: fp16 subnormals are kept)
+__device__ __forceinline__ float gemm_sq_add(gemm_half8 h, float s) {
+  typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+#pragma unroll
+  for (int e = 0; e < 8; e += 2) {
+    const half2v p = {h[e], h[e + 1]};
+    s = __builtin_amdgcn_fdot2(p, p, s, false);
+  }
+  return s;
+}
+
 // How many parts to cut a walk of `tiles` tiles into, for `groups` rows of
 // work-groups each: the count whose last turn of `resident` work-groups is
 // fullest (a part's tiles set its turn's time).
@@ -78,12 +89,13 @@ inline uint32_t gemm_parts(uint32_t groups, uint32_t tiles, uint32_t resident) {
 // Walks tiles 0 .. n_tiles - 1. `a_row0` / `a_last`: the work-group's first
 // row of A and the last valid one (rows past it read that row again);
 // tile_row(t): the first B row of tile t; `b_last` as a_last. a_stride,
-// b_stride: 16-byte chunks from row to row; nck: chunks multiplied. zero: 16 bytes of zeros in global
-// memory, read for chunks past the row in the last slice (both operands, so
-// that no value is multiplied by a stray one). slice(s, y): called with the B
-// fragments of each K step s of a slice; epi(t, acc): called with a tile's sums, lane l holding
-// column l % 32 of B tile b and rows 8*(i/4) + 4*(l/32) + i%4 of A tile a in
-// acc[a][b][i]. epi may use LDS outside [lds, lds + G::kLds).
+// b_stride: 16-byte chunks from row to row; nck: chunks multiplied. zero: 16
+// bytes of zeros in global memory, read for chunks past the row in the last
+// slice (both operands, so that no value is multiplied by a stray one).
+// slice(k, s, y): called with the B fragments of each K step s of slice k;
+// epi(t, acc): called with a tile's sums, lane l holding column l % 32 of B tile
+// b and rows 8*(i/4) + 4*(l/32) + i%4 of A tile a in acc[a][b][i]. epi may use
+// LDS outside [lds, lds + G::kLds).
 template <class G, class TileRow, class Slice, class Epi>
 __device__ __forceinline__ void gemm_walk(char* lds, const void* A, uint32_t a_stride, int64_t a_row0, int64_t a_last,
                                           const void* B, uint32_t b_stride, int64_t b_last, uint32_t nck,
@@ -138,7 +150,7 @@ __device__ __forceinline__ void gemm_walk(char* lds, const void* A, uint32_t a_s
   };
   const uint32_t am = lane & 31u, ah = lane >> 5, fs = G::swizzle(am);
   gemm_acc acc[G::WTM][G::WTN];
-  auto compute = [&](uint32_t buf) {
+  auto compute = [&](uint32_t k, uint32_t buf) {
     const char* la = lds + buf * G::kBuf + (wm * G::WTM * 32 + am) * G::kRowBytes;
     const char* lb = lds + buf * G::kBuf + (G::TM + wn * G::WTN * 32 + am) * G::kRowBytes;
     gemm_half8 x[2][G::WTM], y[2][G::WTN];
@@ -159,7 +171,7 @@ __device__ __forceinline__ void gemm_walk(char* lds, const void* A, uint32_t a_s
 #pragma unroll
         for (int b = 0; b < G::WTN; ++b)
           acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[s & 1][a], y[s & 1][b], acc[a][b], 0, 0, 0);
-      slice(s, y[s & 1]);
+      slice(k, s, y[s & 1]);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
@@ -182,7 +194,7 @@ __device__ __forceinline__ void gemm_walk(char* lds, const void* A, uint32_t a_s
         set_tile(t + 1);
         issue(0, buf ^ 1u);
       }
-      compute(buf);
+      compute(k, buf);
       buf ^= 1u;
     }
     epi(t, acc);

@@ -316,17 +316,6 @@ __device__ __forceinline__ float rabitq_residuals(float4v (&acc)[KT], float x2, 
   return l2;
 }
 
-// |x|^2 over 8 values
-__device__ __forceinline__ float sq_add(half8 h, float s) {
-  typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-#pragma unroll
-  for (int e = 0; e < 8; e += 2) {
-    const half2v p = {h[e], h[e + 1]};
-    s = __builtin_amdgcn_fdot2(p, p, s, false);
-  }
-  return s;
-}
-
 // KT = number of 16-wide output tiles (mp = 16 * KT <= 256).
 template <int KT>
 __global__ __launch_bounds__(256, 2) void rabitq_kernel(const float* __restrict__ x, int64_t n, uint32_t stride,
@@ -444,7 +433,7 @@ __global__ __launch_bounds__(512, 2) void rabitq_split_kernel(const uint16_t* __
         if (s == KS - 1 && dim % 8 != 0) xf[u][s] = keep_below(xf[u][s], 32 * s + 8 * q, dim);
         half8 xh;
         __builtin_memcpy(&xh, &xf[u][s], 16);
-        x2[u] = __builtin_fmaf(rabitq_weight(KS, s), sq_add(xh, 0.0f), x2[u]);
+        x2[u] = __builtin_fmaf(rabitq_weight(KS, s), gemm_sq_add(xh, 0.0f), x2[u]);
       }
     // the small parts' sums first, then the first parts' on top of them
 #pragma unroll
@@ -537,7 +526,7 @@ __global__ __launch_bounds__(512, 2) void rabitq_split_long_kernel(const uint16_
     for (uint32_t s = 0; s < KS; ++s) {
       half8 xh;
       __builtin_memcpy(&xh, &xn, 16);
-      x2 = __builtin_fmaf(rabitq_weight(KS, s), sq_add(xh, 0.0f), x2);
+      x2 = __builtin_fmaf(rabitq_weight(KS, s), gemm_sq_add(xh, 0.0f), x2);
       __builtin_amdgcn_s_waitcnt(0x70);  // vmcnt(0) lgkmcnt(0): this step's slice and rows are here
       __syncthreads();                   // and every wave is done with the other buffer
       if (s + 1 < KS) {

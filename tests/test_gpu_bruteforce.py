@@ -196,3 +196,28 @@ def test_rounds_overflow_and_not_finite_rows(jasper, oracle_lib):
     ids, d = _run(jasper, base, q, 10, "l2")
     assert np.array_equal(d, rd)
     assert np.array_equal(ids, keep[rid])
+
+
+# A pair's distance is the same bits whatever call it is computed in: with fewer
+# or more queries (128- and 256-query tiles), over fewer rows (the one-pass
+# kernels), and for a query that the rounds leave over (a k-th distance that is
+# not finite). Real-valued rows, whose norms depend on the order of their sum.
+@pytest.mark.parametrize("dim", [64, 136, 200, 264, 384, 960])
+def test_a_pairs_distance_does_not_depend_on_the_call(jasper, dim):
+    base = torch.from_numpy(gaussian(20_000, dim, 60).astype(np.float16)).cuda()
+    q = torch.from_numpy(gaussian(300, dim, 61).astype(np.float16)).cuda()
+    q[:100] = base[:100] + q[:100] * 0.25
+    ids, d = jasper.bruteforce_knn(base, q, 20, "l2")
+    seen = [dict(zip(i, x)) for i, x in zip(ids.tolist(), d.view(torch.int32).tolist())]
+    few = base.clone()
+    few[100:, 3] = float("inf")  # 100 rows left: fewer than k, so no 20th finite distance within the first rows
+    shared = 0
+    for rows, count, k in ((base, 100, 20), (base, 200, 20), (base, 1, 20), (base, 300, 10), (base[:3000], 300, 20),
+                           (few, 100, 20)):
+        i, x = jasper.bruteforce_knn(rows, q[:count], k, "l2")
+        for at, (a, b) in enumerate(zip(i.tolist(), x.view(torch.int32).tolist())):
+            for name, bits in zip(a, b):
+                if name in seen[at]:
+                    shared += 1
+                    assert seen[at][name] == bits, (rows.shape[0], count, k, at, name)
+    assert shared > 100 * 20 + 200 * 20 + 300 * 10
