@@ -31,7 +31,6 @@
 #include <algorithm>
 #include <cfloat>
 #include <cstdlib>
-#include <numeric>
 #include <stdexcept>
 #include <type_traits>
 
@@ -362,17 +361,62 @@ constexpr uint32_t kBfCandCap = 1024;  // keys a query's list holds between roun
 constexpr float kBfVsShrink = 1.0f - 0x1p-20f;
 
 // ------------------------------------------------------------ rounds path
-// The base is scored in rounds over its tiles, in an order that spreads every
-// round over the whole base (tile i of the order is tile i * mul mod n_tiles,
-// mul coprime to n_tiles: rows stored cluster by cluster meet every round
-// alike). Round 0 (kBfFirst rows) writes every distance; after each round a
-// trim kernel keeps a query's best k keys and its k-th distance T_q, and the
-// next round, 4 or 16 times as many rows, appends only keys with d <= T_q:
-// about k * (ratio - 1) of them. Every row is scored once.
+// The base is scored in rounds over units of UNIT rows, in an order that spreads
+// every round over the whole base: place i of the order is unit
+// i * mul mod n_units, mul coprime to n_units. Round 0 (kBfFirst rows) writes
+// every distance; after each round a trim kernel keeps a query's best k keys
+// and its k-th distance T_q, and the next round, 4 or 16 times as many rows,
+// appends only keys with d <= T_q: about k * (ratio - 1) of them.
+// Rows stored cluster by cluster: until k rows of a query's cluster have been
+// met, T_q is another cluster's and units of its own enter the list whole, up
+// to more keys than it holds. The rounds then go on with the k best that it
+// holds (T_q still bounds the true k-th distance, and later rounds tighten it),
+// and such queries are scored once more over the whole base against their last
+// T_q, which lists little more than k rows. Only work-groups that hold such a
+// query run then; the others return at once. k = 100, rows in clusters: 1,000
+// queries of 1M x 960 in clusters of 1,000 rows 50.6 -> 5.6 ms (in one pass ->
+// once more; 3.7 ms shuffled), 10k of 1M x 128, 4,000 rows, 85 -> 6.6 ms (6.2).
 constexpr uint32_t kBfFirst = 4096;  // rows of round 0
 
-__device__ __forceinline__ uint32_t bf_tile_at(uint32_t i, uint32_t mul, uint32_t n_tiles) {
-  return (uint32_t)(((uint64_t)i * mul) % n_tiles);
+struct BfOrder {
+  uint32_t mul, n_units;
+  __device__ __forceinline__ uint32_t at(uint32_t place) const { return (uint32_t)(((uint64_t)place * mul) % n_units); }
+  // the unit `by` (< n_units) further in the base, cyclically; by = places * mul mod n_units
+  __device__ __forceinline__ uint32_t on(uint32_t unit, uint32_t by) const {
+    unit += by;
+    return unit >= n_units ? unit - n_units : unit;
+  }
+  __device__ __forceinline__ uint32_t step(uint32_t places) const {  // places * mul mod n_units, few places
+    uint32_t x = 0;
+    for (uint32_t i = 0; i < places; ++i) x = on(x, mul);
+    return x;
+  }
+};
+
+// The order's mul: near the golden ratio of the units, the coprime number whose
+// ratio to them has the smallest largest partial quotient (any run of places
+// then falls evenly over the base, and any run of units over the places).
+static uint32_t bf_order_step(uint32_t n_units) {
+  const uint32_t golden = (uint32_t)(0.6180339887 * n_units);
+  uint32_t best = 1, worst = ~0u;
+  for (uint32_t i = 0; i < 128 && worst > 3; ++i) {
+    const uint32_t mul = i & 1u ? golden - (i + 1) / 2 : golden + i / 2;
+    uint32_t a = n_units, b = mul, largest = 0;
+    while (b != 0) {
+      uint32_t quotient = a / b;
+      const uint32_t rest = a % b;
+      if (rest == 0 && b != 1) quotient = ~0u;  // not coprime
+      if (rest == 0 && b == 1) --quotient;      // (.., q) is (.., q - 1, 1)
+      largest = std::max(largest, quotient);
+      a = b;
+      b = rest;
+    }
+    if (largest < worst) {
+      worst = largest;
+      best = mul;
+    }
+  }
+  return best;
 }
 
 // Work-group barrier for LDS alone: loads in flight (the next tile's) go on.
@@ -382,8 +426,12 @@ __device__ __forceinline__ void lds_block_sync() {
   asm volatile("" ::: "memory");
 }
 
-// One round over the order's tiles [t0, t1) with the product loop of
-// mfma_gemm.hpp: G::TM queries per work-group, tiles of G::TN base rows, n_ch
+// Rows of more than 128 values: units of a matrix tile's columns. With units of
+// whole tiles (256 rows) nearly every query of a base in clusters loses keys.
+constexpr uint32_t kBfTileUnit = 32;
+
+// One round over the order's tiles [t0, t1) (of G::TN / 32 places) with the
+// product loop of mfma_gemm.hpp: G::TM queries per work-group, n_ch
 // work-groups per query block taking contiguous parts of the round. The work
 // order is XCD-aware: work-groups are dealt to the 8 XCDs round-robin by id, so
 // work-group p takes item p / 8 of XCD p % 8's share, and the query blocks of one
@@ -392,7 +440,8 @@ __device__ __forceinline__ void lds_block_sync() {
 // shadow of the MFMAs, in the order of bf_long_sqnorm_kernel; the WAM waves that
 // read the same fragments share the K steps), so the base is read once, without
 // a pass of its own for the norms. dense: round 0, every distance to its own slot of
-// dist [nq][kBfFirst] (NaN for rows past the base).
+// dist [nq][kBfFirst] (NaN for rows past the base). lost: the queries whose
+// threshold is a number are scored again (none, most often).
 // L2 scores first take a cheap conservative test: y = fl(2 q.v - vs') >= c_q,
 // with vs' = fl(||v||^2 (1 - 2^-20)) and c_q <= (||q||^2 - T_q) - 2^-19
 // (||q||^2 + |T_q|). Whenever the exact score d = fl(fl(||q||^2 + ||v||^2) -
@@ -413,9 +462,10 @@ struct BfTileLds {
 template <class G, int METRIC>
 __global__ __launch_bounds__(G::kThreads, 2) void bf_tile_kernel(
     const uint16_t* __restrict__ base, int64_t n, uint32_t dp, const uint16_t* __restrict__ queries, int64_t nq,
-    const float* __restrict__ qsq, const float* __restrict__ qthr, uint32_t t0, uint32_t t1, uint32_t n_tiles,
-    uint32_t mul, uint32_t n_ch, uint32_t qblocks, float* __restrict__ dense, uint32_t* __restrict__ qcount,
-    uint64_t* __restrict__ qcand) {
+    const float* __restrict__ qsq, const float* __restrict__ qthr, uint32_t t0, uint32_t t1, BfOrder order,
+    uint32_t n_ch, uint32_t qblocks, float* __restrict__ dense, uint32_t* __restrict__ qcount,
+    uint64_t* __restrict__ qcand, const uint32_t* __restrict__ lost) {
+  if (lost && !*lost) return;
   // K step j's squares go to part j mod 4 of the norm: the waves that share a
   // column take one step of each slice (four waves) or every other slice (two)
   static_assert((G::KC == 8 && G::WAM == 4) || (G::KC == 4 && G::WAM == 2), "every K step is some wave's");
@@ -436,6 +486,7 @@ __global__ __launch_bounds__(G::kThreads, 2) void bf_tile_kernel(
   const uint32_t total = t1 - t0, each = total / n_ch, more = total % n_ch;
   const uint32_t first = t0 + ch * each + min(ch, more), count = each + (ch < more ? 1u : 0u);
   const int64_t qbase = (int64_t)qblock * G::TM;
+  bool wanted = false;
   for (uint32_t r = threadIdx.x; r < (uint32_t)G::TM; r += G::kThreads) {
     const int64_t q = qbase + r;
     // a NaN threshold passes nothing (rows past the last query)
@@ -443,6 +494,7 @@ __global__ __launch_bounds__(G::kThreads, 2) void bf_tile_kernel(
     const float th = q >= nq ? __builtin_nanf("") : dense ? __builtin_inff() : qthr[q];
     sqs[r] = qn;
     sth[r] = th;
+    wanted = wanted || th == th;
     // IP: fp16(q.v) >= -T_q needs q.v >= -T_q less half an fp16 step; a whole
     // step (or the subnormal step) here.
     const double t = (double)th;
@@ -451,7 +503,7 @@ __global__ __launch_bounds__(G::kThreads, 2) void bf_tile_kernel(
     scr[r] = (float)(c - fabs(c) * 0x1p-22);
     lcnt[r] = 0u;
   }
-  __syncthreads();
+  if (!__syncthreads_or(wanted)) return;
   const uint32_t lane = threadIdx.x & 63u, wave = uniform(threadIdx.x >> 6), am = lane & 31u, ah = lane >> 5;
   const uint32_t wm = wave % G::WAM, wn = wave / G::WAM;
   float vs[kParts][G::WTN];  // this lane's parts of its columns' squared norms
@@ -459,14 +511,23 @@ __global__ __launch_bounds__(G::kThreads, 2) void bf_tile_kernel(
   for (int e = 0; e < kParts; ++e)
 #pragma unroll
     for (int b = 0; b < G::WTN; ++b) vs[e][b] = 0.0f;
-  // the tiles being loaded and being tested
-  uint32_t next = bf_tile_at(first, mul, n_tiles), here = next;
+  // the units being loaded (load j of this wave lies in one) and, by column
+  // blocks, being tested
+  constexpr uint32_t kUnits = G::TN / kBfTileUnit;
+  const uint32_t tile_step = order.step(kUnits);
+  const uint32_t unit0 = order.at(first * kUnits);
+  uint32_t next[G::kLoadsB], here = order.on(unit0, order.step(wn * G::WTN));
+#pragma unroll
+  for (int j = 0; j < G::kLoadsB; ++j) next[j] = order.on(unit0, order.step(G::load_row(j, wave) / kBfTileUnit));
+  // a place's rows; past the base for places beyond the last
+  auto unit_row = [&](uint32_t unit, uint32_t place) {
+    return (int64_t)(place < order.n_units ? unit : order.n_units) * kBfTileUnit;
+  };
   gemm_walk<G>(
       lds, queries, dp / 8, qbase, nq - 1, base, dp / 8, n - 1, dp / 8, &kBfZeroChunk, count,
-      [&](uint32_t) {
-        const int64_t row = (int64_t)next * G::TN;
-        next += mul;
-        next -= next >= n_tiles ? n_tiles : 0u;
+      [&](uint32_t t, int j, uint32_t r) {
+        const int64_t row = unit_row(next[j], (first + t) * kUnits + r / kBfTileUnit) + r % kBfTileUnit;
+        next[j] = order.on(next[j], tile_step);
         return row;
       },
       [&](uint32_t k, int step, const gemm_half8 (&y)[G::WTN]) {
@@ -477,9 +538,15 @@ __global__ __launch_bounds__(G::kThreads, 2) void bf_tile_kernel(
         }
       },
       [&](uint32_t t, const gemm_acc (&acc)[G::WTM][G::WTN]) {
-        const int64_t v0 = (int64_t)here * G::TN + wn * G::WTN * 32 + am;
-        here += mul;
-        here -= here >= n_tiles ? n_tiles : 0u;
+        uint32_t unit = here;
+        const uint32_t place = (first + t) * kUnits + wn * G::WTN;
+        int64_t v0[G::WTN];
+#pragma unroll
+        for (int b = 0; b < G::WTN; ++b) {
+          v0[b] = unit_row(unit, place + b);
+          unit = order.on(unit, order.mul);
+        }
+        here = order.on(here, tile_step);
         float vn[G::WTN];
 #pragma unroll
         for (int b = 0; b < G::WTN; ++b) vn[b] = 0.0f;
@@ -521,7 +588,7 @@ __global__ __launch_bounds__(G::kThreads, 2) void bf_tile_kernel(
               any |= ballot(y >= cq[i]);
             }
             if (any == 0 && !dense) continue;
-            const int64_t v = v0 + 32 * b;
+            const int64_t v = v0[b] + am;
             uint32_t re = r0;
             asm volatile("" : "+v"(re));
 #pragma unroll
@@ -599,8 +666,9 @@ template <class G, int KS, int METRIC>
 __global__ __launch_bounds__(256, 2) void bf_stream_kernel(
     const uint16_t* __restrict__ base, int64_t n, uint32_t dp, const uint16_t* __restrict__ queries, int64_t nq,
     const float* __restrict__ qsq, const float* __restrict__ vsq, const float* __restrict__ qthr, uint32_t t0,
-    uint32_t t1, uint32_t n_tiles, uint32_t mul, uint32_t n_ch, uint32_t qblocks, float* __restrict__ dense,
-    uint32_t* __restrict__ qcount, uint64_t* __restrict__ qcand) {
+    uint32_t t1, BfOrder order, uint32_t n_ch, uint32_t qblocks, float* __restrict__ dense,
+    uint32_t* __restrict__ qcount, uint64_t* __restrict__ qcand, const uint32_t* __restrict__ lost) {
+  if (lost && !*lost) return;
   extern __shared__ uint4 bf_stream_lds[];
   constexpr uint32_t kLocal = G::kLocal;
   const uint32_t nck = dp / 8, tile_bytes = G::TN * nck * 16;
@@ -617,6 +685,7 @@ __global__ __launch_bounds__(256, 2) void bf_stream_kernel(
   const uint32_t total = t1 - t0, each = total / n_ch, more = total % n_ch;
   const uint32_t first = t0 + ch * each + min(ch, more), count = each + (ch < more ? 1u : 0u);
   const int64_t qbase = (int64_t)qblock * G::TM;
+  bool wanted = false;
   for (uint32_t r = threadIdx.x; r < (uint32_t)G::TM; r += G::kThreads) {
     const int64_t q = qbase + r;
     // a NaN threshold passes nothing (rows past the last query)
@@ -624,6 +693,7 @@ __global__ __launch_bounds__(256, 2) void bf_stream_kernel(
     const float th = q >= nq ? __builtin_nanf("") : dense ? __builtin_inff() : qthr[q];
     sqs[r] = qn;
     sth[r] = th;
+    wanted = wanted || th == th;
     const double t = (double)th;
     if (METRIC == kL2) {
       const double c = ((double)qn - t) - ((double)qn + fabs(t)) * 0x1p-13;
@@ -634,6 +704,7 @@ __global__ __launch_bounds__(256, 2) void bf_stream_kernel(
     }
     lcnt[r] = 0u;
   }
+  if (lost && !__syncthreads_or(wanted)) return;
   const uint32_t lane = threadIdx.x & 63u, wave = uniform(threadIdx.x >> 6), am = lane & 31u, ah = lane >> 5;
   // a row's chunk c sits at slot (c + f(r)) mod nck, which spreads eight
   // consecutive rows' equal chunks over the banks: row starts repeat every
@@ -692,15 +763,11 @@ __global__ __launch_bounds__(256, 2) void bf_stream_kernel(
   for (int t = 0; t < 2; ++t)
 #pragma unroll
     for (int i = 0; i < 16; ++i) start[t][i] = scr[64 * wave + 32 * t + 8 * (i >> 2) + 4 * ah + (i & 3)];
-  uint32_t next = bf_tile_at(first, mul, n_tiles), here = next;
-  auto advance = [&](uint32_t x) {
-    x += mul;
-    return x >= n_tiles ? x - n_tiles : x;
-  };
+  uint32_t next = order.at(first), here = next;
   uint32_t nb = 0, cb = 0;
   for (uint32_t k = 0; k < 2 && k < count; ++k) {
     issue(next, nb);
-    next = advance(next);
+    next = order.on(next, order.mul);
     nb = nb == 2 ? 0 : nb + 1;
   }
   for (uint32_t it = 0; it < count; ++it) {
@@ -714,7 +781,7 @@ __global__ __launch_bounds__(256, 2) void bf_stream_kernel(
     asm volatile("" ::: "memory");
     if (it + 2 < count) {
       issue(next, nb);
-      next = advance(next);
+      next = order.on(next, order.mul);
       nb = nb == 2 ? 0 : nb + 1;
     }
     float16v acc[2][2];
@@ -794,7 +861,7 @@ __global__ __launch_bounds__(256, 2) void bf_stream_kernel(
         }
       }
     }
-    here = advance(here);
+    here = order.on(here, order.mul);
     cb = cb == 2 ? 0 : cb + 1;
   }
   if (dense) return;
@@ -818,39 +885,50 @@ __global__ __launch_bounds__(256, 2) void bf_stream_kernel(
 // only the last round sorts, and only k keys. Four waves for round 0's 4,096
 // keys: with 64 per lane the unrolled code ran once per wave from a cold
 // instruction cache (272 us for 10k queries).
-// A list that overflowed, or with fewer than k keys of finite distance
-// (infinite or NaN rows), flags its query for the one-pass kernels, and a NaN
-// threshold keeps later rounds from appending to it.
-// TN > 0: the keys are round 0's distances and the ids those of the order's
-// first tiles of TN rows.
+// A list that overflowed marks its query as having lost keys; the last round
+// leaves such a query its threshold and an empty list, and after it is scored
+// again, STAGE kBfAgain takes its results. One that overflows even then (ties),
+// or with fewer than k keys of finite distance (infinite or NaN rows), is
+// flagged for the one-pass kernels, and a NaN threshold keeps later rounds from
+// appending to it.
+// STAGE kBfDense: the keys are round 0's distances and the ids those of the
+// order's first places, of UNIT rows.
+enum BfStage { kBfDense, kBfRound, kBfLast, kBfAgain };
+enum BfQuery : uint8_t { kBfDone, kBfLeftOver, kBfLost };  // kBfDone: or in work
 constexpr int kBfTrimRows = kBfCandCap / 64;  // keys per lane
 
-template <int TN>
-__global__ __launch_bounds__(TN > 0 ? 256 : 64) void bf_trim_kernel(
-    const float* __restrict__ dense, uint32_t mul, uint32_t n_tiles, uint32_t* __restrict__ qcount,
-    uint64_t* __restrict__ qcand, uint32_t k, bool last, uint32_t* __restrict__ any_flag, float* __restrict__ qthr,
+template <BfStage STAGE, uint32_t UNIT>
+__global__ __launch_bounds__(STAGE == kBfDense ? 256 : 64) void bf_trim_kernel(
+    const float* __restrict__ dense, BfOrder order, uint32_t* __restrict__ qcount, uint64_t* __restrict__ qcand,
+    uint32_t k, uint32_t* __restrict__ any_flag, uint32_t* __restrict__ any_lost, float* __restrict__ qthr,
     int32_t* __restrict__ out_ids, float* __restrict__ out_d, uint8_t* __restrict__ q_flags,
     uint8_t* __restrict__ tile_flags) {
-  constexpr bool DENSE = TN > 0;
+  constexpr bool DENSE = STAGE == kBfDense;
   constexpr int kWaves = DENSE ? 4 : 1;
   static_assert(!DENSE || kBfFirst == 64 * kBfTrimRows * kWaves, "round 0 fills the registers");
+  static_assert(UNIT == 32 || UNIT == 64, "a lane's slots are 64 apart");
+  if (STAGE == kBfAgain && !*any_lost) return;
   __shared__ uint64_t best[128];
   __shared__ uint32_t red[2][4];
   __shared__ uint32_t taken;
   const int64_t q = blockIdx.x;
   const uint32_t lane = threadIdx.x & 63u, wave = uniform(threadIdx.x >> 6);
-  if (!DENSE && q_flags[q]) return;
+  const uint8_t state = DENSE ? (uint8_t)kBfDone : q_flags[q];
+  if (state == kBfLeftOver || (STAGE == kBfAgain && state != kBfLost)) return;
   const uint32_t cnt = DENSE ? kBfFirst : uniform(qcount[q]);
   uint64_t* list = qcand + (size_t)q * kBfCandCap;
   uint32_t hi[kBfTrimRows], lo[kBfTrimRows];  // empty slots and NaN: all ones
   const uint32_t rows = DENSE ? (uint32_t)kBfTrimRows : min((cnt + 63u) / 64u, (uint32_t)kBfTrimRows);
+  // DENSE: slots 64 (wave kBfTrimRows + j) + lane, UNIT to a place
+  uint32_t unit = DENSE ? order.at(wave * (uint32_t)kBfTrimRows * (64u / UNIT)) : 0u;
+  const uint32_t step = DENSE ? order.step(64u / UNIT) : 0u;
 #pragma unroll
   for (int j = 0; j < kBfTrimRows; ++j) {
     hi[j] = lo[j] = ~0u;
     if constexpr (DENSE) {
-      const uint32_t slot = (wave * kBfTrimRows + (uint32_t)j) * 64u;  // of lane 0
-      const float d = dense[(size_t)q * kBfFirst + slot + lane];
-      lo[j] = bf_tile_at(slot / (uint32_t)TN, mul, n_tiles) * (uint32_t)TN + slot % (uint32_t)TN + lane;
+      const float d = dense[(size_t)q * kBfFirst + (wave * kBfTrimRows + (uint32_t)j) * 64u + lane];
+      lo[j] = (lane < UNIT ? unit : order.on(unit, order.mul)) * UNIT + lane % UNIT;
+      unit = order.on(unit, step);
       if (d == d) hi[j] = dist_to_ord(d);
     } else if ((uint32_t)j < rows && (uint32_t)j * 64u + lane < cnt) {
       const uint64_t key = list[(uint32_t)j * 64u + lane];
@@ -915,14 +993,27 @@ __global__ __launch_bounds__(TN > 0 ? 256 : 64) void bf_trim_kernel(
     }
   }
   const float t = ord_to_dist(v);
-  if (cnt > 64u * kBfTrimRows * kWaves || v == ~0u || !(fabsf(t) < __builtin_inff())) {
+  const bool over = cnt > 64u * kBfTrimRows * kWaves;
+  if ((over && STAGE == kBfAgain) || v == ~0u || !(fabsf(t) < __builtin_inff())) {
     if (threadIdx.x == 0) {
-      q_flags[q] = 1;
+      q_flags[q] = kBfLeftOver;
       tile_flags[q >> 5] = 1;
       *any_flag = 1;
       qthr[q] = __builtin_nanf("");
     }
     return;
+  }
+  if (over && threadIdx.x == 0) {
+    q_flags[q] = kBfLost;
+    *any_lost = 1;
+  }
+  if (STAGE == kBfLast) {
+    const bool again = over || state == kBfLost;
+    if (threadIdx.x == 0) {
+      qthr[q] = again ? t : __builtin_nanf("");
+      qcount[q] = 0;
+    }
+    if (again) return;
   }
   // ties at it: the smallest k - below ids
   uint32_t w = ~0u;
@@ -943,17 +1034,18 @@ __global__ __launch_bounds__(TN > 0 ? 256 : 64) void bf_trim_kernel(
     if (hi[j] < v || (hi[j] == v && lo[j] <= w)) {
       const uint64_t key = ((uint64_t)hi[j] << 32) | lo[j];
       const uint32_t at = atomicAdd(&taken, 1u);  // exactly k in all
-      if (last) best[at] = key;
+      if (STAGE == kBfLast || STAGE == kBfAgain) best[at] = key;
       else list[at] = key;
     }
   }
-  if (DENSE || !last) {  // (round 0 is never the last)
+  if (STAGE == kBfDense || STAGE == kBfRound) {  // (round 0 is never the last)
     if (threadIdx.x == 0) {
       qcount[q] = k;
       qthr[q] = t;
     }
     return;
   }
+  if (STAGE == kBfAgain && threadIdx.x == 0) q_flags[q] = kBfDone;
   const uint32_t N = max(pow2_ceil(k), 2u);
   for (uint32_t i = k + lane; i < N; i += 64u) best[i] = ~0ull;
   wave_sync();
@@ -964,10 +1056,10 @@ __global__ __launch_bounds__(TN > 0 ? 256 : 64) void bf_trim_kernel(
   }
 }
 
-__global__ void bf_clear_kernel(uint8_t* __restrict__ flags, int64_t n, uint32_t* __restrict__ word) {
+__global__ void bf_clear_kernel(uint8_t* __restrict__ flags, int64_t n, uint32_t* __restrict__ words) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) flags[i] = 0;
-  if (i == 0) *word = 0;
+  if (i < 2) words[i] = 0;
 }
 
 // The one-pass path (scan + merge) over base rows [0, n), for all queries or
@@ -1030,40 +1122,47 @@ static void bf_one_pass(const void* base, int64_t n, uint32_t dp, const void* qu
 
 // Scores the whole base in rounds and writes the results; flags (cleared by
 // the caller) name the queries that are left to the one-pass kernels. G: the
-// tiles; round(parts, t0, t1, mul, dist): launches one round.
-template <class G, class Round>
+// tiles, of units of UNIT rows; round(parts, qblocks, t0, t1, order, dist, lost): launches one round.
+template <class G, uint32_t UNIT, class Round>
 static void bf_rounds(int64_t n, int64_t nq, uint32_t k, float* dense, uint32_t* qcount, uint64_t* qcand, float* qthr,
                       uint8_t* q_flags, uint8_t* tile_flags, int32_t* out_ids, float* out_d, hipStream_t s,
                       Round round) {
   const uint32_t n_tiles = (uint32_t)((n + G::TN - 1) / G::TN);
   const uint32_t qblocks = (uint32_t)((nq + G::TM - 1) / G::TM);
-  uint32_t mul = std::max<uint32_t>(1u, (uint32_t)(0.6180339887 * n_tiles));
-  while (std::gcd(mul, n_tiles) != 1u) ++mul;
+  const uint32_t n_units = (uint32_t)((n + UNIT - 1) / UNIT);
+  const BfOrder order{bf_order_step(n_units), n_units};
+  uint32_t* any_flag = qcount + nq;
+  uint32_t* any_lost = any_flag + 1;
   // work-groups the chip holds at once: eight waves per CU (two per SIMD)
   constexpr uint32_t kResident = 256u * (8 / G::kWaves);
   constexpr uint32_t kFirstTiles = kBfFirst / G::TN;
   static_assert(kFirstTiles * G::TN == kBfFirst, "round 0 is whole tiles");
-  uint32_t t0 = 0, t1 = kFirstTiles;  // n >= 4 kBfFirst
-  while (true) {
-    round(gemm_parts(qblocks, t1 - t0, kResident), qblocks, t0, t1, n_tiles, mul, t0 == 0 ? dense : nullptr);
+  auto score = [&](uint32_t t0, uint32_t t1, float* dist, const uint32_t* lost) {
+    round(gemm_parts(qblocks, t1 - t0, kResident), qblocks, t0, t1, order, dist, lost);
     hip_check(hipGetLastError(), "launch a brute-force round");
-    const bool last = t1 == n_tiles;
-    auto trim = [&](auto kern, uint32_t threads) {
-      hipLaunchKernelGGL(kern, dim3((uint32_t)nq), dim3(threads), 0, s, (const float*)dense, mul, n_tiles, qcount,
-                         qcand, k, last, qcount + nq, qthr, out_ids, out_d, q_flags, tile_flags);
-      hip_check(hipGetLastError(), "launch bf_trim_kernel");
-    };
-    if (t0 == 0) trim(bf_trim_kernel<G::TN>, 256);
-    else trim(bf_trim_kernel<0>, 64);
-    if (last) break;
+  };
+  auto trim = [&](auto kern, uint32_t threads) {
+    hipLaunchKernelGGL(kern, dim3((uint32_t)nq), dim3(threads), 0, s, (const float*)dense, order, qcount, qcand, k,
+                       any_flag, any_lost, qthr, out_ids, out_d, q_flags, tile_flags);
+    hip_check(hipGetLastError(), "launch bf_trim_kernel");
+  };
+  uint32_t t0 = 0, t1 = kFirstTiles;  // n >= 4 kBfFirst
+  score(t0, t1, dense, nullptr);
+  trim(bf_trim_kernel<kBfDense, UNIT>, 256);
+  while (t1 < n_tiles) {
     // fourfold: about 3 k candidates per query and round, few where most rows
     // are. With few queries, where a round is mostly its launches, one step of
     // 16 (a list holds 16 k keys with room at k <= 32); with 10k queries it
     // cost 0.25 ms more in exact scores than the round it saves
-    t0 = t1;
     const uint64_t grow = k <= 32 && nq <= 1024 && (uint64_t)t1 * 64 <= n_tiles ? 16 : 4;
+    t0 = t1;
     t1 = (uint32_t)std::min<uint64_t>(n_tiles, (uint64_t)t1 * grow);
+    score(t0, t1, nullptr, nullptr);
+    if (t1 < n_tiles) trim(bf_trim_kernel<kBfRound, UNIT>, 64);
+    else trim(bf_trim_kernel<kBfLast, UNIT>, 64);
   }
+  score(0, n_tiles, nullptr, any_lost);
+  trim(bf_trim_kernel<kBfAgain, UNIT>, 64);
 }
 
 // The rounds path: scratch, the rounds, and the one-pass kernels for the
@@ -1075,13 +1174,13 @@ static void bf_in_rounds(const void* base, int64_t n, uint32_t dim, uint32_t dp,
   float* vsq = nullptr;
   float* qthr = nullptr;
   float* dense = nullptr;     // [nq][kBfFirst] round 0's distances
-  uint32_t* qcount = nullptr;  // [nq] counts, then one word: is any query flagged
+  uint32_t* qcount = nullptr;  // [nq] counts, then two words: is any query flagged, has any lost keys
   uint64_t* qcand = nullptr;
   uint8_t* flags = nullptr;  // [nq] query flags, then [ceil(nq / 32)] tile flags
   const int64_t ntiles = (nq + 31) / 32;
   hip_check(hipMallocAsync((void**)&qthr, (size_t)nq * 4, s), "alloc thresholds");
   hip_check(hipMallocAsync((void**)&dense, (size_t)nq * kBfFirst * 4, s), "alloc first distances");
-  hip_check(hipMallocAsync((void**)&qcount, (size_t)(nq + 1) * 4, s), "alloc candidate counts");
+  hip_check(hipMallocAsync((void**)&qcount, (size_t)(nq + 2) * 4, s), "alloc candidate counts");
   hip_check(hipMallocAsync((void**)&qcand, (size_t)nq * kBfCandCap * 8, s), "alloc candidate lists");
   hip_check(hipMallocAsync((void**)&flags, (size_t)(nq + ntiles), s), "alloc overflow flags");
   hipLaunchKernelGGL(bf_clear_kernel, dim3((uint32_t)((nq + ntiles + 255) / 256)), dim3(256), 0, s, flags,
@@ -1103,12 +1202,12 @@ static void bf_in_rounds(const void* base, int64_t n, uint32_t dim, uint32_t dp,
       auto kern = metric == kL2 ? bf_stream_kernel<G, KS, kL2> : bf_stream_kernel<G, KS, kIP>;
       if (lds > 64 * 1024)
         hip_check(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), "LDS");
-      bf_rounds<G>(n, nq, k, dense, qcount, qcand, qthr, flags, flags + nq, out_ids, out_d, s,
-                   [&](uint32_t parts, uint32_t qblocks, uint32_t t0, uint32_t t1, uint32_t n_tiles, uint32_t mul,
-                       float* dist) {
+      bf_rounds<G, G::TN>(n, nq, k, dense, qcount, qcand, qthr, flags, flags + nq, out_ids, out_d, s,
+                   [&](uint32_t parts, uint32_t qblocks, uint32_t t0, uint32_t t1, BfOrder order, float* dist,
+                       const uint32_t* lost) {
                      hipLaunchKernelGGL(kern, dim3(qblocks * parts), dim3(G::kThreads), lds, s, base16, n, dp,
                                         queries16, nq, (const float*)qsq, (const float*)vsq, (const float*)qthr, t0,
-                                        t1, n_tiles, mul, parts, qblocks, dist, qcount, qcand);
+                                        t1, order, parts, qblocks, dist, qcount, qcand, lost);
                    });
     };
     switch ((dp + 15) / 16) {
@@ -1127,12 +1226,12 @@ static void bf_in_rounds(const void* base, int64_t n, uint32_t dim, uint32_t dp,
       constexpr size_t lds = BfTileLds<G>::bytes;
       auto kern = metric == kL2 ? bf_tile_kernel<G, kL2> : bf_tile_kernel<G, kIP>;
       hip_check(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), "LDS");
-      bf_rounds<G>(n, nq, k, dense, qcount, qcand, qthr, flags, flags + nq, out_ids, out_d, s,
-                   [&](uint32_t parts, uint32_t qblocks, uint32_t t0, uint32_t t1, uint32_t n_tiles, uint32_t mul,
-                       float* dist) {
+      bf_rounds<G, kBfTileUnit>(n, nq, k, dense, qcount, qcand, qthr, flags, flags + nq, out_ids, out_d, s,
+                   [&](uint32_t parts, uint32_t qblocks, uint32_t t0, uint32_t t1, BfOrder order, float* dist,
+                       const uint32_t* lost) {
                      hipLaunchKernelGGL(kern, dim3(qblocks * parts), dim3(G::kThreads), lds, s, base16, n, dp,
-                                        queries16, nq, (const float*)qsq, (const float*)qthr, t0, t1, n_tiles, mul,
-                                        parts, qblocks, dist, qcount, qcand);
+                                        queries16, nq, (const float*)qsq, (const float*)qthr, t0, t1, order, parts,
+                                        qblocks, dist, qcount, qcand, lost);
                    });
     };
     // 256 queries per work-group at 991 TFLOP/s or 128 at 850 (mfma_gemm.hpp),

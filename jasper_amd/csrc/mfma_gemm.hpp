@@ -47,6 +47,12 @@ struct GemmTile {
   static_assert(KC == 4 || KC == 8, "swizzles exist for slices of 4 and 8 chunks");
   static_assert(kLoadsA * 1024 * kWaves == TM * kRowBytes && kLoadsB * 1024 * kWaves == TN * kRowBytes,
                 "every wave loads whole kilobytes of each operand");
+  // load j of a wave fills kilobyte j * waves + wave of an operand's slice:
+  // kRowsPerLoad rows from load_row on, lane l row l / KC, slot l % KC
+  static constexpr uint32_t kRowsPerLoad = 64 / KC;
+  static __device__ __forceinline__ uint32_t load_row(int j, uint32_t wave) {
+    return ((uint32_t)j * kWaves + wave) * kRowsPerLoad;
+  }
   static __device__ __forceinline__ uint32_t swizzle(uint32_t r) { return KC == 8 ? (r & 7u) : ((r >> 1) & 3u); }
 };
 
@@ -88,7 +94,8 @@ inline uint32_t gemm_parts(uint32_t groups, uint32_t tiles, uint32_t resident) {
 
 // Walks tiles 0 .. n_tiles - 1. `a_row0` / `a_last`: the work-group's first
 // row of A and the last valid one (rows past it read that row again);
-// tile_row(t): the first B row of tile t; `b_last` as a_last. a_stride,
+// tile_row(t, j, r): the B row at row r of tile t, r the first of load j of this
+// wave (whose rows follow each other); `b_last` as a_last. a_stride,
 // b_stride: 16-byte chunks from row to row; nck: chunks multiplied. zero: 16
 // bytes of zeros in global memory, read for chunks past the row in the last
 // slice (both operands, so that no value is multiplied by a stray one).
@@ -104,25 +111,21 @@ __device__ __forceinline__ void gemm_walk(char* lds, const void* A, uint32_t a_s
   const uint32_t lane = threadIdx.x & 63u, wave = uniform(threadIdx.x >> 6);
   const uint32_t wm = wave % G::WAM, wn = wave / G::WAM;
   const uint32_t ns = (nck + G::KC - 1) / G::KC, rem = nck - (ns - 1) * G::KC;  // chunks in the last slice
-  // load j of a wave fills kilobyte j * waves + wave of an operand's slice:
-  // 64 / KC rows, lane l row l / KC, slot l % KC
-  constexpr uint32_t kRowsPerLoad = 64 / G::KC;
   const uint32_t lr = lane / G::KC, slot = lane % G::KC;
   const char* pa[G::kLoadsA];
   const char* pb[G::kLoadsB];
   auto chunk_of = [&](uint32_t r) { return slot ^ G::swizzle(r); };
 #pragma unroll
   for (int j = 0; j < G::kLoadsA; ++j) {
-    const uint32_t r = ((uint32_t)j * G::kWaves + wave) * kRowsPerLoad + lr;
+    const uint32_t r = G::load_row(j, wave) + lr;
     const int64_t row = min(a_row0 + (int64_t)r, a_last);
     pa[j] = (const char*)A + (size_t)row * a_stride * 16 + chunk_of(r) * 16;
   }
   auto set_tile = [&](uint32_t t) {
-    const int64_t row0 = tile_row(t);
 #pragma unroll
     for (int j = 0; j < G::kLoadsB; ++j) {
-      const uint32_t r = ((uint32_t)j * G::kWaves + wave) * kRowsPerLoad + lr;
-      const int64_t row = min(row0 + (int64_t)r, b_last);
+      const uint32_t r = G::load_row(j, wave) + lr;
+      const int64_t row = min(tile_row(t, j, G::load_row(j, wave)) + (int64_t)lr, b_last);
       pb[j] = (const char*)B + (size_t)row * b_stride * 16 + chunk_of(r) * 16;
     }
   };
@@ -138,12 +141,12 @@ __device__ __forceinline__ void gemm_walk(char* lds, const void* A, uint32_t a_s
     } else {
 #pragma unroll
       for (int j = 0; j < G::kLoadsA; ++j) {
-        const uint32_t r = ((uint32_t)j * G::kWaves + wave) * kRowsPerLoad + lr;
+        const uint32_t r = G::load_row(j, wave) + lr;
         gemm_load_lds16(chunk_of(r) < rem ? (const void*)(pa[j] + ko) : zero, la + j * G::kWaves * 1024);
       }
 #pragma unroll
       for (int j = 0; j < G::kLoadsB; ++j) {
-        const uint32_t r = ((uint32_t)j * G::kWaves + wave) * kRowsPerLoad + lr;
+        const uint32_t r = G::load_row(j, wave) + lr;
         gemm_load_lds16(chunk_of(r) < rem ? (const void*)(pb[j] + ko) : zero, lb + j * G::kWaves * 1024);
       }
     }

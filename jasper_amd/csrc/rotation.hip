@@ -231,7 +231,7 @@ __global__ __launch_bounds__(G::kThreads, 2) void rotate_gemm_kernel(const uint1
   char* turn = lds + G::kLds + wave * 4096;
   gemm_walk<G>(
       lds, pt, kp / 8, i_base, mp - 1, x, dp_in / 8, n - 1, (dim + 7u) / 8u, &kRotZeroChunk, count,
-      [&](uint32_t t) { return (int64_t)(first + t) * G::TN; }, [](uint32_t, int, const gemm_half8 (&)[G::WTN]) {},
+      [&](uint32_t t, int, uint32_t r) { return (int64_t)(first + t) * G::TN + r; }, [](uint32_t, int, const gemm_half8 (&)[G::WTN]) {},
       [&](uint32_t t, const gemm_acc (&acc)[G::WTM][G::WTN]) {
         const int64_t r0 = (int64_t)(first + t) * G::TN + wn * G::WTN * 32;
         const uint32_t c = lane & 7u, i0 = i_base + wm * 64 + 8 * c;  // the chunk of outputs this lane writes
