@@ -377,6 +377,12 @@ constexpr float kBfVsShrink = 1.0f - 0x1p-20f;
 // queries of 1M x 960 in clusters of 1,000 rows 50.6 -> 5.6 ms (in one pass ->
 // once more; 3.7 ms shuffled), 10k of 1M x 128, 4,000 rows, 85 -> 6.6 ms (6.2).
 constexpr uint32_t kBfFirst = 4096;  // rows of round 0
+// A query's slots in the scratch: round 0's distances, then, once its trim has
+// read them, the list in the first half.
+constexpr uint32_t kBfListStride = kBfFirst / 2;
+constexpr int64_t kBfBlock = 16384;  // queries scored together
+static_assert(kBfListStride >= kBfCandCap, "the list fits in the distances' place");
+static_assert(kBfBlock * kBfListStride < (1ll << 32), "list slots have 32-bit numbers");
 
 struct BfOrder {
   uint32_t mul, n_units;
@@ -392,6 +398,28 @@ struct BfOrder {
     return x;
   }
 };
+
+enum BfQuery : uint8_t { kBfDone, kBfLeftOver, kBfLost };  // kBfDone: or in work
+
+// What the kernels know of the queries' states, in one piece of the scratch.
+struct BfState {
+  uint32_t* any;  // [2] is any query left over, has any lost keys
+  uint8_t* tile;  // [ceil(nq / 32)] holds a query left over
+  uint8_t* q;     // [nq] BfQuery
+  __host__ __device__ BfState(uint32_t* a, int64_t nq)
+      : any(a), tile(reinterpret_cast<uint8_t*>(a + 2)), q(tile + (nq + 31) / 32) {}
+};
+
+// A round's start: round 0 clears what its trim does not write; with nothing to
+// score again, the work-group returns.
+__device__ __forceinline__ bool bf_begin(uint32_t* any, int64_t nq, bool first, bool again) {
+  if (first && blockIdx.x == 0) {
+    const BfState state(any, nq);
+    for (uint32_t i = threadIdx.x; i < (uint32_t)((nq + 31) / 32); i += blockDim.x) state.tile[i] = 0;
+    if (threadIdx.x < 2) any[threadIdx.x] = 0;
+  }
+  return !again || any[1] != 0;
+}
 
 // The order's mul: near the golden ratio of the units, the coprime number whose
 // ratio to them has the smallest largest partial quotient (any run of places
@@ -440,7 +468,7 @@ constexpr uint32_t kBfTileUnit = 32;
 // shadow of the MFMAs, in the order of bf_long_sqnorm_kernel; the WAM waves that
 // read the same fragments share the K steps), so the base is read once, without
 // a pass of its own for the norms. dense: round 0, every distance to its own slot of
-// dist [nq][kBfFirst] (NaN for rows past the base). lost: the queries whose
+// dist [nq][kBfFirst] (NaN for rows past the base). again: the queries whose
 // threshold is a number are scored again (none, most often).
 // L2 scores first take a cheap conservative test: y = fl(2 q.v - vs') >= c_q,
 // with vs' = fl(||v||^2 (1 - 2^-20)) and c_q <= (||q||^2 - T_q) - 2^-19
@@ -464,8 +492,8 @@ __global__ __launch_bounds__(G::kThreads, 2) void bf_tile_kernel(
     const uint16_t* __restrict__ base, int64_t n, uint32_t dp, const uint16_t* __restrict__ queries, int64_t nq,
     const float* __restrict__ qsq, const float* __restrict__ qthr, uint32_t t0, uint32_t t1, BfOrder order,
     uint32_t n_ch, uint32_t qblocks, float* __restrict__ dense, uint32_t* __restrict__ qcount,
-    uint64_t* __restrict__ qcand, const uint32_t* __restrict__ lost) {
-  if (lost && !*lost) return;
+    uint64_t* __restrict__ qcand, uint32_t* __restrict__ any, bool again) {
+  if (!bf_begin(any, nq, dense != nullptr, again)) return;
   // K step j's squares go to part j mod 4 of the norm: the waves that share a
   // column take one step of each slice (four waves) or every other slice (two)
   static_assert((G::KC == 8 && G::WAM == 4) || (G::KC == 4 && G::WAM == 2), "every K step is some wave's");
@@ -612,9 +640,9 @@ __global__ __launch_bounds__(G::kThreads, 2) void bf_tile_kernel(
                 if (s < kLocal) lbuf[(size_t)r * kLocal + s] = key;
                 else {
                   // (inline: a call would save every accumulator around it)
-                  const size_t q = (size_t)qbase + r;
+                  const uint32_t q = (uint32_t)qbase + r;
                   const uint32_t at = atomicAdd(&qcount[q], 1u);
-                  if (at < kBfCandCap) qcand[q * kBfCandCap + at] = key;
+                  if (at < kBfCandCap) qcand[q * kBfListStride + at] = key;
                 }
               }
             }
@@ -629,7 +657,7 @@ __global__ __launch_bounds__(G::kThreads, 2) void bf_tile_kernel(
     if (qbase + r >= nq || c == 0) continue;
     const uint32_t at = atomicAdd(&qcount[qbase + r], c);
     for (uint32_t i = 0; i < c && at + i < kBfCandCap; ++i)
-      qcand[(size_t)(qbase + r) * kBfCandCap + at + i] = lbuf[(size_t)r * kLocal + i];
+      qcand[(size_t)(qbase + r) * kBfListStride + at + i] = lbuf[(size_t)r * kLocal + i];
   }
 }
 
@@ -667,8 +695,8 @@ __global__ __launch_bounds__(256, 2) void bf_stream_kernel(
     const uint16_t* __restrict__ base, int64_t n, uint32_t dp, const uint16_t* __restrict__ queries, int64_t nq,
     const float* __restrict__ qsq, const float* __restrict__ vsq, const float* __restrict__ qthr, uint32_t t0,
     uint32_t t1, BfOrder order, uint32_t n_ch, uint32_t qblocks, float* __restrict__ dense,
-    uint32_t* __restrict__ qcount, uint64_t* __restrict__ qcand, const uint32_t* __restrict__ lost) {
-  if (lost && !*lost) return;
+    uint32_t* __restrict__ qcount, uint64_t* __restrict__ qcand, uint32_t* __restrict__ any, bool again) {
+  if (!bf_begin(any, nq, dense != nullptr, again)) return;
   extern __shared__ uint4 bf_stream_lds[];
   constexpr uint32_t kLocal = G::kLocal;
   const uint32_t nck = dp / 8, tile_bytes = G::TN * nck * 16;
@@ -704,7 +732,7 @@ __global__ __launch_bounds__(256, 2) void bf_stream_kernel(
     }
     lcnt[r] = 0u;
   }
-  if (lost && !__syncthreads_or(wanted)) return;
+  if (!__syncthreads_or(wanted)) return;
   const uint32_t lane = threadIdx.x & 63u, wave = uniform(threadIdx.x >> 6), am = lane & 31u, ah = lane >> 5;
   // a row's chunk c sits at slot (c + f(r)) mod nck, which spreads eight
   // consecutive rows' equal chunks over the banks: row starts repeat every
@@ -853,9 +881,9 @@ __global__ __launch_bounds__(256, 2) void bf_stream_kernel(
             const uint32_t s = atomicAdd(&lcnt[r], 1u);
             if (s < kLocal) lbuf[(size_t)r * kLocal + s] = key;
             else {
-              const size_t q = (size_t)qbase + r;
+              const uint32_t q = (uint32_t)qbase + r;
               const uint32_t at = atomicAdd(&qcount[q], 1u);
-              if (at < kBfCandCap) qcand[q * kBfCandCap + at] = key;
+              if (at < kBfCandCap) qcand[q * kBfListStride + at] = key;
             }
           }
         }
@@ -872,7 +900,7 @@ __global__ __launch_bounds__(256, 2) void bf_stream_kernel(
     if (qbase + r >= nq || c == 0) continue;
     const uint32_t at = atomicAdd(&qcount[qbase + r], c);
     for (uint32_t i = 0; i < c && at + i < kBfCandCap; ++i)
-      qcand[(size_t)(qbase + r) * kBfCandCap + at + i] = lbuf[(size_t)r * kLocal + i];
+      qcand[(size_t)(qbase + r) * kBfListStride + at + i] = lbuf[(size_t)r * kLocal + i];
   }
 }
 
@@ -894,29 +922,27 @@ __global__ __launch_bounds__(256, 2) void bf_stream_kernel(
 // STAGE kBfDense: the keys are round 0's distances and the ids those of the
 // order's first places, of UNIT rows.
 enum BfStage { kBfDense, kBfRound, kBfLast, kBfAgain };
-enum BfQuery : uint8_t { kBfDone, kBfLeftOver, kBfLost };  // kBfDone: or in work
 constexpr int kBfTrimRows = kBfCandCap / 64;  // keys per lane
 
 template <BfStage STAGE, uint32_t UNIT>
 __global__ __launch_bounds__(STAGE == kBfDense ? 256 : 64) void bf_trim_kernel(
-    const float* __restrict__ dense, BfOrder order, uint32_t* __restrict__ qcount, uint64_t* __restrict__ qcand,
-    uint32_t k, uint32_t* __restrict__ any_flag, uint32_t* __restrict__ any_lost, float* __restrict__ qthr,
-    int32_t* __restrict__ out_ids, float* __restrict__ out_d, uint8_t* __restrict__ q_flags,
-    uint8_t* __restrict__ tile_flags) {
+    uint64_t* qcand, BfOrder order, uint32_t* __restrict__ qcount, uint32_t k, BfState state,
+    float* __restrict__ qthr, int32_t* __restrict__ out_ids, float* __restrict__ out_d) {
   constexpr bool DENSE = STAGE == kBfDense;
   constexpr int kWaves = DENSE ? 4 : 1;
   static_assert(!DENSE || kBfFirst == 64 * kBfTrimRows * kWaves, "round 0 fills the registers");
   static_assert(UNIT == 32 || UNIT == 64, "a lane's slots are 64 apart");
-  if (STAGE == kBfAgain && !*any_lost) return;
+  if (STAGE == kBfAgain && !state.any[1]) return;
   __shared__ uint64_t best[128];
   __shared__ uint32_t red[2][4];
   __shared__ uint32_t taken;
   const int64_t q = blockIdx.x;
   const uint32_t lane = threadIdx.x & 63u, wave = uniform(threadIdx.x >> 6);
-  const uint8_t state = DENSE ? (uint8_t)kBfDone : q_flags[q];
-  if (state == kBfLeftOver || (STAGE == kBfAgain && state != kBfLost)) return;
+  const uint8_t was = DENSE ? (uint8_t)kBfDone : state.q[q];
+  if (was == kBfLeftOver || (STAGE == kBfAgain && was != kBfLost)) return;
   const uint32_t cnt = DENSE ? kBfFirst : uniform(qcount[q]);
-  uint64_t* list = qcand + (size_t)q * kBfCandCap;
+  uint64_t* list = qcand + (size_t)q * kBfListStride;
+  const float* dense = reinterpret_cast<const float*>(list);  // (read whole before the list is written)
   uint32_t hi[kBfTrimRows], lo[kBfTrimRows];  // empty slots and NaN: all ones
   const uint32_t rows = DENSE ? (uint32_t)kBfTrimRows : min((cnt + 63u) / 64u, (uint32_t)kBfTrimRows);
   // DENSE: slots 64 (wave kBfTrimRows + j) + lane, UNIT to a place
@@ -926,7 +952,7 @@ __global__ __launch_bounds__(STAGE == kBfDense ? 256 : 64) void bf_trim_kernel(
   for (int j = 0; j < kBfTrimRows; ++j) {
     hi[j] = lo[j] = ~0u;
     if constexpr (DENSE) {
-      const float d = dense[(size_t)q * kBfFirst + (wave * kBfTrimRows + (uint32_t)j) * 64u + lane];
+      const float d = dense[(wave * kBfTrimRows + (uint32_t)j) * 64u + lane];
       lo[j] = (lane < UNIT ? unit : order.on(unit, order.mul)) * UNIT + lane % UNIT;
       unit = order.on(unit, step);
       if (d == d) hi[j] = dist_to_ord(d);
@@ -996,19 +1022,20 @@ __global__ __launch_bounds__(STAGE == kBfDense ? 256 : 64) void bf_trim_kernel(
   const bool over = cnt > 64u * kBfTrimRows * kWaves;
   if ((over && STAGE == kBfAgain) || v == ~0u || !(fabsf(t) < __builtin_inff())) {
     if (threadIdx.x == 0) {
-      q_flags[q] = kBfLeftOver;
-      tile_flags[q >> 5] = 1;
-      *any_flag = 1;
+      state.q[q] = kBfLeftOver;
+      state.tile[q >> 5] = 1;
+      state.any[0] = 1;
       qthr[q] = __builtin_nanf("");
     }
     return;
   }
+  if (DENSE && threadIdx.x == 0) state.q[q] = kBfDone;
   if (over && threadIdx.x == 0) {
-    q_flags[q] = kBfLost;
-    *any_lost = 1;
+    state.q[q] = kBfLost;
+    state.any[1] = 1;
   }
   if (STAGE == kBfLast) {
-    const bool again = over || state == kBfLost;
+    const bool again = over || was == kBfLost;
     if (threadIdx.x == 0) {
       qthr[q] = again ? t : __builtin_nanf("");
       qcount[q] = 0;
@@ -1045,7 +1072,7 @@ __global__ __launch_bounds__(STAGE == kBfDense ? 256 : 64) void bf_trim_kernel(
     }
     return;
   }
-  if (STAGE == kBfAgain && threadIdx.x == 0) q_flags[q] = kBfDone;
+  if (STAGE == kBfAgain && threadIdx.x == 0) state.q[q] = kBfDone;
   const uint32_t N = max(pow2_ceil(k), 2u);
   for (uint32_t i = k + lane; i < N; i += 64u) best[i] = ~0ull;
   wave_sync();
@@ -1056,36 +1083,39 @@ __global__ __launch_bounds__(STAGE == kBfDense ? 256 : 64) void bf_trim_kernel(
   }
 }
 
-__global__ void bf_clear_kernel(uint8_t* __restrict__ flags, int64_t n, uint32_t* __restrict__ words) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) flags[i] = 0;
-  if (i < 2) words[i] = 0;
-}
+// How the one-pass path cuts the base.
+struct BfChunks {
+  int64_t chunk;      // rows
+  uint32_t n_chunks;
+  size_t list_bytes;  // of the chunks' results
+
+  BfChunks(int64_t n, int64_t nq, uint32_t k) {
+    // chunks: each a multiple of 64 vectors (a whole number of 32-vector steps)
+    // about 2,048 work-groups (single waves): longer chunks spend fewer of
+    // their steps filling and compacting the buffers before the threshold
+    // settles (65,536 x 128 rows, 10k queries: 8,192 work-groups took 0.80 ms
+    // longer, 4,096 0.18, 1,024 0.33);
+    // JASPER_BF_SCAN_WGS overrides it (tuning)
+    static const int64_t target = [] {
+      const char* e = std::getenv("JASPER_BF_SCAN_WGS");
+      return e ? std::max<int64_t>(1, std::atoll(e)) : 2048;
+    }();
+    int64_t want = std::max<int64_t>(1, target / ((nq + 31) / 32));
+    want = std::min<int64_t>(want, (n + 63) / 64);
+    chunk = ((n + want - 1) / want + 63) / 64 * 64;
+    n_chunks = (uint32_t)((n + chunk - 1) / chunk);
+    list_bytes = (size_t)nq * n_chunks * k * 8;
+  }
+};
 
 // The one-pass path (scan + merge) over base rows [0, n), for all queries or
-// only the flagged ones.
+// only the flagged ones. lists: BfChunks::list_bytes of scratch.
 static void bf_one_pass(const void* base, int64_t n, uint32_t dp, const void* queries, int64_t nq, uint32_t k,
-                        int metric, const float* vsq, const float* qsq, int32_t* out_ids, float* out_d,
-                        const uint8_t* tile_flags, const uint8_t* q_flags, hipStream_t s) {
+                        int metric, const float* vsq, const float* qsq, uint64_t* lists, int32_t* out_ids,
+                        float* out_d, const uint8_t* tile_flags, const uint8_t* q_flags, hipStream_t s) {
   const uint32_t ks = (dp + 15) / 16;  // 16-wide K steps (the last may be half empty)
-  // chunks: each a multiple of 64 vectors (a whole number of 32-vector steps)
-  // about 2,048 work-groups (single waves): longer chunks spend fewer of
-  // their steps filling and compacting the buffers before the threshold
-  // settles (65,536 x 128 rows, 10k queries: 8,192 work-groups took 0.80 ms
-  // longer, 4,096 0.18, 1,024 0.33);
-  // JASPER_BF_SCAN_WGS overrides it (tuning)
-  const int64_t qtiles = (nq + 31) / 32;
-  static const int64_t target = [] {
-    const char* e = std::getenv("JASPER_BF_SCAN_WGS");
-    return e ? std::max<int64_t>(1, std::atoll(e)) : 2048;
-  }();
-  int64_t want = std::max<int64_t>(1, target / qtiles);
-  want = std::min<int64_t>(want, (n + 63) / 64);
-  int64_t chunk = ((n + want - 1) / want + 63) / 64 * 64;
-  const uint32_t n_chunks = (uint32_t)((n + chunk - 1) / chunk);
-  uint64_t* lists = nullptr;
-  hip_check(hipMallocAsync((void**)&lists, (size_t)nq * n_chunks * k * 8, s), "alloc chunk lists");
-  const dim3 grid((uint32_t)qtiles, n_chunks);
+  const BfChunks cut(n, nq, k);
+  const dim3 grid((uint32_t)((nq + 31) / 32), cut.n_chunks);
   // at least 64 slots: a buffer is compacted (a 64-key register sort, then
   // every row's threshold reloaded) once it holds more than cap - kBfStep
   // keys, so at k = 10 the 48 slots of k + kBfStep compacted each query
@@ -1096,7 +1126,7 @@ static void bf_one_pass(const void* base, int64_t n, uint32_t dp, const void* qu
   const size_t lds = ((size_t)32 * cap + kBfScratch) * 8;
   auto go = [&](auto kern) {
     hipLaunchKernelGGL(kern, grid, dim3(64), lds, s, (const uint16_t*)base, n, dp, (const uint16_t*)queries, nq,
-                       vsq, qsq, k, cap, chunk, n_chunks, lists, tile_flags);
+                       vsq, qsq, k, cap, cut.chunk, cut.n_chunks, lists, tile_flags);
   };
 #define JA_BF_CASE(K)                                              \
   case K:                                                          \
@@ -1114,40 +1144,70 @@ static void bf_one_pass(const void* base, int64_t n, uint32_t dp, const void* qu
   }
 #undef JA_BF_CASE
   hip_check(hipGetLastError(), "launch bf_scan_kernel");
-  hipLaunchKernelGGL(bf_merge_kernel, dim3((uint32_t)nq), dim3(64), 0, s, (const uint64_t*)lists, nq, n_chunks, k,
+  hipLaunchKernelGGL(bf_merge_kernel, dim3((uint32_t)nq), dim3(64), 0, s, (const uint64_t*)lists, nq, cut.n_chunks, k,
                      out_ids, out_d, q_flags);
   hip_check(hipGetLastError(), "launch bf_merge_kernel");
-  (void)hipFreeAsync(lists, s);
 }
 
-// Scores the whole base in rounds and writes the results; flags (cleared by
-// the caller) name the queries that are left to the one-pass kernels. G: the
-// tiles, of units of UNIT rows; round(parts, qblocks, t0, t1, order, dist, lost): launches one round.
+// Scratch of the rounds path, one allocation (with eight, back-to-back calls of
+// 300 queries and 65,536 x 128 rows, k = 1, took 254 us each instead of 113, and
+// the first of 10k queries and 1M rows 4.2 ms instead of 3.5): per query its
+// distances' and list's slots, whose place the one-pass lists take after the
+// last round; a count, a threshold, a norm and a state; then the base's norms.
+struct BfScratch {
+  uint64_t* qcand;
+  float* vsq;
+  uint32_t* qcount;
+  float *qthr, *qsq;
+  uint32_t* any;  // BfState
+
+  // for blocks of `block` of nq queries
+  static size_t slots(int64_t n, int64_t nq, int64_t block, uint32_t k) {
+    size_t most = (size_t)block * kBfListStride * 8;
+    for (int64_t part : {block, nq % block})
+      if (part > 0) most = std::max(most, BfChunks(n, part, k).list_bytes);
+    return most;
+  }
+  static size_t bytes(int64_t n, int64_t nq, int64_t block, uint32_t k, bool norms) {
+    return slots(n, nq, block, k) + (norms ? (size_t)n * 4 : 0) + (size_t)block * (3 * 4 + 1) +
+           (size_t)(block + 31) / 32 + 8;
+  }
+  BfScratch(void* mem, int64_t n, int64_t nq, int64_t block, uint32_t k, bool norms) {
+    qcand = (uint64_t*)mem;
+    vsq = (float*)((char*)mem + slots(n, nq, block, k));
+    qcount = (uint32_t*)(vsq + (norms ? n : 0));
+    qthr = (float*)(qcount + block);
+    qsq = qthr + block;
+    any = (uint32_t*)(qsq + block);
+  }
+};
+
+// Scores the whole base in rounds and writes the results; the scratch's state
+// names the queries that are left to the one-pass kernels. G: the tiles, of
+// units of UNIT rows; round(parts, qblocks, t0, t1, order, dist, again):
+// launches one round.
 template <class G, uint32_t UNIT, class Round>
-static void bf_rounds(int64_t n, int64_t nq, uint32_t k, float* dense, uint32_t* qcount, uint64_t* qcand, float* qthr,
-                      uint8_t* q_flags, uint8_t* tile_flags, int32_t* out_ids, float* out_d, hipStream_t s,
-                      Round round) {
+static void bf_rounds(int64_t n, int64_t nq, uint32_t k, const BfScratch& m, int32_t* out_ids, float* out_d,
+                      hipStream_t s, Round round) {
   const uint32_t n_tiles = (uint32_t)((n + G::TN - 1) / G::TN);
   const uint32_t qblocks = (uint32_t)((nq + G::TM - 1) / G::TM);
   const uint32_t n_units = (uint32_t)((n + UNIT - 1) / UNIT);
   const BfOrder order{bf_order_step(n_units), n_units};
-  uint32_t* any_flag = qcount + nq;
-  uint32_t* any_lost = any_flag + 1;
   // work-groups the chip holds at once: eight waves per CU (two per SIMD)
   constexpr uint32_t kResident = 256u * (8 / G::kWaves);
   constexpr uint32_t kFirstTiles = kBfFirst / G::TN;
   static_assert(kFirstTiles * G::TN == kBfFirst, "round 0 is whole tiles");
-  auto score = [&](uint32_t t0, uint32_t t1, float* dist, const uint32_t* lost) {
-    round(gemm_parts(qblocks, t1 - t0, kResident), qblocks, t0, t1, order, dist, lost);
+  auto score = [&](uint32_t t0, uint32_t t1, float* dist, bool again) {
+    round(gemm_parts(qblocks, t1 - t0, kResident), qblocks, t0, t1, order, dist, again);
     hip_check(hipGetLastError(), "launch a brute-force round");
   };
   auto trim = [&](auto kern, uint32_t threads) {
-    hipLaunchKernelGGL(kern, dim3((uint32_t)nq), dim3(threads), 0, s, (const float*)dense, order, qcount, qcand, k,
-                       any_flag, any_lost, qthr, out_ids, out_d, q_flags, tile_flags);
+    hipLaunchKernelGGL(kern, dim3((uint32_t)nq), dim3(threads), 0, s, m.qcand, order, m.qcount, k, BfState(m.any, nq), m.qthr,
+                       out_ids, out_d);
     hip_check(hipGetLastError(), "launch bf_trim_kernel");
   };
   uint32_t t0 = 0, t1 = kFirstTiles;  // n >= 4 kBfFirst
-  score(t0, t1, dense, nullptr);
+  score(t0, t1, (float*)m.qcand, false);
   trim(bf_trim_kernel<kBfDense, UNIT>, 256);
   while (t1 < n_tiles) {
     // fourfold: about 3 k candidates per query and round, few where most rows
@@ -1157,44 +1217,25 @@ static void bf_rounds(int64_t n, int64_t nq, uint32_t k, float* dense, uint32_t*
     const uint64_t grow = k <= 32 && nq <= 1024 && (uint64_t)t1 * 64 <= n_tiles ? 16 : 4;
     t0 = t1;
     t1 = (uint32_t)std::min<uint64_t>(n_tiles, (uint64_t)t1 * grow);
-    score(t0, t1, nullptr, nullptr);
+    score(t0, t1, nullptr, false);
     if (t1 < n_tiles) trim(bf_trim_kernel<kBfRound, UNIT>, 64);
     else trim(bf_trim_kernel<kBfLast, UNIT>, 64);
   }
-  score(0, n_tiles, nullptr, any_lost);
+  score(0, n_tiles, nullptr, true);
   trim(bf_trim_kernel<kBfAgain, UNIT>, 64);
 }
 
-// The rounds path: scratch, the rounds, and the one-pass kernels for the
-// queries the rounds flagged (none, in the ordinary case: they then end at
-// once).
+// The rounds path for one block of queries: the rounds, and the one-pass kernels
+// for the queries they left over (none, in the ordinary case: they then end at
+// once). The base's norms are computed (rows of up to 128 values) or there is
+// space for them.
 static void bf_in_rounds(const void* base, int64_t n, uint32_t dim, uint32_t dp, const void* queries, int64_t nq,
-                         uint32_t k, int metric, int32_t* out_ids, float* out_d, hipStream_t s) {
-  float* qsq = nullptr;
-  float* vsq = nullptr;
-  float* qthr = nullptr;
-  float* dense = nullptr;     // [nq][kBfFirst] round 0's distances
-  uint32_t* qcount = nullptr;  // [nq] counts, then two words: is any query flagged, has any lost keys
-  uint64_t* qcand = nullptr;
-  uint8_t* flags = nullptr;  // [nq] query flags, then [ceil(nq / 32)] tile flags
-  const int64_t ntiles = (nq + 31) / 32;
-  hip_check(hipMallocAsync((void**)&qthr, (size_t)nq * 4, s), "alloc thresholds");
-  hip_check(hipMallocAsync((void**)&dense, (size_t)nq * kBfFirst * 4, s), "alloc first distances");
-  hip_check(hipMallocAsync((void**)&qcount, (size_t)(nq + 2) * 4, s), "alloc candidate counts");
-  hip_check(hipMallocAsync((void**)&qcand, (size_t)nq * kBfCandCap * 8, s), "alloc candidate lists");
-  hip_check(hipMallocAsync((void**)&flags, (size_t)(nq + ntiles), s), "alloc overflow flags");
-  hipLaunchKernelGGL(bf_clear_kernel, dim3((uint32_t)((nq + ntiles + 255) / 256)), dim3(256), 0, s, flags,
-                     nq + ntiles, qcount + nq);
-  const uint32_t* flagged = qcount + nq;
+                         uint32_t k, int metric, const BfScratch& m, int32_t* out_ids, float* out_d, hipStream_t s) {
+  const BfState state(m.any, nq);
   const uint16_t* base16 = (const uint16_t*)base;
   const uint16_t* queries16 = (const uint16_t*)queries;
-  if (metric == kL2) {
-    hip_check(hipMallocAsync((void**)&qsq, (size_t)nq * 4, s), "alloc query norms");
-    hip_check(hipMallocAsync((void**)&vsq, (size_t)n * 4, s), "alloc base norms");
-  }
-  if (metric == kL2) bf_sqnorms(queries, nq, dp, dim, qsq, nullptr, s);
+  if (metric == kL2) bf_sqnorms(queries, nq, dp, dim, m.qsq, nullptr, s);
   if (dp <= 128) {
-    if (metric == kL2) bf_sqnorms(base, n, dp, dim, vsq, nullptr, s);
     auto go = [&](auto tag) {
       constexpr int KS = decltype(tag)::value;
       using G = BfStream<KS>;
@@ -1202,12 +1243,11 @@ static void bf_in_rounds(const void* base, int64_t n, uint32_t dim, uint32_t dp,
       auto kern = metric == kL2 ? bf_stream_kernel<G, KS, kL2> : bf_stream_kernel<G, KS, kIP>;
       if (lds > 64 * 1024)
         hip_check(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), "LDS");
-      bf_rounds<G, G::TN>(n, nq, k, dense, qcount, qcand, qthr, flags, flags + nq, out_ids, out_d, s,
-                   [&](uint32_t parts, uint32_t qblocks, uint32_t t0, uint32_t t1, BfOrder order, float* dist,
-                       const uint32_t* lost) {
+      bf_rounds<G, G::TN>(n, nq, k, m, out_ids, out_d, s,
+                   [&](uint32_t parts, uint32_t qblocks, uint32_t t0, uint32_t t1, BfOrder order, float* dist, bool again) {
                      hipLaunchKernelGGL(kern, dim3(qblocks * parts), dim3(G::kThreads), lds, s, base16, n, dp,
-                                        queries16, nq, (const float*)qsq, (const float*)vsq, (const float*)qthr, t0,
-                                        t1, order, parts, qblocks, dist, qcount, qcand, lost);
+                                        queries16, nq, (const float*)m.qsq, (const float*)m.vsq, (const float*)m.qthr,
+                                        t0, t1, order, parts, qblocks, dist, m.qcount, m.qcand, m.any, again);
                    });
     };
     switch ((dp + 15) / 16) {
@@ -1226,12 +1266,11 @@ static void bf_in_rounds(const void* base, int64_t n, uint32_t dim, uint32_t dp,
       constexpr size_t lds = BfTileLds<G>::bytes;
       auto kern = metric == kL2 ? bf_tile_kernel<G, kL2> : bf_tile_kernel<G, kIP>;
       hip_check(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), "LDS");
-      bf_rounds<G, kBfTileUnit>(n, nq, k, dense, qcount, qcand, qthr, flags, flags + nq, out_ids, out_d, s,
-                   [&](uint32_t parts, uint32_t qblocks, uint32_t t0, uint32_t t1, BfOrder order, float* dist,
-                       const uint32_t* lost) {
+      bf_rounds<G, kBfTileUnit>(n, nq, k, m, out_ids, out_d, s,
+                   [&](uint32_t parts, uint32_t qblocks, uint32_t t0, uint32_t t1, BfOrder order, float* dist, bool again) {
                      hipLaunchKernelGGL(kern, dim3(qblocks * parts), dim3(G::kThreads), lds, s, base16, n, dp,
-                                        queries16, nq, (const float*)qsq, (const float*)qthr, t0, t1, order, parts,
-                                        qblocks, dist, qcount, qcand, lost);
+                                        queries16, nq, (const float*)m.qsq, (const float*)m.qthr, t0, t1, order, parts,
+                                        qblocks, dist, m.qcount, m.qcand, m.any, again);
                    });
     };
     // 256 queries per work-group at 991 TFLOP/s or 128 at 850 (mfma_gemm.hpp),
@@ -1239,16 +1278,10 @@ static void bf_in_rounds(const void* base, int64_t n, uint32_t dim, uint32_t dp,
     const uint64_t by256 = (uint64_t)((nq + 255) / 256) * 256 * 850, by128 = (uint64_t)((nq + 127) / 128) * 128 * 991;
     if (by256 <= by128) go(GemmTile<2, 4, 4, 2, 8>{});
     else go(GemmTile<2, 4, 2, 2, 4>{});
-    if (metric == kL2) bf_sqnorms(base, n, dp, dim, vsq, flagged, s);  // for the flagged queries, if there are any
+    if (metric == kL2) bf_sqnorms(base, n, dp, dim, m.vsq, m.any, s);  // if any query is left over
   }
-  bf_one_pass(base, n, dp, queries, nq, k, metric, vsq, qsq, out_ids, out_d, flags + nq, flags, s);
-  (void)hipFreeAsync(qthr, s);
-  (void)hipFreeAsync(dense, s);
-  (void)hipFreeAsync(qcount, s);
-  (void)hipFreeAsync(qcand, s);
-  (void)hipFreeAsync(flags, s);
-  if (vsq) (void)hipFreeAsync(vsq, s);
-  if (qsq) (void)hipFreeAsync(qsq, s);
+  bf_one_pass(base, n, dp, queries, nq, k, metric, m.vsq, m.qsq, m.qcand, out_ids, out_d, state.tile,
+              state.q, s);
 }
 
 void bruteforce_knn(const void* base, int64_t n, uint32_t dim, uint32_t dp, const void* queries, int64_t nq,
@@ -1267,27 +1300,35 @@ void bruteforce_knn(const void* base, int64_t n, uint32_t dim, uint32_t dp, cons
   // queries: 0.63 and 0.75; 1M x 256, k = 10, 3,750: 5.1 and 3.4). Longer rows
   // (40,000 x 384, k = 10, 2,000 queries: 0.58 and 0.31) and larger k (50,000
   // x 64, k = 32: 3.1 and 0.8), where the scan's buffers are compacted ever
-  // more often, do not.
+  // more often, do not; nor do they with one to a hundred queries (16,384 x
+  // 128, k = 17, 1 query: 0.30 and 0.12; x 384, k = 1, 10 queries: 0.17 and
+  // 0.13). At the lines, few queries: 65,536 x 128, k = 1, 300 queries 0.15 and
+  // 0.14.
   const int64_t scanned = k > 16 || dp > 256 ? 0 : dp > 128 ? 262144 : 65536;
   if (n >= std::max<int64_t>(4 * (int64_t)kBfFirst, scanned)) {
-    // the scratch is 24 KB per query: 1.6 GB for a block of queries
-    constexpr int64_t kBlock = 65536;
-    for (int64_t q = 0; q < nq; q += kBlock)
-      bf_in_rounds(base, n, dim, dp, (const uint16_t*)queries + (size_t)q * dp, std::min(kBlock, nq - q), k, metric,
+    // 16 KB of scratch per query, 268 MB for a block of queries
+    const int64_t block = std::min<int64_t>(nq, kBfBlock);
+    void* scratch = nullptr;
+    hip_check(hipMallocAsync(&scratch, BfScratch::bytes(n, nq, block, k, metric == kL2), s), "alloc round scratch");
+    const BfScratch m(scratch, n, nq, block, k, metric == kL2);
+    if (metric == kL2 && dp <= 128) bf_sqnorms(base, n, dp, dim, m.vsq, nullptr, s);
+    for (int64_t q = 0; q < nq; q += block)
+      bf_in_rounds(base, n, dim, dp, (const uint16_t*)queries + (size_t)q * dp, std::min(block, nq - q), k, metric, m,
                    out_ids + (size_t)q * k, out_d + (size_t)q * k, s);
+    (void)hipFreeAsync(scratch, s);
     return;
   }
-  float* vsq = nullptr;
-  float* qsq = nullptr;
+  const size_t list_bytes = BfChunks(n, nq, k).list_bytes;
+  void* scratch = nullptr;
+  hip_check(hipMallocAsync(&scratch, list_bytes + (metric == kL2 ? (size_t)(n + nq) * 4 : 0), s), "alloc chunk lists");
+  float* vsq = metric == kL2 ? (float*)((char*)scratch + list_bytes) : nullptr;
+  float* qsq = metric == kL2 ? vsq + n : nullptr;
   if (metric == kL2) {
-    hip_check(hipMallocAsync((void**)&vsq, (size_t)n * 4, s), "alloc base norms");
-    hip_check(hipMallocAsync((void**)&qsq, (size_t)nq * 4, s), "alloc query norms");
     bf_sqnorms(base, n, dp, dim, vsq, nullptr, s);
     bf_sqnorms(queries, nq, dp, dim, qsq, nullptr, s);
   }
-  bf_one_pass(base, n, dp, queries, nq, k, metric, vsq, qsq, out_ids, out_d, nullptr, nullptr, s);
-  if (vsq) (void)hipFreeAsync(vsq, s);
-  if (qsq) (void)hipFreeAsync(qsq, s);
+  bf_one_pass(base, n, dp, queries, nq, k, metric, vsq, qsq, (uint64_t*)scratch, out_ids, out_d, nullptr, nullptr, s);
+  (void)hipFreeAsync(scratch, s);
 }
 
 }  // namespace jasper_amd

@@ -260,3 +260,49 @@ def test_rows_in_cluster_order(jasper, dim, n, nq, size, k):
     ratio = min(r[0][0] for r in runs) / min(r[1][0] for r in runs)
     print(f"cluster order against shuffled: {ratio:.2f}")
     assert ratio <= 2.5
+
+
+# At the line where the rounds take over (65,536 rows of up to 128 values at
+# small k) a call of few queries is mostly launches and allocations: one more row
+# must not cost more than they do. (With seven allocations 1.3 to 1.4 times.)
+@pytest.mark.parametrize("dim", [32, 128])
+def test_the_rounds_first_size_takes_little_longer(jasper, dim):
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(dim)
+    base = torch.randn((65_536, dim), generator=gen, device="cuda").half()
+    q = torch.randn((300, dim), generator=gen, device="cuda").half()
+
+    def once(rows):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        for _ in range(20):
+            jasper.bruteforce_knn(rows, q, 1, "l2")
+        b.record()
+        torch.cuda.synchronize()
+        return a.elapsed_time(b)
+
+    runs = [(once(base[:-1]), once(base)) for _ in range(8)]
+    ratio = min(r[1] for r in runs) / min(r[0] for r in runs)
+    print(f"65,536 rows against 65,535: {ratio:.2f}")
+    assert ratio <= 1.2
+
+
+# Queries are scored in blocks of 16,384: the second block's results, its queries
+# that are scored again and those left over, and the norms and scratch that it
+# shares with the first.
+@pytest.mark.parametrize("dim,nq", [(8, 16_385), (136, 16_500)])
+@pytest.mark.parametrize("distance", ["l2", "ip"])
+def test_more_queries_than_a_block(jasper, oracle_lib, dim, nq, distance):
+    rng = np.random.default_rng(dim)
+    base = rng.integers(0, 12, size=(16_400, dim)).astype(np.float32)
+    base[3000:9000] = base[7]  # more ties than a list holds
+    q = rng.integers(0, 12, size=(nq, dim)).astype(np.float32)
+    q[40:60] = q[-1:] = base[7]
+    ids, d = _run(jasper, base, q, 17, distance)
+    some = np.r_[0:300, 16_300:nq]
+    rid, rd = _ref(base, q[some], 17, distance)
+    assert np.array_equal(d[some], rd)
+    assert np.array_equal(ids[some], rid)
+    for part in range(0, nq, 4000):  # the others by smaller calls
+        pids, pd = _run(jasper, base, q[part:part + 4000], 17, distance)
+        assert np.array_equal(d[part:part + 4000], pd) and np.array_equal(ids[part:part + 4000], pids)
