@@ -1304,7 +1304,17 @@ void bruteforce_knn(const void* base, int64_t n, uint32_t dim, uint32_t dp, cons
   // 128, k = 17, 1 query: 0.30 and 0.12; x 384, k = 1, 10 queries: 0.17 and
   // 0.13). At the lines, few queries: 65,536 x 128, k = 1, 300 queries 0.15 and
   // 0.14.
-  const int64_t scanned = k > 16 || dp > 256 ? 0 : dp > 128 ? 262144 : 65536;
+  // At k <= 2 the scan's buffers hardly ever fill, and it keeps two more ranges:
+  // up to 64 queries of rows of more than 256 values, where a round leaves most
+  // of its 128 query rows empty (x 960, k = 1, by inner product: 16,384 rows, one
+  // query 66 us and 93, 50 queries 103 and 129; 65,536 rows, 30 queries 1%
+  // apart; 131,072 rows, one query 3%), and 128 to 2,048 queries by inner
+  // product of rows of up to 128, where there are no norms to share (131,072 x
+  // 128, k = 1, 500 queries: 1.27 times as long in rounds; 262,144 rows 0.86
+  // times, 100 queries 1.03, 5,000 0.68).
+  int64_t scanned = k > 16 ? 0 : dp > 256 ? 0 : dp > 128 ? 262144 : 65536;
+  if (k <= 2 && dp > 256 && nq <= 64) scanned = 98304 - 1024 * nq;
+  if (k <= 2 && dp <= 128 && metric == kIP && nq >= 128 && nq <= 2048) scanned = 196608;
   if (n >= std::max<int64_t>(4 * (int64_t)kBfFirst, scanned)) {
     // 16 KB of scratch per query, 268 MB for a block of queries
     const int64_t block = std::min<int64_t>(nq, kBfBlock);

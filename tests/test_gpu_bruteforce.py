@@ -287,6 +287,31 @@ def test_the_rounds_first_size_takes_little_longer(jasper, dim):
     assert ratio <= 1.2
 
 
+# ... nor where it is hardly more than launches: a few queries of long rows, and
+# inner products (no norms) of short ones, at k = 1. (1.3 to 1.4 times.)
+@pytest.mark.parametrize("dim,n,nq,distance", [(960, 16_384, 1, "l2"), (960, 16_384, 1, "ip"), (960, 16_384, 50, "ip"),
+                                               (128, 65_536, 500, "ip")])
+def test_one_row_more_takes_little_longer(jasper, dim, n, nq, distance):
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(dim)
+    base = torch.randn((n, dim), generator=gen, device="cuda").half()
+    q = torch.randn((nq, dim), generator=gen, device="cuda").half()
+
+    def once(rows):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        for _ in range(20):
+            jasper.bruteforce_knn(rows, q, 1, distance)
+        b.record()
+        torch.cuda.synchronize()
+        return a.elapsed_time(b)
+
+    runs = [(once(base[:-1]), once(base)) for _ in range(8)]
+    ratio = min(r[1] for r in runs) / min(r[0] for r in runs)
+    print(f"{n} rows against {n - 1}: {ratio:.2f}")
+    assert ratio <= 1.15
+
+
 # Queries are scored in blocks of 16,384: the second block's results, its queries
 # that are scored again and those left over, and the norms and scratch that it
 # shares with the first.
