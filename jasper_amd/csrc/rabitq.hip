@@ -316,12 +316,14 @@ __device__ __forceinline__ float rabitq_residuals(float4v (&acc)[KT], float x2, 
   return l2;
 }
 
-// KT = number of 16-wide output tiles (mp = 16 * KT <= 256).
+// KT = number of 16-wide output tiles (mp = 16 * KT <= 256). Three waves per SIMD
+// where that takes at most 30 spilled registers (13 and 14 tiles): 1M x 200
+// 2.11 -> 1.87 ms, x 224 2.32 -> 2.06, against two waves; 15 tiles would spill 41
+// (2.45 -> 2.56), and 12 lose 11% at 1,000 rows.
 template <int KT>
-__global__ __launch_bounds__(256, 2) void rabitq_kernel(const float* __restrict__ x, int64_t n, uint32_t stride,
-                                                     uint32_t dim, const float* __restrict__ pt, uint32_t kp,
-                                                     const float* __restrict__ rc, int metric,
-                                                     uint32_t* __restrict__ out) {
+__global__ __launch_bounds__(256, KT == 13 || KT == 14 ? 3 : 2) void rabitq_kernel(
+    const float* __restrict__ x, int64_t n, uint32_t stride, uint32_t dim, const float* __restrict__ pt, uint32_t kp,
+    const float* __restrict__ rc, int metric, uint32_t* __restrict__ out) {
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t wave = threadIdx.x >> 6;
   const uint32_t col = lane & 15u;  // vector within the tile
