@@ -95,9 +95,8 @@ def test_generate_groundtruth_uses_kernel(jasper, oracle_lib):
 
 @pytest.mark.parametrize("distance", ["l2", "ip"])
 def test_two_pass_integer_exact(jasper, oracle_lib, distance):
-    """n >= 262,144 takes the two-pass path (sample thresholds, filtered GEMM,
-    per-query select); on integer data it must equal the reference arithmetic
-    bit for bit, ties ordered by id."""
+    """A base scored in several rounds; on integer data it must equal the
+    reference arithmetic bit for bit, ties ordered by id."""
     base = integer_clustered(300_000, 64, 44)
     q = integer_clustered(100, 64, 45)
     for k in (10, 64, 100):
@@ -144,8 +143,8 @@ def test_long_rows_config4_data(jasper, oracle_lib):
 
 
 def test_two_pass_overflow_falls_back(jasper, oracle_lib):
-    """Most rows equal: every copy ties at the sample's k-th distance, the
-    candidate lists overflow, and the flagged queries are redone in one pass."""
+    """Most rows equal: every copy ties at the k-th distance, the lists overflow
+    also when such queries are scored again, and they are redone in one pass."""
     rng = np.random.default_rng(46)
     base = np.repeat(rng.integers(0, 50, size=(1, 32)), 290_000, axis=0).astype(np.float32)
     idx = rng.choice(290_000, size=5_000, replace=False)
@@ -331,3 +330,53 @@ def test_more_queries_than_a_block(jasper, oracle_lib, dim, nq, distance):
     for part in range(0, nq, 4000):  # the others by smaller calls
         pids, pd = _run(jasper, base, q[part:part + 4000], 17, distance)
         assert np.array_equal(d[part:part + 4000], pd) and np.array_equal(ids[part:part + 4000], pids)
+
+
+def _check_close(ids, d, base, q, k, distance):
+    """Ids and distances against 64-bit ones, as far as rounding decides them:
+    an id that is listed has the distance that it is listed with, and no row that
+    is nearer by more than the rounding is missing."""
+    b = base.astype(np.float16).astype(np.float64)
+    x = q.astype(np.float16).astype(np.float64)
+    dot = x @ b.T
+    if distance == "l2":
+        bn, qn = (b * b).sum(1), (x * x).sum(1)
+        ref = np.maximum(qn[:, None] + bn[None] - 2 * dot, 0)
+        # fp32 sums of dim products, in any order, of the norms and the product
+        err = (base.shape[1] + 4) * 2.0**-24 * (qn[:, None] + bn[None] + 2 * (np.abs(x) @ np.abs(b).T))
+    else:
+        ref = -dot
+        # the sum's rounding, then that to fp16 (half a step; subnormal ones too)
+        err = (base.shape[1] + 4) * 2.0**-24 * (np.abs(x) @ np.abs(b).T)
+        err = err + (np.abs(dot) + err) * 2.0**-11 + 2.0**-25
+    rows = np.arange(len(q))[:, None]
+    assert (np.abs(d - ref[rows, ids]) <= err[rows, ids]).all()
+    assert all(len(set(i)) == k for i in ids.tolist())
+    upper = d[:, -1:].astype(np.float64)
+    nearer = ref + err < upper
+    nearer[rows, ids] = False
+    assert not nearer.any(), np.argwhere(nearer)[:5]
+
+
+# The rounds drop a score by a cheap test whose margins only matter where sums
+# round: real-valued rows on every round kernel and both metrics; norms far larger
+# than the distances (a common offset), where the margins are tightest; queries
+# that are base rows (a threshold near zero); values among fp16's subnormals.
+@pytest.mark.parametrize("dim,n,nq,k", [(96, 17_003, 130, 32), (100, 66_001, 70, 10), (128, 70_001, 300, 10),
+                                        (128, 17_001, 100, 100), (40, 65_537, 64, 1), (136, 17_005, 100, 20),
+                                        (264, 20_001, 200, 10), (520, 17_001, 100, 100), (960, 17_001, 257, 10)])
+@pytest.mark.parametrize("distance", ["l2", "ip"])
+@pytest.mark.parametrize("values", ["gaussian", "offset", "subnormal"])
+def test_rounds_real_values(jasper, dim, n, nq, k, distance, values):
+    base, q = gaussian(n, dim, dim), gaussian(nq, dim, dim + 1)
+    near = np.random.default_rng(dim).integers(0, n, size=nq // 2)
+    if values == "offset":
+        shift = 16.0 if distance == "l2" else 4.0  # an inner product is an fp16 number: 16 * 960 < 65,504
+        base, q = base + shift, q + shift
+    elif values == "subnormal":
+        base, q = base * 2.0**-18, q * 2.0**-18
+    q[: nq // 2] = base[near]
+    ids, d = _run(jasper, base, q, k, distance)
+    _check_close(ids, d, base, q, k, distance)
+    if distance == "l2" and values == "gaussian":
+        assert np.array_equal(ids[: nq // 2, 0], near)

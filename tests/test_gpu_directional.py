@@ -353,6 +353,19 @@ def test_rotate_operator(jasper, oracle_lib, dim, n):
     assert torch.equal(got_h.cpu(), got.cpu())
 
 
+# Many rows take larger tiles (from 256 tiles of 256 x 256 on), whose work-groups
+# walk several of them: the same bits as the rows in small calls, with ragged last
+# rows, outputs and K slices.
+@pytest.mark.parametrize("dim,n", [(960, 16_500), (1000, 70_001), (200, 140_003)])
+def test_rotate_many_rows(jasper, dim, n):
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(dim)
+    x = (torch.randn((n, dim), generator=gen, device="cuda") * 4).half()
+    got = jasper.rotate(x, seed=42)
+    for at in range(0, n, 2100):
+        assert torch.equal(got[at:at + 2100], jasper.rotate(x[at:at + 2100], seed=42)), at
+
+
 def test_prerotation_recorded_in_file(jasper, oracle_lib, tmp_path):
     # the trailer records the prerotation (flag 8 and the seed); a load that
     # does not ask for it still rotates queries the same way
