@@ -679,7 +679,7 @@ __global__ __launch_bounds__(G::kThreads, 2) void bf_tile_kernel(
 // IP compares each sum with its bound (its error has no bound without norms).
 // 10k x 1M x 128, k = 10, L2, the whole call: 4.71 ms with thresholds from a
 // scan of 65,536 rows and 32 queries per wave, 3.3 ms this way (the last round
-// 1,014 TFLOP/s); k = 100 by inner product at 96 values 40 -> 6.1 ms.
+// 1,002 TFLOP/s); k = 100 by inner product at 96 values 40 -> 6.1 ms.
 template <int KS>
 struct BfStream {
   static constexpr int TM = 256, TN = 64, kWaves = 4, kThreads = 256, kBuffers = 3;

@@ -359,7 +359,8 @@ def _check_close(ids, d, base, q, k, distance):
 
 
 # The rounds drop a score by a cheap test whose margins only matter where sums
-# round: real-valued rows on every round kernel and both metrics; norms far larger
+# round: real-valued rows on every round kernel and both metrics, against 64 bits
+# and, bit for bit, against the one-pass kernels, which compute the same sums; norms far larger
 # than the distances (a common offset), where the margins are tightest; queries
 # that are base rows (a threshold near zero); values among fp16's subnormals.
 @pytest.mark.parametrize("dim,n,nq,k", [(96, 17_003, 130, 32), (100, 66_001, 70, 10), (128, 70_001, 300, 10),
@@ -378,5 +379,13 @@ def test_rounds_real_values(jasper, dim, n, nq, k, distance, values):
     q[: nq // 2] = base[near]
     ids, d = _run(jasper, base, q, k, distance)
     _check_close(ids, d, base, q, k, distance)
+    # the same bits as parts of the base too small for rounds, merged
+    parts = [_run(jasper, base[at:at + 16_000], q, k, distance) for at in range(0, n - k, 16_000)]
+    pi = np.concatenate([i + 16_000 * at for at, (i, _) in enumerate(parts)], axis=1)
+    pd = np.concatenate([x for _, x in parts], axis=1)
+    bits = pd.view(np.int32)
+    first = np.lexsort((pi, np.where(bits < 0, bits ^ 0x7FFFFFFF, bits)), axis=1)[:, :k]
+    assert np.array_equal(ids, np.take_along_axis(pi, first, 1))
+    assert np.array_equal(d.view(np.int32), np.take_along_axis(bits, first, 1))
     if distance == "l2" and values == "gaussian":
         assert np.array_equal(ids[: nq // 2, 0], near)
